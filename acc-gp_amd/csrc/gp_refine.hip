@@ -1623,7 +1623,8 @@ __global__ void k_lp_arm(unsigned long long* ctr, int k, unsigned long long run,
 // labels of an improving round (n bytes from labels to keep) instead of a
 // separate k_lp_keep launch.
 __global__ void __launch_bounds__(256) k_lp_decide(unsigned long long* ctr, LoopParams P,
-                                                   unsigned long long* mailbox, const Label* labels, Label* keep,
+                                                   unsigned long long* mailbox, unsigned long long* flag,
+                                                   unsigned long long seq, const Label* labels, Label* keep,
                                                    std::int64_t n) {
     unsigned long long* loads = ctr + kCtrCount;
     unsigned long long* L = loads + P.k;
@@ -1699,20 +1700,23 @@ __global__ void __launch_bounds__(256) k_lp_decide(unsigned long long* ctr, Loop
         }
     }
     __syncthreads();
-    if (!s_run) return;
+    if (!s_run) {
+        publish_to_host(flag, seq);
+        return;
+    }
     // Running: the first kMailWords loop words to the mailbox; stopped:
     // every loop word, then the loads and the best loads.
-    if (mailbox)
-        for (int i = threadIdx.x; i < (s_stop ? (int)kLoopWords : kMailWords); i += blockDim.x) mailbox[i] = s_words[i];
+    for (int i = threadIdx.x; i < (s_stop ? (int)kLoopWords : kMailWords); i += blockDim.x) mailbox[i] = s_words[i];
     for (int p = threadIdx.x; p < P.k; p += blockDim.x) {
         const unsigned long long load = loads[p];
         const unsigned long long best = s_improved ? load : L[kLoopWords + p];
         if (s_improved) L[kLoopWords + p] = load;
-        if (mailbox && s_stop) {
+        if (s_stop) {
             mailbox[kLoopWords + p] = load;
             mailbox[kLoopWords + P.k + p] = best;
         }
     }
+    publish_to_host(flag, seq);
     for (int i = threadIdx.x; i < kCtrCount; i += blockDim.x) ctr[i] = 0;
     if (keep && s_improved)
         for (std::int64_t v = threadIdx.x; v < n; v += blockDim.x) keep[v] = labels[v];
@@ -2810,7 +2814,8 @@ public:
     // The launches of one LP round of a device-controlled loop: the frontier
     // compaction does nothing once the loop word kRun is zero, so every later
     // launch of the round finds empty lists; k_lp_decide ends the round.
-    void round_issue(const LoopParams& P, Label* best_labels, bool vec) {
+    // Returns the number the round publishes in the mailbox flag.
+    unsigned long long round_issue(const LoopParams& P, Label* best_labels, bool vec) {
         const hipStream_t s = c_.stream();
         const std::int64_t n = a_.n;
         unsigned long long* L = ctr_.get() + kCtrCount + a_.k;
@@ -2822,14 +2827,16 @@ public:
         // Levels of at most kKeepInline vertices checkpoint inside the
         // decision kernel; larger ones in a launch of their own.
         const bool inline_keep = n <= kKeepInline;
-        hipLaunchKernelGGL(k_lp_decide, dim3(1), dim3(256), 0, s, ctr_.get(), P, c_.mailbox(), a_.labels,
-                           inline_keep ? best_labels : nullptr, n);
+        const unsigned long long seq = c_.next_seq();
+        hipLaunchKernelGGL(k_lp_decide, dim3(1), dim3(256), 0, s, ctr_.get(), P, c_.mailbox(), c_.mailbox_flag(), seq,
+                           a_.labels, inline_keep ? best_labels : nullptr, n);
         GP_LAUNCH_CHECK();
         if (!inline_keep) {
             hipLaunchKernelGGL(k_lp_keep, dim3(grid_for(ceil_div(n, 16), 256, 1024)), dim3(256), 0, s, L + kImproved,
                                a_.labels, best_labels, n, vec);
             GP_LAUNCH_CHECK();
         }
+        return seq;
     }
 
     // The LP proposal and afterburner sweeps of a round (counter block clear).
@@ -2885,16 +2892,16 @@ public:
             GP_LAUNCH_CHECK();
             mail[kRun] = 1;  // the stream is idle: no round of an earlier run is in flight
             std::vector<std::size_t> marks;
-            int issued = 0;
+            unsigned long long seqs[2] = {0, 0};  // of the last two rounds issued
             auto issue = [&] {
                 marks.push_back(c_.pending_mark());
-                round_issue(P, best_labels, vec);
-                c_.mark(issued++);
+                seqs[0] = seqs[1];
+                seqs[1] = round_issue(P, best_labels, vec);
             };
             issue();
             for (;;) {
                 if (ahead) issue();
-                c_.wait_mark(issued - 1 - ahead);
+                c_.wait_flag(c_.mailbox_flag(), seqs[ahead ? 0 : 1]);
                 if (!mail[kRun]) break;
                 if (!ahead) issue();
             }
