@@ -637,11 +637,13 @@ int gp_refine_partition(gp_context* ctx, const gp_graph* g, int32_t* labels, con
         gp::DBuf<std::int32_t> lab = c.buf<std::int32_t>(static_cast<std::size_t>(d.n));
         c.upload(lab.get(), labels, static_cast<std::size_t>(d.n) * 4);
         std::vector<std::uint64_t> loads(static_cast<std::size_t>(o.parts));
-        gp::device_loads(c, d, lab.get(), o.parts, loads.data());
+        const std::uint64_t directed = gp::recount(c, d, lab.get(), o.parts, loads.data());
         std::uint64_t total = 0;
         for (auto x : loads) total += x;
         const std::uint64_t cap = gp::capacity_of(total, o.parts, o.imbalance);
-        gp::LevelStats st = gp::refine_level(c, d, lab.get(), loads, o, cap, o.max_rounds, false, 0);
+        if (directed & 1ULL) throw std::runtime_error("refinement cut is not symmetric");
+        gp::LevelStats st =
+            gp::refine_level(c, d, lab.get(), loads, o, cap, o.max_rounds, !o.strict_verify, directed / 2);
         c.download(labels, lab.get(), static_cast<std::size_t>(d.n) * 4);
         if (stats) *stats = to_c(st);
     });

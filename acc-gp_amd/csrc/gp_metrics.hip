@@ -1,29 +1,39 @@
 // Edge cut and part loads of device-resident labels: the verification
 // counts of the reference (host_cut, include/graph.hpp:67-69; the device cut
 // and load recounts of src/refine.cu:63-98 and the final check of
-// src/uncoarsen.cu:90-100), in two passes with no atomics to global memory.
+// src/uncoarsen.cu:90-100), in one launch.
 //
-// Pass 1: each block walks chunks of 64 consecutive vertices per wave.  A
-// wave stages the chunk's 65 offsets and 64 labels in LDS, adds the vertex
-// weights into a wave-private LDS table of part loads, then its lanes walk
-// the chunk's entries in coalesced 64-entry strides, find each entry's
-// source row by a binary search over the staged offsets and compare the
-// source label with the gathered neighbour label.  The block writes one row
-// of partials: [directed cut weight, labels outside [0, k), load_0 ..
-// load_{k-1}].  Pass 2: one block sums the rows column by column.
+// Rows and entries together are split evenly over the waves, whatever the row
+// lengths: a wave finds its first row and entry with a 64-way search (each
+// step, 64 lanes probe 64 offsets) and walks its entries in windows of
+// kCutRows rows, whose ends and labels it stages in LDS.  The row of a given
+// entry is the number of row ends at or below it, so ballots tell the rows of
+// a batch's first and last entry: a batch in one row (hubs) broadcasts its
+// label, otherwise each lane finds its row by a binary search between the two.
+// kCutBatch neighbours per lane are loaded before their labels are gathered.
+// Part loads are summed per block in LDS over an even split of the vertices.
+// Each block writes one row of partials: [directed cut weight, labels outside
+// [0, k), load_0 .. load_{k-1}]; the last block to finish adds the rows up and
+// writes the totals straight to the host's read-back buffer.
 //
-// Bound: HBM.  Algorithmic bytes per call: 4(n+1) offsets + 4n labels + 4n
-// vertex weights + m (4 neighbour + 4 neighbour label [+ 4 edge weight]).
+// R-MAT scale 20 (31 M entries, k = 64): 145 us; 64 vertices per wave, the
+// earlier split, took 14.5 ms, one wave walking all the hubs, and an even
+// split of the entries alone 360 us, where a wave meets hundreds of rows with
+// an entry or none.  kCutBatch 8 instead of 4: 196 us.
+//
+// Bound: the gather of a label per entry (L2 serves most of it).  Bytes per
+// call: 4(n+1) offsets + 4n labels + 4n vertex weights + m (4 neighbour
+// [+ 4 edge weight]).
 #include "gp_metrics.hpp"
 
+#include <algorithm>
 #include <mutex>
 #include <stdexcept>
 #include <unordered_map>
 
 // Scratch of the allocation-free evaluation (edge_cut_noalloc): room for the
-// partial rows and the totals row of the largest evaluation, 1024 partial
-// blocks + 1 totals row of 130 words (cut, out-of-range count, 128 loads),
-// 1,066,000 bytes.  Every GPU holds its own copy until the process ends.
+// partial rows of the largest evaluation, at most 1025 rows of 130 words
+// (cut, out-of-range count, 128 loads), 1,066,000 bytes.  Every GPU holds its own copy until the process ends.
 // Host code never passes this name to a kernel: it is a host-side stand-in,
 // and the device address comes from hipGetSymbolAddress per device.
 static __device__ __align__(256) unsigned long long scratch[gp::kNoAllocScratchWords];
@@ -32,50 +42,122 @@ namespace gp {
 
 namespace {
 
-constexpr int kCutThreads = 256;
+constexpr int kCutThreads = 1024;
 constexpr int kCutWaves = kCutThreads / kWave;
+constexpr int kCutBatch = 4;                // entries per lane in flight
+constexpr int kCutPer = 4;                  // staged rows per lane
+constexpr int kCutRows = kCutPer * kWave;   // rows of a window
 
-template <bool Weighted>
-__global__ void __launch_bounds__(kCutThreads) k_cut_partials(std::int64_t n, const std::int32_t* off,
-                                                              const std::int32_t* nbr, const std::uint32_t* ew,
-                                                              const std::uint32_t* vw, const std::int32_t* labels,
-                                                              int k, unsigned long long* partials) {
-    __shared__ unsigned long long loads[kCutWaves][kMaxParts];
-    __shared__ std::int32_t soff[kCutWaves][kWave + 1];
-    __shared__ std::int32_t slab[kCutWaves][kWave];
+// Where the walk over rows and their entries stands after `d` steps, a row
+// counting one step before its entries: the row reached, the last r in [0, n)
+// with off[r] + r <= d.  The whole wave takes part.
+__device__ inline std::int64_t wave_row_at(const std::int32_t* off, std::int64_t n, std::int64_t d) {
+    std::int64_t lo = 0, len = n;  // the answer lies in [lo, lo + len)
+    while (len > 1) {
+        const std::int64_t step = (len + kWave - 1) / kWave;
+        const std::int64_t at = lo + step * lane_id();
+        const bool below = step * lane_id() < len && off[at] + at <= d;
+        const int hits = __popcll(__ballot(below));  // ascending: the first hits lanes
+        const std::int64_t first = step * (hits > 0 ? hits - 1 : 0);
+        lo += first;
+        len = len - first < step ? len - first : step;
+    }
+    return lo;
+}
+
+template <bool Weighted, class L>
+__global__ void __launch_bounds__(kCutThreads) k_edge_cut(std::int64_t n, const std::int32_t* off,
+                                                          const std::int32_t* nbr, const std::uint32_t* ew,
+                                                          const std::uint32_t* vw, const L* labels, int k,
+                                                          unsigned long long* partials, unsigned int* ticket,
+                                                          unsigned long long* host, unsigned long long* flag,
+                                                          unsigned long long seq) {
+    __shared__ unsigned long long loads[kMaxParts];
+    __shared__ std::int32_t send[kCutWaves][kCutRows];
+    __shared__ L slab[kCutWaves][kCutRows];
     __shared__ unsigned long long red[kCutWaves][2];
     const int lane = lane_id(), w = threadIdx.x / kWave;
-    for (int p = lane; p < k; p += kWave) loads[w][p] = 0;
-    wave_sync();
+    for (int p = threadIdx.x; p < k; p += kCutThreads) loads[p] = 0;
+    __syncthreads();
     unsigned long long cut = 0, bad = 0;
-    const std::int64_t chunks = (n + kWave - 1) / kWave;
-    for (std::int64_t ch = (std::int64_t)blockIdx.x * kCutWaves + w; ch < chunks;
-         ch += (std::int64_t)gridDim.x * kCutWaves) {
-        const std::int64_t v0 = ch * kWave;
-        const int cnt = static_cast<int>(n - v0 < kWave ? n - v0 : kWave);
-        if (lane < cnt) {
-            const std::int32_t lab = labels[v0 + lane];
-            soff[w][lane] = off[v0 + lane];
-            slab[w][lane] = lab;
-            if (static_cast<unsigned>(lab) < static_cast<unsigned>(k))
-                atomicAdd(&loads[w][lab], static_cast<unsigned long long>(vw[v0 + lane]));
-            else
-                ++bad;
+
+    for (std::int64_t v = blockIdx.x * (std::int64_t)kCutThreads + threadIdx.x; v < n;
+         v += (std::int64_t)gridDim.x * kCutThreads) {
+        const int lab = (int)labels[v];
+        if (static_cast<unsigned>(lab) < static_cast<unsigned>(k))
+            atomicAdd(&loads[lab], static_cast<unsigned long long>(vw[v]));
+        else
+            ++bad;
+    }
+
+    // This wave's entries [pos, stop): an even share of rows and entries.
+    const std::int64_t m = n > 0 ? (std::int64_t)off[n] : 0;
+    const std::int64_t waves = (std::int64_t)gridDim.x * kCutWaves;
+    const std::int64_t share = (n + m + waves - 1) / waves;
+    const std::int64_t d0 = (blockIdx.x * (std::int64_t)kCutWaves + w) * share;
+    std::int64_t row = 0, pos = 0, stop = 0;
+    if (d0 < n + m) {
+        row = wave_row_at(off, n, d0);
+        const std::int64_t d1 = d0 + share, row1 = d1 < n + m ? wave_row_at(off, n, d1) : 0;
+        const std::int64_t e0 = off[row + 1], e1 = off[row1 + 1];
+        pos = d0 - row < e0 ? d0 - row : e0;
+        stop = d1 >= n + m ? m : d1 - row1 < e1 ? d1 - row1 : e1;
+    }
+    while (pos < stop) {
+        std::int32_t end[kCutPer];
+#pragma unroll
+        for (int i = 0; i < kCutPer; ++i) {
+            const std::int64_t r = row + i * kWave + lane;
+            end[i] = off[r < n ? r + 1 : n];
+            send[w][i * kWave + lane] = end[i];
+            slab[w][i * kWave + lane] = labels[r < n ? r : n - 1];
         }
-        if (lane == 0) soff[w][cnt] = off[v0 + cnt];
         wave_sync();
-        const std::int32_t e0 = soff[w][0], e1 = soff[w][cnt];
-        for (std::int32_t e = e0 + lane; e < e1; e += kWave) {
-            int lo = 0, hi = cnt - 1;  // last row whose first entry is <= e
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (soff[w][mid] <= e) lo = mid;
-                else hi = mid - 1;
+        const std::int64_t last_end = __shfl(end[kCutPer - 1], kWave - 1);
+        const std::int64_t window = last_end < stop ? last_end : stop;
+        while (pos < window) {
+            const std::int64_t batch = pos + kCutBatch * kWave < window ? pos + kCutBatch * kWave : window;
+            std::int32_t u[kCutBatch];
+            std::uint32_t wt[kCutBatch];
+#pragma unroll
+            for (int j = 0; j < kCutBatch; ++j) {
+                const std::int64_t e = pos + j * kWave + lane;
+                const std::int64_t x = e < batch ? e : batch - 1;
+                u[j] = nbr[x];
+                wt[j] = Weighted ? ew[x] : 1u;
             }
-            if (slab[w][lo] != labels[nbr[e]]) cut += Weighted ? static_cast<unsigned long long>(ew[e]) : 1ULL;
+            // Rows of the batch's first and last entry.
+            int r0 = 0, r1 = 0;
+#pragma unroll
+            for (int i = 0; i < kCutPer; ++i) {
+                r0 += __popcll(__ballot(end[i] <= pos));
+                r1 += __popcll(__ballot(end[i] < batch));
+            }
+            L lu[kCutBatch];
+#pragma unroll
+            for (int j = 0; j < kCutBatch; ++j) lu[j] = labels[u[j]];
+            const L lab0 = slab[w][r0];
+#pragma unroll
+            for (int j = 0; j < kCutBatch; ++j) {
+                const std::int32_t e = (std::int32_t)pos + j * kWave + lane;
+                L lab = lab0;
+                if (r0 != r1) {
+                    int lo = r0, hi = r1;  // first staged row whose end lies after e
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (send[w][mid] <= e) lo = mid + 1;
+                        else hi = mid;
+                    }
+                    lab = slab[w][lo];
+                }
+                if (e < batch && lab != lu[j]) cut += wt[j];
+            }
+            pos = batch;
         }
+        row += kCutRows;
         wave_sync();
     }
+
     cut = wave_sum(cut);
     bad = wave_sum(bad);
     if (lane == 0) {
@@ -83,70 +165,120 @@ __global__ void __launch_bounds__(kCutThreads) k_cut_partials(std::int64_t n, co
         red[w][1] = bad;
     }
     __syncthreads();
-    unsigned long long* row = partials + static_cast<std::size_t>(blockIdx.x) * (k + 2);
+    const int cols = k + 2;
+    unsigned long long* own = partials + static_cast<std::size_t>(blockIdx.x) * cols;
     if (threadIdx.x < 2) {
         unsigned long long s = 0;
         for (int x = 0; x < kCutWaves; ++x) s += red[x][threadIdx.x];
-        row[threadIdx.x] = s;
+        own[threadIdx.x] = s;
     }
-    for (int p = threadIdx.x; p < k; p += kCutThreads) {
+    for (int p = threadIdx.x; p < k; p += kCutThreads) own[2 + p] = loads[p];
+    if (!block_is_last(ticket)) return;
+
+    // Column sums: groups of threads take every groups-th row, then a tree in
+    // LDS (the staging arrays are done with).
+    __shared__ unsigned long long sums[kMaxParts + 2];
+    for (int c = threadIdx.x; c < cols; c += kCutThreads) sums[c] = 0;
+    __syncthreads();
+    const int groups = kCutThreads / cols;
+    const int g = threadIdx.x / cols, c = threadIdx.x % cols;
+    if (g < groups) {
         unsigned long long s = 0;
-        for (int x = 0; x < kCutWaves; ++x) s += loads[x][p];
-        row[2 + p] = s;
+        for (unsigned b = g; b < gridDim.x; b += groups) s += partials[static_cast<std::size_t>(b) * cols + c];
+        if (s) atomicAdd(&sums[c], s);
+    }
+    __syncthreads();
+    for (int x = threadIdx.x; x < cols; x += kCutThreads) host[x] = sums[x];
+    publish_to_host(flag, seq);
+}
+
+// Labels as bytes, 255 for one outside [0, k).
+__global__ void __launch_bounds__(256) k_byte_labels(std::int64_t n, const std::int32_t* labels, int k,
+                                                     std::uint8_t* out) {
+    for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
+         v += (std::int64_t)gridDim.x * blockDim.x) {
+        const std::int32_t lab = labels[v];
+        out[v] = static_cast<unsigned>(lab) < static_cast<unsigned>(k) ? static_cast<std::uint8_t>(lab) : 255;
     }
 }
 
-__global__ void __launch_bounds__(kCutThreads) k_cut_finish(const unsigned long long* partials, int blocks, int cols,
-                                                            unsigned long long* out) {
-    for (int c = threadIdx.x; c < cols; c += kCutThreads) {
-        unsigned long long s = 0;
-        for (int b = 0; b < blocks; ++b) s += partials[static_cast<std::size_t>(b) * cols + c];
-        out[c] = s;
-    }
+// From this many vertices on (1 MiB of int32 labels, a quarter of an XCD's L2),
+// int32 labels are narrowed to bytes before the entries gather them, where
+// scratch can be allocated.  Whole calls with and without: R-MAT scale 18 63
+// and 66 us, scale 20 145 and 174, a mesh of 2 M points 120 and 190, a grid of
+// 4 M cells (its gathers are local) 83 and 80.
+constexpr std::int64_t kByteLabelsMin = 1 << 18;
+
+// Launch and read-back: `totals` gets the directed cut, the number of labels
+// outside [0, k) and the k part loads.
+template <class L>
+void count_into(Context& c, const DGraph& g, const L* labels, int k, unsigned long long* partials,
+                unsigned long long* totals) {
+    const int blocks = edge_cut_blocks(g.n, g.m);
+    const unsigned long long seq = c.next_seq();
+    if (g.ew)
+        hipLaunchKernelGGL((k_edge_cut<true, L>), dim3(blocks), dim3(kCutThreads), 0, c.stream(), g.n, g.off.get(),
+                           g.nbr.get(), g.ew.get(), g.vw.get(), labels, k, partials, c.ticket(), c.read_buffer(),
+                           c.read_flag(), seq);
+    else
+        hipLaunchKernelGGL((k_edge_cut<false, L>), dim3(blocks), dim3(kCutThreads), 0, c.stream(), g.n, g.off.get(),
+                           g.nbr.get(), nullptr, g.vw.get(), labels, k, partials, c.ticket(), c.read_buffer(),
+                           c.read_flag(), seq);
+    GP_LAUNCH_CHECK();
+    c.wait_flag(c.read_flag(), seq);
+    std::memcpy(totals, c.read_buffer(), static_cast<std::size_t>(k + 2) * sizeof(unsigned long long));
 }
 
 }  // namespace
 
-int edge_cut_blocks(std::int64_t n) {
-    const std::int64_t chunks = (n + kWave - 1) / kWave;
-    const std::int64_t b = (chunks + kCutWaves - 1) / kCutWaves;
+// One batch per thread on small graphs; on large ones two blocks per CU, all
+// resident.
+int edge_cut_blocks(std::int64_t n, std::int64_t m) {
+    const std::int64_t b = (n + m + kCutBatch * kCutThreads - 1) / (kCutBatch * kCutThreads);
     return static_cast<int>(b < 1 ? 1 : (b > kEdgeCutMaxBlocks ? kEdgeCutMaxBlocks : b));
 }
 
-std::size_t edge_cut_scratch_words(std::int64_t n, int k) {
-    return static_cast<std::size_t>(edge_cut_blocks(n) + 1) * static_cast<std::size_t>(k + 2);
+std::size_t edge_cut_scratch_words(std::int64_t n, std::int64_t m, int k) {
+    return static_cast<std::size_t>(edge_cut_blocks(n, m)) * static_cast<std::size_t>(k + 2);
 }
 
 void edge_cut_into(Context& c, const DGraph& g, const std::int32_t* labels, int k, unsigned long long* scratch,
-                   std::uint64_t* cut, std::uint64_t* loads) {
+                   std::uint8_t* byte_labels, std::uint64_t* cut, std::uint64_t* loads) {
     if (k < 2 || k > kMaxParts) throw std::invalid_argument("parts must be in [2, 128]");
     if (!labels && g.n > 0) throw std::invalid_argument("labels must be a device pointer");
-    const int blocks = edge_cut_blocks(g.n);
-    const int cols = k + 2;
-    unsigned long long* partials = scratch;
-    unsigned long long* out = scratch + static_cast<std::size_t>(blocks) * cols;
-    const hipStream_t s = c.stream();
-    if (g.ew)
-        hipLaunchKernelGGL(k_cut_partials<true>, dim3(blocks), dim3(kCutThreads), 0, s, g.n, g.off.get(), g.nbr.get(),
-                           g.ew.get(), g.vw.get(), labels, k, partials);
-    else
-        hipLaunchKernelGGL(k_cut_partials<false>, dim3(blocks), dim3(kCutThreads), 0, s, g.n, g.off.get(),
-                           g.nbr.get(), nullptr, g.vw.get(), labels, k, partials);
-    GP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_cut_finish, dim3(1), dim3(kCutThreads), 0, s, partials, blocks, cols, out);
-    GP_LAUNCH_CHECK();
     unsigned long long host[kMaxParts + 2];
-    c.read(host, out, static_cast<std::size_t>(cols) * sizeof(unsigned long long));
+    if (byte_labels) {
+        hipLaunchKernelGGL(k_byte_labels, dim3(static_cast<unsigned>(std::min<std::int64_t>(ceil_div(g.n, 256), 2048))),
+                           dim3(256), 0, c.stream(), g.n, labels, k, byte_labels);
+        GP_LAUNCH_CHECK();
+        count_into(c, g, byte_labels, k, scratch, host);
+    } else {
+        count_into(c, g, labels, k, scratch, host);
+    }
     if (host[1]) throw std::invalid_argument("labels outside [0, parts)");
     if (host[0] & 1ULL) throw std::runtime_error("directed cut is odd: the graph is not symmetric");
     *cut = host[0] / 2;
     for (int p = 0; p < k; ++p) loads[p] = host[2 + p];
 }
 
+template <class L>
+std::uint64_t recount(Context& c, const DGraph& g, const L* labels, int k, std::uint64_t* loads) {
+    DBuf<unsigned long long> partials = c.buf<unsigned long long>(edge_cut_scratch_words(g.n, g.m, k));
+    unsigned long long host[kMaxParts + 2];
+    count_into(c, g, labels, k, partials.get(), host);
+    if (loads)
+        for (int p = 0; p < k; ++p) loads[p] = host[2 + p];
+    return host[0];
+}
+template std::uint64_t recount(Context&, const DGraph&, const std::uint8_t*, int, std::uint64_t*);
+template std::uint64_t recount(Context&, const DGraph&, const std::int32_t*, int, std::uint64_t*);
+
 void edge_cut(Context& c, const DGraph& g, const std::int32_t* labels, int k, std::uint64_t* cut,
               std::uint64_t* loads) {
-    DBuf<unsigned long long> buf = c.buf<unsigned long long>(edge_cut_scratch_words(g.n, k));
-    edge_cut_into(c, g, labels, k, buf.get(), cut, loads);
+    DBuf<unsigned long long> buf = c.buf<unsigned long long>(edge_cut_scratch_words(g.n, g.m, k));
+    DBuf<std::uint8_t> bytes;
+    if (g.n >= kByteLabelsMin && labels) bytes = c.buf<std::uint8_t>(static_cast<std::size_t>(g.n));
+    edge_cut_into(c, g, labels, k, buf.get(), bytes.get(), cut, loads);
 }
 
 namespace {
@@ -174,7 +306,7 @@ unsigned long long* resolve_noalloc_scratch(int device) {
 void edge_cut_noalloc(Context& c, const DGraph& g, const std::int32_t* labels, int k, std::uint64_t* cut,
                       std::uint64_t* loads) {
     if (k < 2 || k > kMaxParts) throw std::invalid_argument("parts must be in [2, 128]");
-    const std::size_t words = edge_cut_scratch_words(g.n, k);
+    const std::size_t words = edge_cut_scratch_words(g.n, g.m, k);
     if (words > kNoAllocScratchWords)
         throw std::invalid_argument("evaluation needs " + std::to_string(words) + " scratch words, above the " +
                                     std::to_string(kNoAllocScratchWords) + " of the static scratch");
@@ -185,10 +317,9 @@ void edge_cut_noalloc(Context& c, const DGraph& g, const std::int32_t* labels, i
         if (it != g_scratch_address.end()) p = it->second;
     }
     if (!p) throw std::logic_error("evaluation scratch of this device was not resolved at context creation");
-    // No word of the scratch has to start at zero: the partial pass writes
-    // every row the finishing pass reads, and the finishing pass writes the
-    // totals row that is read back.
-    edge_cut_into(c, g, labels, k, p, cut, loads);
+    // No word of the scratch has to start at zero: every block writes the
+    // whole partial row that the last one reads.
+    edge_cut_into(c, g, labels, k, p, nullptr, cut, loads);
 }
 
 }  // namespace gp

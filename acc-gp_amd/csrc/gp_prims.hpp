@@ -531,6 +531,20 @@ inline int bit_width_u64(std::uint64_t v) {
     return b;
 }
 
+// Whether the calling block is the last of its grid to get here; true for
+// one block, which then sees what every other wrote before its call.  ticket:
+// a zero device word, zero again afterwards.
+__device__ inline bool block_is_last(unsigned int* ticket) {
+    __shared__ bool last;
+    block_stores_done();
+    if (threadIdx.x == 0) {
+        last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u == gridDim.x;
+        if (last) *ticket = 0;
+    }
+    __syncthreads();
+    return last;
+}
+
 // ---------------------------------------------------------- reductions
 // One global atomic per block (blocks of at most 1024 threads).
 template <typename T>

@@ -4,6 +4,7 @@
 // capacity-complementary exchange.  Restates src/refine.cu and
 // src/refinement/*.cuh of the reference; order-dependent steps follow the
 // canonical vertex-id order.
+#include "gp_metrics.hpp"
 #include "gp_refine.hpp"
 #include "gp_rows.hpp"
 
@@ -2577,44 +2578,6 @@ __global__ void k_project(std::int64_t n, const std::int32_t* map, const L* coar
          v += (std::int64_t)gridDim.x * blockDim.x)
         fine[v] = coarse[map[v]];
 }
-template <typename L>
-__global__ void k_cut(std::int64_t n, const std::int32_t* off, const std::int32_t* nbr, const std::uint32_t* ew,
-                      const L* labels, unsigned long long* out) {
-    const int lane = lane_id();
-    unsigned long long local = 0;
-    for (std::int64_t base = (blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x) - lane; base < n;
-         base += (std::int64_t)gridDim.x * blockDim.x) {
-        const std::int64_t v = base + lane;
-        std::int64_t b = 0, e = 0;
-        if (v < n) {
-            b = off[v];
-            e = off[v + 1];
-        }
-        const bool heavy = v < n && e - b > 64;
-        if (v < n && !heavy) {
-            const int s = labels[v];
-            for (std::int64_t x = b; x < e; ++x)
-                if (labels[nbr[x]] != s) local += ew_at(ew, x);
-        }
-        unsigned long long hv = __ballot(heavy);
-        while (hv) {
-            const int src = __ffsll(hv) - 1;
-            hv &= hv - 1;
-            const std::int64_t hvx = __shfl(v, src);
-            const int s = labels[hvx];
-            for (std::int64_t x = off[hvx] + lane; x < off[hvx + 1]; x += kWave)
-                if (labels[nbr[x]] != s) local += ew_at(ew, x);
-        }
-    }
-    local = wave_sum(local);
-    if (lane == 0 && local) atomicAdd(out, local);
-}
-template <typename L>
-__global__ void k_loads(std::int64_t n, const std::uint32_t* vw, const L* labels, unsigned long long* loads) {
-    for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
-         v += (std::int64_t)gridDim.x * blockDim.x)
-        atomicAdd(&loads[labels[v]], (unsigned long long)vw[v]);
-}
 template <typename A, typename B>
 __global__ void k_convert(std::int64_t n, const A* in, B* out) {
     for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
@@ -2633,27 +2596,12 @@ void convert(Context& c, std::int64_t n, const A* in, B* out) {
     GP_LAUNCH_CHECK();
 }
 
+// Cut of symmetric labels and, with loads, the part loads, in one pass.
 template <typename L>
-std::uint64_t cut_of(Context& c, const DGraph& g, const L* labels) {
-    DBuf<unsigned long long> out = c.buf<unsigned long long>(1);
-    fill<unsigned long long>(c, out.get(), 1, 0ULL);
-    if (g.n > 0) {
-        hipLaunchKernelGGL((k_cut<L>), dim3(grid_for(g.n)), dim3(256), 0, c.stream(), g.n, g.off.get(), g.nbr.get(),
-                           g.ew_ptr(), labels, out.get());
-        GP_LAUNCH_CHECK();
-    }
-    const unsigned long long d = c.read_scalar(out.get());
+std::uint64_t cut_of(Context& c, const DGraph& g, const L* labels, int k, std::uint64_t* loads = nullptr) {
+    const std::uint64_t d = recount(c, g, labels, k, loads);
     if (d & 1ULL) throw std::runtime_error("refinement cut is not symmetric");
     return d / 2;
-}
-
-template <typename L>
-void loads_of(Context& c, const DGraph& g, const L* labels, int k, std::uint64_t* loads_host) {
-    DBuf<unsigned long long> out = c.buf<unsigned long long>(static_cast<std::size_t>(k));
-    fill<unsigned long long>(c, out.get(), k, 0ULL);
-    hipLaunchKernelGGL((k_loads<L>), dim3(grid_for(g.n)), dim3(256), 0, c.stream(), g.n, g.vw.get(), labels, out.get());
-    GP_LAUNCH_CHECK();
-    c.read(loads_host, out.get(), static_cast<std::size_t>(k) * sizeof(unsigned long long));
 }
 
 }  // namespace
@@ -2666,8 +2614,6 @@ void project(Context& c, std::int64_t n, const std::int32_t* map, const std::int
     GP_LAUNCH_CHECK();
 }
 
-std::uint64_t device_cut(Context& c, const DGraph& g, const std::int32_t* labels) { return cut_of(c, g, labels); }
-
 std::uint64_t device_edge_weight_sum(Context& c, const DGraph& g) {
     if (!g.ew) return static_cast<std::uint64_t>(g.m);
     DBuf<unsigned long long> out = c.buf<unsigned long long>(1);
@@ -2678,10 +2624,6 @@ std::uint64_t device_edge_weight_sum(Context& c, const DGraph& g) {
         GP_LAUNCH_CHECK();
     }
     return c.read_scalar(out.get());
-}
-
-void device_loads(Context& c, const DGraph& g, const std::int32_t* labels, int k, std::uint64_t* loads_host) {
-    loads_of(c, g, labels, k, loads_host);
 }
 
 namespace {
@@ -3020,9 +2962,9 @@ public:
     // incremental cut must equal a full CSR recount of the labels and the
     // part loads a full recount of the vertex weights.
     void verify(std::uint64_t cut) {
-        if (cut_of(c_, g_, a_.labels) != cut) throw std::runtime_error("incremental cut differs from CSR scan");
         std::vector<std::uint64_t> loads(static_cast<std::size_t>(a_.k));
-        loads_of(c_, g_, a_.labels, a_.k, loads.data());
+        if (cut_of(c_, g_, a_.labels, a_.k, loads.data()) != cut)
+            throw std::runtime_error("incremental cut differs from CSR scan");
         if (loads != loads_host_) throw std::runtime_error("incremental part weights differ from a recount");
         ++st_.strict_checks;
     }
@@ -3438,10 +3380,10 @@ LevelStats refine_level_impl(Context& c, const DGraph& g, Label* labels, std::ve
     st.refined = 1;
     const int k = o.parts;
     LevelRefiner R(c, g, labels, loads, o, cap, st);
-    std::uint64_t cut = has_known_cut ? known_cut : cut_of(c, g, labels);
+    std::uint64_t cut = has_known_cut ? known_cut : cut_of(c, g, labels, k);
     if (o.strict_verify && has_known_cut) {
         // incremental.cuh:777-778: the carried cut must equal a recount.
-        if (cut_of(c, g, labels) != known_cut) throw std::runtime_error("known projection cut differs from CSR scan");
+        if (cut_of(c, g, labels, k) != known_cut) throw std::runtime_error("known projection cut differs from CSR scan");
         ++st.strict_checks;
     }
     st.initial_cut = cut;
@@ -3531,14 +3473,16 @@ UncoarsenResult uncoarsen(Context& c, const Hierarchy& h, const std::int32_t* co
     DBuf<Label> labels = c.buf<Label>(static_cast<std::size_t>(cg.n));
     convert(c, cg.n, coarsest_labels, labels.get());
     std::vector<std::uint64_t> loads(static_cast<std::size_t>(k), 0);
-    loads_of(c, cg, labels.get(), k, loads.data());
+    const std::uint64_t directed = recount(c, cg, labels.get(), k, loads.data());
     std::uint64_t total = 0;
     for (auto x : loads) total += x;
     const long double raw = (long double)total * o.imbalance / k;
     const std::uint64_t cap = (std::uint64_t)std::floor(raw);
     if (cap < total / (unsigned)k + (total % (unsigned)k != 0))
         throw std::invalid_argument("integer partition capacity cannot hold total weight");
-    LevelStats st = refine_level_impl(c, cg, labels.get(), loads, o, cap, o.max_rounds, false, 0);
+    if (directed & 1ULL) throw std::runtime_error("refinement cut is not symmetric");
+    LevelStats st =
+        refine_level_impl(c, cg, labels.get(), loads, o, cap, o.max_rounds, !o.strict_verify, directed / 2);
     res.levels.push_back(st);
     std::uint64_t last_cut = st.final_cut;
     std::int64_t last_refined = cg.n;
@@ -3557,8 +3501,7 @@ UncoarsenResult uncoarsen(Context& c, const Hierarchy& h, const std::int32_t* co
         if (o.strict_verify) {
             // refine.cu:641-659: projection preserves the cut and the part loads.
             std::vector<std::uint64_t> projected(static_cast<std::size_t>(k));
-            loads_of(c, fg, labels.get(), k, projected.data());
-            if (cut_of(c, fg, labels.get()) != last_cut || projected != loads)
+            if (cut_of(c, fg, labels.get(), k, projected.data()) != last_cut || projected != loads)
                 throw std::runtime_error("GPU projection failed cut or part-weight preservation");
             ++ls.strict_checks;
         }

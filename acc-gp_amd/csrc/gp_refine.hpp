@@ -14,11 +14,8 @@ struct UncoarsenResult {
 // Projection fine[v] = coarse[map[v]] (src/refine.cu:100-111).
 void project(Context& c, std::int64_t n, const std::int32_t* map, const std::int32_t* coarse, std::int32_t* fine);
 
-// Exact directed cut / 2 and part loads.
-std::uint64_t device_cut(Context& c, const DGraph& g, const std::int32_t* labels);
 // Directed edge-weight sum (m for implicit unit weights).
 std::uint64_t device_edge_weight_sum(Context& c, const DGraph& g);
-void device_loads(Context& c, const DGraph& g, const std::int32_t* labels, int k, std::uint64_t* loads_host);
 
 // One refinement level on device labels (run_incremental_refinement).
 LevelStats refine_level(Context& c, const DGraph& g, std::int32_t* labels, std::vector<std::uint64_t>& loads,
