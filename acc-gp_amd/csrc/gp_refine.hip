@@ -34,26 +34,28 @@ constexpr int kJointSeeds = 128;
 constexpr int kJointSide = 4;
 constexpr int kJointArchive = 4;
 
-// Counter slots (device array of u64).
+// Counter slots (device array of u64).  Those that many blocks of one launch
+// add to lie in cache lines of their own: atomics on one line queue up (12 ns
+// each from different waves), on several lines they run side by side.
+constexpr int kCtrLine = 16;  // words of a 128-byte line
 enum Ctr {
     kFrontier = 0,
-    kCand = 1,
-    kTier = 2,  // two slots: medium, heavy
-    kMovers = 4,
-    kDelta = 5,
-    kDonors = 6,
-    kActive = 7,
-    kRowSum = 8,  // entries of the rows scanned by the last LP proposal sweep
+    kCand = kCtrLine,
+    kTier = 2 * kCtrLine,  // two slots: medium, heavy
+    kMovers = 3 * kCtrLine,
+    kDelta = 4 * kCtrLine,
+    kDonors = 5 * kCtrLine,
+    kRowSum = 6 * kCtrLine,  // profiling: entries of the rows scanned by the last LP proposal sweep
     // Tier list counters of the second and third sweep of a round, so that
     // one clear of the whole block at the round start serves all three.
-    kTierB = 9,
-    kTierC = 11,
+    kTierB = 7 * kCtrLine,
+    kTierC = 8 * kCtrLine,
     // (entries, rows) handled by the afterburner, update and repair-proposal
     // sweeps, counted only when the context profiles kernel classes.
-    kEntAfter = 13,
-    kEntUpdate = 15,
-    kEntRepair = 17,
-    kCtrCount = 19
+    kEntAfter = 9 * kCtrLine,
+    kEntUpdate = kEntAfter + 2,
+    kEntRepair = kEntAfter + 4,
+    kCtrCount = 10 * kCtrLine
 };
 
 // Part ids inside refinement: k <= 128 fits a byte, which keeps the label
@@ -481,10 +483,9 @@ struct UpdateBody : RowBody {
                 if (!moves || r.u > v) gain += (std::int64_t)ew_at(a.ew, x) * ((s != old_u) - (tv != new_u));
             });
         gain = t.sum(gain);
-        if (samples && a.samples && t.leader()) {
-            atomicAdd(&a.samples[s].loss, (unsigned long long)(-gain));
-            atomicAdd(&a.samples[s].weight, (unsigned long long)a.vw[v]);
-        }
+        // The commit adds it to the price samples (a mover's gain word is free
+        // until its next proposal resets it).
+        if (samples && t.leader()) set_gain(a, v, gain);
         return RowOut{false, gain};
     }
 };
@@ -527,26 +528,48 @@ struct BoundaryBody : RowBody {
     }
 };
 
-// incremental_commit (incremental.cuh:532-547) with per-block load deltas.
-__global__ void k_commit(RefArgs a, const std::int32_t* list, const unsigned long long* count_ptr, bool lp) {
-    __shared__ unsigned long long delta[kMaxParts];
-    for (int p = threadIdx.x; p < a.k; p += blockDim.x) delta[p] = 0;
-    __syncthreads();
+// incremental_commit (incremental.cuh:532-547) with per-block load deltas;
+// with samples also the repair's price samples, from the gains the update
+// sweep left at the movers.  Sums per part meet in LDS and reach global memory
+// once per block, and the blocks are few and large (kCommitBlocks): k atomics
+// per block on k words queue up, 40 ns a block at k = 64.  (The samples were
+// two global atomics per mover in the update sweep, 77 us of its 90 on the
+// repairs of R-MAT scale 19 at k = 32.)
+constexpr int kCommitThreads = 1024;
+constexpr int kCommitBlocks = 128;
+__global__ void __launch_bounds__(kCommitThreads) k_commit(RefArgs a, const std::int32_t* list,
+                                                           const unsigned long long* count_ptr, bool lp, bool samples) {
+    __shared__ unsigned long long delta[kMaxParts], loss[kMaxParts], weight[kMaxParts];
     const std::int64_t count = (std::int64_t)*count_ptr;
-    for (std::int64_t i = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; i < count;
-         i += (std::int64_t)gridDim.x * blockDim.x) {
+    if (blockIdx.x * (std::int64_t)kCommitThreads >= count) return;
+    for (int p = threadIdx.x; p < a.k; p += kCommitThreads) {
+        delta[p] = 0;
+        loss[p] = 0;
+        weight[p] = 0;
+    }
+    __syncthreads();
+    for (std::int64_t i = blockIdx.x * (std::int64_t)kCommitThreads + threadIdx.x; i < count;
+         i += (std::int64_t)gridDim.x * kCommitThreads) {
         const std::int32_t v = list[i];
         const int s = a.labels[v], t = a.targets[v];
         const unsigned long long w = a.vw[v];
         atomicAdd(&delta[s], 0ULL - w);
         atomicAdd(&delta[t], w);
+        if (samples) {
+            const std::int64_t gain = a.gains32 ? (std::int64_t)a.gains32[v] : a.gains[v];
+            atomicAdd(&loss[s], (unsigned long long)(-gain));
+            atomicAdd(&weight[s], w);
+        }
         a.labels[v] = (Label)t;
         if (lp) a.locks[v] = 1;
         a.member[v] = 1;
     }
     __syncthreads();
-    for (int p = threadIdx.x; p < a.k; p += blockDim.x)
+    for (int p = threadIdx.x; p < a.k; p += kCommitThreads) {
         if (delta[p]) atomicAdd(&a.loads[p], delta[p]);
+        if (loss[p]) atomicAdd(&a.samples[p].loss, loss[p]);
+        if (weight[p]) atomicAdd(&a.samples[p].weight, weight[p]);
+    }
 }
 
 // Sets byte lanes of every state word: state = (state & keep) | put.
@@ -559,13 +582,17 @@ __global__ void k_set_lanes(std::uint32_t* state, std::int64_t n, std::uint32_t 
 // Frontier list from member flags (order irrelevant: per-vertex decisions).
 // Each wave reads kScanRounds x 64 consecutive flags before appending them.
 constexpr int kScanRounds = 8;
+// Large blocks: each reserves its part of the list with one atomic.
+constexpr int kCompactThreads = 1024;
+constexpr int kCompactTile = kCompactThreads * kScanRounds;
 // gate: null, or a device word; when it is zero the launch does nothing (a
 // round of a device-controlled loop that has ended).
 template <typename F>
-__global__ void k_compact_flags(std::int64_t n, F flags, std::int32_t* out, unsigned long long* count,
-                                const unsigned long long* gate) {
+__global__ void __launch_bounds__(kCompactThreads) k_compact_flags(std::int64_t n, F flags, std::int32_t* out,
+                                                                   unsigned long long* count,
+                                                                   const unsigned long long* gate) {
     if (gate && !*gate) return;
-    __shared__ std::int32_t sb[kTierThreads / kWave][kStage];
+    __shared__ std::int32_t sb[kCompactThreads / kWave][kStage];
     Stage st{sb[threadIdx.x / kWave], out, count, 0};
     const std::int64_t wave = (blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x) / kWave;
     const std::int64_t waves = (std::int64_t)gridDim.x * blockDim.x / kWave;
@@ -579,7 +606,7 @@ __global__ void k_compact_flags(std::int64_t n, F flags, std::int32_t* out, unsi
 #pragma unroll
         for (int r = 0; r < kScanRounds; ++r) st.push(f[r], (std::int32_t)(base + r * kWave + lane_id()));
     }
-    st.flush();
+    block_flush<1>({&st}, 0, nullptr);
 }
 
 // ------------------------------------------------------------- repair
@@ -605,9 +632,11 @@ __device__ inline int gain_bucket(const RefArgs& a, double gain) {
 // cleared and loads0 = loads, as k_repair_begin does but for the counter
 // block, which the caller knows to be zero.  The donor test then reads the
 // part loads themselves, the values loads0 is given.
-__global__ void k_repair_donors(RefArgs a, std::int32_t* donors, unsigned long long* count,
-                                unsigned long long* loads0, unsigned long long* counts, std::int64_t ncounts) {
-    __shared__ std::int32_t sb[kTierThreads / kWave][kStage];
+__global__ void __launch_bounds__(kCompactThreads) k_repair_donors(RefArgs a, std::int32_t* donors,
+                                                                   unsigned long long* count,
+                                                                   unsigned long long* loads0,
+                                                                   unsigned long long* counts, std::int64_t ncounts) {
+    __shared__ std::int32_t sb[kCompactThreads / kWave][kStage];
     if (counts)
         for (std::int64_t i = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; i < ncounts;
              i += (std::int64_t)gridDim.x * blockDim.x) {
@@ -637,7 +666,7 @@ __global__ void k_repair_donors(RefArgs a, std::int32_t* donors, unsigned long l
             st.push(d, (std::int32_t)v);
         }
     }
-    st.flush();
+    block_flush<1>({&st}, 0, nullptr);
 }
 
 struct RepairPick {
@@ -2742,7 +2771,7 @@ public:
         const std::int64_t n = a_.n;
         if (!ctr_clear_) fill<unsigned long long>(c_, ctr_.get(), kCtrCount, 0ULL);
         ctr_clear_ = false;
-        hipLaunchKernelGGL(k_compact_flags<StateLane<std::uint8_t>>, dim3(grid_for(n, 256 * kScanRounds, 2048)), dim3(256), 0, s, n,
+        hipLaunchKernelGGL(k_compact_flags<StateLane<std::uint8_t>>, dim3(grid_for(n, kCompactTile, 512)), dim3(kCompactThreads), 0, s, n,
                            a_.member,
                            frontier_.get(), ctr_.get() + kFrontier, nullptr);
         GP_LAUNCH_CHECK();
@@ -2761,8 +2790,7 @@ public:
         const hipStream_t s = c_.stream();
         const std::int64_t n = a_.n;
         unsigned long long* L = ctr_.get() + kCtrCount + a_.k;
-        hipLaunchKernelGGL(k_compact_flags<StateLane<std::uint8_t>>, dim3(grid_for(n, 256 * kScanRounds, 2048)),
-                           dim3(256), 0, s, n, a_.member, frontier_.get(), ctr_.get() + kFrontier, L + kRun);
+        hipLaunchKernelGGL(k_compact_flags<StateLane<std::uint8_t>>, dim3(grid_for(n, kCompactTile, 512)), dim3(kCompactThreads), 0, s, n, a_.member, frontier_.get(), ctr_.get() + kFrontier, L + kRun);
         GP_LAUNCH_CHECK();
         propose_sweeps();
         apply_launch(true, false, true);
@@ -2783,13 +2811,14 @@ public:
 
     // The LP proposal and afterburner sweeps of a round (counter block clear).
     void propose_sweeps() {
+        unsigned long long* row_sum = c_.profiling() ? ctr_.get() + kRowSum : nullptr;
         c_.timed("lp_propose", 0.0, [&] {
             if (narrow_bins())
                 tiers(LpProposeBody<unsigned>{{a_}}, frontier_.get(), 0, ctr_.get() + kFrontier, cand_.get(),
-                      ctr_.get() + kCand, ctr_.get() + kRowSum, a_.k, kTier, true);
+                      ctr_.get() + kCand, row_sum, a_.k, kTier, true);
             else
                 tiers(LpProposeBody<unsigned long long>{{a_}}, frontier_.get(), 0, ctr_.get() + kFrontier, cand_.get(),
-                      ctr_.get() + kCand, ctr_.get() + kRowSum, a_.k, kTier, true);
+                      ctr_.get() + kCand, row_sum, a_.k, kTier, true);
         });
         c_.timed("after", 0.0, [&] {
             if (a_.gains32)
@@ -2906,10 +2935,10 @@ public:
         if (!zeroed) fill<unsigned long long>(c_, ctr_.get() + kDelta, 1, 0ULL);
         if (!zeroed && c_.profiling()) fill<unsigned long long>(c_, ctr_.get() + kEntUpdate, 2, 0ULL);
         c_.timed("update", 0.0, [&] {
-            tiers(UpdateBody{{a_}, samples}, movers_.get(), 0, ctr_.get() + kMovers, nullptr, nullptr,
+            tiers(UpdateBody{{a_}, samples && a_.samples}, movers_.get(), 0, ctr_.get() + kMovers, nullptr, nullptr,
                   ctr_.get() + kDelta, 0, kTierC, zeroed, kEntUpdate);
-            hipLaunchKernelGGL(k_commit, dim3(grid_for(a_.n, 256, 1024)), dim3(256), 0, s, a_, movers_.get(),
-                               ctr_.get() + kMovers, lp);
+            hipLaunchKernelGGL(k_commit, dim3(grid_for(a_.n, kCommitThreads, kCommitBlocks)), dim3(kCommitThreads), 0,
+                               s, a_, movers_.get(), ctr_.get() + kMovers, lp, samples && a_.samples);
             GP_LAUNCH_CHECK();
         });
         if (samples) samples_clear_ = false;
@@ -3124,15 +3153,16 @@ public:
             // (every iteration's last); then one launch starts the iteration.
             const bool zeroed = ctr_clear_;
             ctr_clear_ = false;
-            const int donor_grid = grid_for(n, 256 * kScanRounds, 2048);
+            const int donor_grid = grid_for(n, kCompactTile, 512);
             if (zeroed) {
-                hipLaunchKernelGGL(k_repair_donors, dim3(std::max(donor_grid, grid_for(ncounts))), dim3(256), 0, s, a_,
+                hipLaunchKernelGGL(k_repair_donors, dim3(std::max(donor_grid, grid_for(ncounts, kCompactThreads))),
+                                   dim3(kCompactThreads), 0, s, a_,
                                    cand_.get(), ctr_.get() + kDonors, loads0_.get(), counts_.get(), ncounts);
             } else {
                 hipLaunchKernelGGL(k_repair_begin, dim3(grid_for(ncounts)), dim3(256), 0, s, a_, loads0_.get(),
                                    counts_.get(), ncounts, ctr_.get(), (int)kCtrCount);
                 GP_LAUNCH_CHECK();
-                hipLaunchKernelGGL(k_repair_donors, dim3(donor_grid), dim3(256), 0, s, a_, cand_.get(),
+                hipLaunchKernelGGL(k_repair_donors, dim3(donor_grid), dim3(kCompactThreads), 0, s, a_, cand_.get(),
                                    ctr_.get() + kDonors, nullptr, nullptr, 0);
             }
             GP_LAUNCH_CHECK();
@@ -3254,7 +3284,7 @@ public:
             // profiled entries).
             hipLaunchKernelGGL(k_joint_accept, dim3(ceil_div(active, 256)), dim3(256), 0, s, a_, moves.get(), active,
                                stops.get(), (int)kMovers, (int)kCtrCount);
-            hipLaunchKernelGGL(k_compact_flags<StateLane<std::uint8_t>>, dim3(grid_for(n, 256 * kScanRounds, 2048)), dim3(256), 0, s,
+            hipLaunchKernelGGL(k_compact_flags<StateLane<std::uint8_t>>, dim3(grid_for(n, kCompactTile, 512)), dim3(kCompactThreads), 0, s,
                                n, a_.flags,
                                movers_.get(), ctr_.get() + kMovers, nullptr);
             GP_LAUNCH_CHECK();
