@@ -610,7 +610,9 @@ __global__ void __launch_bounds__(kCompactThreads) k_compact_flags(std::int64_t 
 }
 
 // ------------------------------------------------------------- repair
-__device__ inline int gain_bucket(const RefArgs& a, double gain) {
+// pow15: the table kPow15 (the block's LDS copy: the search is a chain of six
+// loads).
+__device__ inline int gain_bucket(const double* pow15, double gain) {
     if (gain > 0) return 0;
     if (gain == 0) return 1;
     // First j in -23..23 with x <= 1.5^j gives bucket 25 + j (at least 2);
@@ -619,7 +621,7 @@ __device__ inline int gain_bucket(const RefArgs& a, double gain) {
     int lo = 0, hi = 47;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (kPow15.p[mid] < x)
+        if (pow15[mid] < x)
             lo = mid + 1;
         else
             hi = mid;
@@ -739,45 +741,109 @@ __device__ inline bool agg_add(unsigned long long* agg, std::uint32_t key, unsig
     return false;
 }
 
-__device__ inline void repair_finish(const RefArgs& a, std::int64_t v, int s, std::uint64_t w, std::uint64_t current,
-                                     RepairPick best, const unsigned long long* load0, unsigned long long* agg) {
-    if (best.p < 0) {
-        // Slack-weighted hash routing in part order.
-        std::uint64_t tot = 0;
-        for (int p = 0; p < a.k; ++p) {
-            const std::uint64_t l = load0[p];
-            if (p != s && l < a.cap && w <= a.cap - l) {
-                const std::uint64_t sl = a.cap - l;
-                tot = ~0ULL - tot < sl ? ~0ULL : tot + sl;
-            }
+// Words of the table a repair-proposal block stages in LDS: frozen loads, the
+// bucket sums above, prefix sums of the parts' room in part order, their
+// total, the smallest room of a part with any, and the powers of 1.5.
+struct RepairTable {
+    int k;
+    __host__ __device__ int rooms() const { return k + kAggWords; }
+    __host__ __device__ int total() const { return rooms() + k; }
+    __host__ __device__ int smallest() const { return total() + 1; }  // 0: room sums might wrap
+    __host__ __device__ int pow15() const { return total() + 2; }
+    __host__ __device__ int words() const { return pow15() + 48; }
+};
+
+// Destination of a donor without an admissible connected part: a hash picks a
+// unit of room among the parts that can take its weight (in part order).
+// The sum and the search go over all parts, so they are split over the team's
+// lanes; a donor no heavier than the smallest room (every donor of unit
+// weight) can go to any part with room, and the table's prefix sums answer it
+// with a binary search.  One lane walking the k parts twice was most of the
+// light proposal sweep at k = 128: most donors of an overloaded part lie in
+// its inside (300,007 weighted vertices: 55 us a sweep, now 29).
+template <int W>
+__device__ inline int repair_route(const RefArgs& a, std::int64_t v, int s, std::uint64_t w,
+                                   const unsigned long long* tab, int lg) {
+    const RepairTable at{a.k};
+    const std::uint32_t h = mix32((std::uint32_t)v);
+    auto ticket_of = [&](std::uint64_t tot) {
+        return tot <= 0xffffffffULL ? (std::uint64_t)(h % (std::uint32_t)tot) : (std::uint64_t)h % tot;
+    };
+    if (w <= tab[at.smallest()] && tab[at.smallest()]) {
+        const std::uint64_t tot = tab[at.total()];
+        if (!tot) return -1;
+        const std::uint64_t ticket = ticket_of(tot);
+        int lo = 0, hi = a.k - 1;  // the last part whose prefix is at or below the ticket
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (tab[at.rooms() + mid] <= ticket)
+                lo = mid;
+            else
+                hi = mid - 1;
         }
-        best.conn = 0;
-        if (tot) {
-            const std::uint32_t h = mix32((std::uint32_t)v);
-            std::uint64_t ticket = tot <= 0xffffffffULL ? (std::uint64_t)(h % (std::uint32_t)tot) : (std::uint64_t)h % tot;
-            for (int p = 0; p < a.k; ++p) {
-                const std::uint64_t l = load0[p];
-                if (p != s && l < a.cap && w <= a.cap - l) {
-                    const std::uint64_t sl = a.cap - l;
-                    if (ticket < sl) {
-                        best.p = p;
-                        break;
-                    }
-                    ticket -= sl;
-                }
+        return lo;
+    }
+    const int per = (a.k + W - 1) / W, p0 = lg * per, p1 = p0 + per < a.k ? p0 + per : a.k;
+    auto room = [&](int p) {
+        const std::uint64_t l = tab[p];
+        return p != s && l < a.cap && w <= a.cap - l ? a.cap - l : 0;
+    };
+    std::uint64_t own = 0;  // saturating, as the ticket range is
+    for (int p = p0; p < p1; ++p) {
+        const std::uint64_t sl = room(p);
+        own = ~0ULL - own < sl ? ~0ULL : own + sl;
+    }
+    std::uint64_t inc = own;
+    for (int d = 1; d < W; d <<= 1) {
+        const std::uint64_t y = __shfl_up(inc, d, W);
+        if (lg >= d) inc = ~0ULL - inc < y ? ~0ULL : inc + y;
+    }
+    const std::uint64_t before = __shfl_up(inc, 1, W);
+    const std::uint64_t exc = lg ? before : 0;
+    const std::uint64_t tot = __shfl(inc, W - 1, W);
+    if (!tot) return -1;
+    std::uint64_t ticket = ticket_of(tot);
+    int pick = -1;
+    if (ticket >= exc && ticket - exc < own) {
+        ticket -= exc;
+        for (int p = p0; p < p1; ++p) {
+            const std::uint64_t sl = room(p);
+            if (ticket < sl) {
+                pick = p;
+                break;
             }
+            ticket -= sl;
         }
     }
+    for (int d = W / 2; d; d >>= 1) {
+        const int o = __shfl_xor(pick, d, W);
+        pick = o > pick ? o : pick;
+    }
+    return pick;
+}
+
+// Called by every lane of the team; W lanes share the routing (lg: the lane
+// among them) and one writes.
+template <int W>
+__device__ inline void repair_finish(const RefArgs& a, std::int64_t v, int s, std::uint64_t w, std::uint64_t current,
+                                     RepairPick best, unsigned long long* tab, int lg, bool writer) {
+    if (best.p < 0) {
+        best.conn = 0;
+        best.p = repair_route<W>(a, v, s, w, tab, lg);
+    }
+    if (!writer) return;
     a.targets[v] = best.p;
     if (best.p < 0) return;
+    const RepairTable at{a.k};
     const double gain = best.conn >= current ? (double)(best.conn - current) : -(double)(current - best.conn);
-    const std::uint64_t excess = load0[s] - a.cap;
+    const std::uint64_t excess = tab[s] - a.cap;
     const std::uint64_t relief = w < excess ? w : excess;
     const double gpw = gain / (double)relief;
-    const int lb = gain_bucket(a, gpw) * kBalanceSections + (int)(mix32((std::uint32_t)v) % kBalanceSections);
+    const int lb = gain_bucket(reinterpret_cast<const double*>(tab + at.pow15()), gpw) * kBalanceSections +
+                   (int)(mix32((std::uint32_t)v) % kBalanceSections);
     a.bucket[v] = s * kBalanceWidth + lb;
     const std::uint32_t slot = (std::uint32_t)(s * kBalanceWidth + count_slot(lb));
-    if (!agg || !agg_add(agg, slot, (unsigned long long)w)) atomicAdd(&a.counts[slot], (unsigned long long)w);
+    if (!agg_add(tab + a.k, slot, (unsigned long long)w)) atomicAdd(&a.counts[slot], (unsigned long long)w);
 }
 
 template <class Bin>
@@ -786,10 +852,30 @@ struct RepairProposeBody : RowBody {
     // Frozen part loads in LDS for the destination scan, then the block's
     // table of bucket sums: the donors of one part mostly share a few
     // buckets, so each block adds its sums to the global counts once.
-    __host__ __device__ int part_words() const { return a.k + kAggWords; }
+    __host__ __device__ int part_words() const { return RepairTable{a.k}.words(); }
     __device__ void stage(unsigned long long* t) const {
+        const RepairTable at{a.k};
         for (int p = threadIdx.x; p < a.k; p += blockDim.x) t[p] = a.loads0[p];
         for (int i = threadIdx.x; i < kAggWords; i += blockDim.x) t[a.k + i] = i < kAggSlots / 2 ? ~0ULL : 0ULL;
+        for (int i = threadIdx.x; i < 48; i += blockDim.x)
+            t[at.pow15() + i] = (unsigned long long)__double_as_longlong(kPow15.p[i]);
+        if (threadIdx.x < kWave) {
+            std::uint64_t sum = 0, smallest = ~0ULL;
+            for (int p0 = 0; p0 < a.k; p0 += kWave) {
+                const int p = p0 + lane_id();
+                const std::uint64_t l = p < a.k ? a.loads0[p] : a.cap;
+                const std::uint64_t room = l < a.cap ? a.cap - l : 0;
+                if (room && room < smallest) smallest = room;
+                const std::uint64_t inc = wave_inclusive_scan<PlusOp>(room);
+                if (p < a.k) t[at.rooms() + p] = sum + inc - room;
+                sum += __shfl(inc, kWave - 1);
+            }
+            smallest = ~wave_max(~smallest);
+            if (lane_id() == 0) {
+                t[at.total()] = sum;
+                t[at.smallest()] = a.cap < (1ULL << 55) ? smallest : 0;  // at most 128 rooms below 2^63
+            }
+        }
     }
     __device__ void flush(const unsigned long long* t) const {
         const std::uint32_t* keys = reinterpret_cast<const std::uint32_t*>(t + a.k);
@@ -802,7 +888,8 @@ struct RepairProposeBody : RowBody {
         const int s = a.labels[v];
         const std::uint64_t w = a.vw[v];
         RepairPick best{-1, 0, 0};
-        const unsigned long long* load0 = t.part ? t.part : a.loads0;
+        unsigned long long* tab = const_cast<unsigned long long*>(t.part);
+        const unsigned long long* load0 = tab;
         auto consider = [&](int p, std::uint64_t c) {
             if (p == s || !c || load0[p] >= a.cap || w > a.cap - load0[p]) return;
             RepairPick x{p, c, a.cap - load0[p]};
@@ -830,8 +917,9 @@ struct RepairProposeBody : RowBody {
                 for (int p = t.rank(); p < a.k; p += Team::size) consider(p, bh[p]);
             best = team_reduce(t, best);
         }
-        unsigned long long* agg = t.part ? const_cast<unsigned long long*>(t.part) + a.k : nullptr;
-        if (t.leader()) repair_finish(a, v, s, w, current, best, load0, agg);
+        // A block team's waves all find the same route; one thread writes.
+        constexpr int kRouteLanes = Team::size < kWave ? Team::size : kWave;
+        repair_finish<kRouteLanes>(a, v, s, w, current, best, tab, t.rank() % kRouteLanes, t.leader());
         return RowOut{false, 0};
     }
 };
@@ -1262,6 +1350,8 @@ __device__ inline bool choice_better(const Choice& x, const Choice& y) {
 // open falls back to the first untried part in that block-wide order (open
 // when its room admits the donor; rooms after it are no larger).
 constexpr int kChooseLanes = 4;
+// Entries of a connection row per lane loaded before the first is judged.
+constexpr int kChooseBatch = 4;
 __global__ void __launch_bounds__(kTierThreads) k_choose(RefArgs a, ReserveState r, int attempt, std::int32_t* keys,
                                                         unsigned long long* active) {
     constexpr int W = kChooseLanes;
@@ -1297,13 +1387,23 @@ __global__ void __launch_bounds__(kTierThreads) k_choose(RefArgs a, ReserveState
                 const unsigned long long tried0 = r.tried[2 * e], tried1 = r.tried[2 * e + 1];
                 auto closed = [&](int p) { return p == lv || ((((p >> 6) ? tried1 : tried0) >> (p & 63)) & 1ULL); };
                 const int cnt = r.conn_nnz[e];
-                for (int j = lg; j < cnt; j += W) {
-                    const int p = r.conn_part[e * a.k + j];
-                    if (closed(p)) continue;
-                    const unsigned long long avail = room[p];
-                    if (avail < w) continue;
-                    const Choice x{p, r.conn[e * a.k + j], avail};
-                    if (choice_better(x, best)) best = x;
+                for (int j0 = lg; j0 < cnt; j0 += W * kChooseBatch) {
+                    std::uint8_t part[kChooseBatch];
+                    unsigned long long conn[kChooseBatch];
+#pragma unroll
+                    for (int q = 0; q < kChooseBatch; ++q) {
+                        const int j = j0 + q * W;
+                        const std::int64_t x = e * a.k + (j < cnt ? j : cnt - 1);
+                        part[q] = r.conn_part[x];
+                        conn[q] = r.conn[x];
+                    }
+#pragma unroll
+                    for (int q = 0; q < kChooseBatch; ++q) {
+                        const int p = part[q];
+                        if (j0 + q * W >= cnt || closed(p) || room[p] < w) continue;
+                        const Choice x{p, conn[q], room[p]};
+                        if (choice_better(x, best)) best = x;
+                    }
                 }
                 for (int d = W / 2; d; d >>= 1) {
                     const Choice o{__shfl_xor(best.p, d, W), __shfl_xor(best.conn, d, W), __shfl_xor(best.room, d, W)};
@@ -1417,22 +1517,37 @@ __global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, Reserv
             if (i < nl) {
                 d = r.live[pos[i]];
                 const std::int64_t e = d.e;
-                if (!r.done[e] && attempt == 0) {
+                // Independent loads first: the donor's state, then its row in
+                // batches, so that a choice waits for three round trips plus
+                // one per kChooseBatch parts.
+                const std::uint8_t done = r.done[e];
+                const unsigned long long tried0 = r.tried[2 * e], tried1 = r.tried[2 * e + 1];
+                const int cnt = attempt ? r.conn_nnz[e] : 0;
+                if (!done && attempt == 0) {
                     key = a.targets[d.v];
-                } else if (!r.done[e]) {
+                } else if (!done) {
                     const std::uint64_t wd = d.w;
                     const int lv = d.label;
-                    const unsigned long long tried0 = r.tried[2 * e], tried1 = r.tried[2 * e + 1];
                     auto closed = [&](int p) {
                         return p == lv || ((((p >> 6) ? tried1 : tried0) >> (p & 63)) & 1ULL);
                     };
                     Choice best{-1, 0, 0};
-                    const int cnt = r.conn_nnz[e];
-                    for (int j = 0; j < cnt; ++j) {
-                        const int p = r.conn_part[e * a.k + j];
-                        if (closed(p) || room[p] < wd) continue;
-                        const Choice x{p, r.conn[e * a.k + j], room[p]};
-                        if (choice_better(x, best)) best = x;
+                    for (int j0 = 0; j0 < cnt; j0 += kChooseBatch) {
+                        std::uint8_t part[kChooseBatch];
+                        unsigned long long conn[kChooseBatch];
+#pragma unroll
+                        for (int q = 0; q < kChooseBatch; ++q) {
+                            const std::int64_t x = e * a.k + (j0 + q < cnt ? j0 + q : cnt - 1);
+                            part[q] = r.conn_part[x];
+                            conn[q] = r.conn[x];
+                        }
+#pragma unroll
+                        for (int q = 0; q < kChooseBatch; ++q) {
+                            const int p = part[q];
+                            if (j0 + q >= cnt || closed(p) || room[p] < wd) continue;
+                            const Choice x{p, conn[q], room[p]};
+                            if (choice_better(x, best)) best = x;
+                        }
                     }
                     if (best.p < 0)
                         for (int q = 0; q < a.k; ++q) {
