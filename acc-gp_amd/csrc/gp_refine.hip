@@ -1467,59 +1467,210 @@ struct AdmitFn {
 };
 
 // The remaining attempts of a reservation whose live donors fit one block
-// (at most kTailDonors, in rounds of one donor per thread), looped inside one launch: per
-// attempt the same start-of-attempt room and part order, the same choice
-// per donor (attempt 0: the proposed target), the same ranks (exclusive
-// weight prefix per requested part in donor order on top of the part's
-// request total) and admissions as the per-attempt launches, and the loop
-// stops after an attempt with no chooser.  Connection rows must be built
-// before the launch.
+// (at most kTailDonors), looped inside one launch: per attempt the same
+// start-of-attempt room and part order, the same choice per donor (attempt 0:
+// the proposed target), the same ranks (exclusive weight prefix per requested
+// part in donor order on top of the part's request total) and admissions as
+// the per-attempt launches; the loop stops after an attempt with no chooser.
+// Connection rows must be built before the launch.
+//
+// Bound: the latency of an attempt, up to k of them in a chain.  While more
+// donors wait than the block has threads, an attempt goes over them in rounds
+// and their state stays in memory.  Once each has a thread of its own (most
+// launches start there) the rest runs with the donor's record, its tried parts
+// and the first kRowCache entries of its connection row in registers, and the
+// parts' totals in LDS, so that an attempt touches memory only for longer rows
+// and admissions; the part order is made only in attempts where a donor has no
+// open connected part.  Average launch with all state in memory and in this
+// form: weighted graph at k = 128 38 and 18 us, R-MAT scale 18 at k = 64 86
+// and 69, a grid at k = 16 11 and 8.
 constexpr int kTailThreads = 1024;
 constexpr int kTailDonors = 4096;  // donors per launch: rounds of kTailThreads
-__global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, ReserveState r, int attempt0,
-                                                               std::int32_t* movers, unsigned long long* mcount) {
-    constexpr int kWaves = kTailThreads / kWave;
-    __shared__ unsigned long long room[kMaxParts];
-    __shared__ unsigned long long run[kMaxParts];  // this attempt's requests of earlier rounds
-    __shared__ std::uint8_t order[kMaxParts];
-    __shared__ unsigned long long wt[kWaves][kMaxParts];
-    __shared__ std::int32_t sb[kWaves][kStage];
+constexpr int kRowCache = 4;
+
+struct TailShared {
+    static constexpr int kWaves = kTailThreads / kWave;
+    unsigned long long room[kMaxParts];
+    unsigned long long requests[kMaxParts];
+    unsigned long long slack[kMaxParts];
+    unsigned long long run[kMaxParts];  // this attempt's requests of earlier rounds
+    unsigned long long wt[kWaves][kMaxParts];
+    int rank[kMaxParts];
+    std::uint8_t order[kMaxParts];
+    std::int32_t stage[kWaves][kStage];
     // Positions in r.live of the donors still choosing, ascending: donors
     // that were admitted or found no part are dropped after each attempt
     // (they would choose nothing again), so later attempts visit only the
     // waiting ones.  Ranks are weight prefixes over choosing donors in
     // list order, which dropping non-choosers leaves unchanged.
-    __shared__ std::uint16_t pos[kTailDonors];
-    __shared__ int wcount[kWaves];
-    __shared__ int active;
+    std::uint16_t pos[kTailDonors];
+    int wcount[kWaves];
+};
+
+// order[] = the parts by (room desc, id asc); the rooms are in place and the
+// whole block calls it.  Eight threads count each part's rank.
+__device__ inline void tail_order(TailShared& s, int k) {
+    constexpr int kSplit = kTailThreads / kMaxParts;
+    const int t = threadIdx.x, p = t % kMaxParts;
+    if (t < kMaxParts) s.rank[t] = 0;
+    __syncthreads();
+    if (p < k) {
+        const unsigned long long mine = s.room[p];
+        int rank = 0;
+        for (int q = t / kMaxParts; q < k; q += kSplit) rank += s.room[q] > mine || (s.room[q] == mine && q < p);
+        atomicAdd(&s.rank[p], rank);
+    }
+    __syncthreads();
+    if (t < k) s.order[s.rank[t]] = static_cast<std::uint8_t>(t);
+    __syncthreads();
+}
+
+__device__ inline bool part_closed(int p, int label, unsigned long long tried0, unsigned long long tried1) {
+    return p == label || ((((p >> 6) ? tried1 : tried0) >> (p & 63)) & 1ULL);
+}
+
+// The first part in the block's order that is not closed, if the weight fits.
+__device__ inline int tail_fallback(const TailShared& s, int k, std::uint64_t w, int label, unsigned long long tried0,
+                                    unsigned long long tried1) {
+    for (int q = 0; q < k; ++q) {
+        const int p = s.order[q];
+        if (part_closed(p, label, tried0, tried1)) continue;
+        return s.room[p] >= w ? p : -1;
+    }
+    return -1;
+}
+
+// Attempts from `attempt` on with one donor per thread (s.pos[0, nl), at most
+// kTailThreads of them).
+__device__ inline void tail_resident(TailShared& s, const RefArgs& a, const ReserveState& r, int attempt, int nl,
+                                     Stage& st) {
+    const int t = threadIdx.x, w = t / kWave, k = a.k;
+    const int waves = (nl + kWave - 1) / kWave;
+    DonorInfo d{-1, 0, 0, 0};
+    bool alive = false;
+    unsigned long long tried0 = 0, tried1 = 0;
+    int cnt = 0;
+    std::uint8_t part[kRowCache];
+    unsigned long long conn[kRowCache];
+    std::int64_t row = 0;
+#pragma unroll
+    for (int q = 0; q < kRowCache; ++q) {
+        part[q] = 0;
+        conn[q] = 0;
+    }
+    if (t < nl) {
+        d = r.live[s.pos[t]];
+        row = (std::int64_t)d.e * k;
+        alive = !r.done[d.e];
+        tried0 = r.tried[2 * (std::int64_t)d.e];
+        tried1 = r.tried[2 * (std::int64_t)d.e + 1];
+        cnt = r.conn_nnz[d.e];
+#pragma unroll
+        for (int q = 0; q < kRowCache; ++q)
+            if (q < cnt) {
+                part[q] = r.conn_part[row + q];
+                conn[q] = r.conn[row + q];
+            }
+    }
+    const std::uint64_t wd = d.w;
+    for (; attempt < k; ++attempt) {
+        if (t < k) s.room[t] = s.requests[t] < s.slack[t] ? s.slack[t] - s.requests[t] : 0;
+        __syncthreads();
+        int key = -1;
+        if (attempt == 0) {
+            if (alive) key = a.targets[d.v];
+        } else {
+            Choice best{-1, 0, 0};
+            auto consider = [&](int p, unsigned long long c) {
+                if (part_closed(p, d.label, tried0, tried1) || s.room[p] < wd) return;
+                const Choice x{p, c, s.room[p]};
+                if (choice_better(x, best)) best = x;
+            };
+            if (alive) {
+#pragma unroll
+                for (int q = 0; q < kRowCache; ++q)
+                    if (q < cnt) consider(part[q], conn[q]);
+                for (int j0 = kRowCache; j0 < cnt; j0 += kChooseBatch) {
+                    std::uint8_t pp[kChooseBatch];
+                    unsigned long long cc[kChooseBatch];
+#pragma unroll
+                    for (int q = 0; q < kChooseBatch; ++q) {
+                        const std::int64_t x = row + (j0 + q < cnt ? j0 + q : cnt - 1);
+                        pp[q] = r.conn_part[x];
+                        cc[q] = r.conn[x];
+                    }
+#pragma unroll
+                    for (int q = 0; q < kChooseBatch; ++q)
+                        if (j0 + q < cnt) consider(pp[q], cc[q]);
+                }
+            }
+            const bool lost = alive && best.p < 0;
+            if (__syncthreads_or(lost)) {
+                tail_order(s, k);
+                if (lost) best.p = tail_fallback(s, k, wd, d.label, tried0, tried1);
+            }
+            if (best.p < 0) alive = false;  // rooms only shrink: it never chooses again
+            key = best.p;
+        }
+        const std::uint64_t ex = wave_keyed_exclusive(key, key >= 0 ? d.w : 0, s.wt[w]);
+        if (!__syncthreads_or(key >= 0)) break;
+        bool admit = false;
+        if (key >= 0) {
+            std::uint64_t rank = s.requests[key] + ex;
+            for (int j = 0; j < w; ++j) rank += s.wt[j][key];
+            (key >> 6 ? tried1 : tried0) |= 1ULL << (key & 63);
+            if (rank <= s.slack[key] && wd <= s.slack[key] - rank) {
+                a.targets[d.v] = key;
+                a.flags[d.v] = 1;
+                alive = false;
+                admit = true;
+            }
+        }
+        st.push(admit, d.v);
+        if (!__syncthreads_or(alive)) break;
+        if (t < k) {
+            unsigned long long add = 0;
+            for (int j = 0; j < waves; ++j) {
+                add += s.wt[j][t];
+                s.wt[j][t] = 0;
+            }
+            s.requests[t] += add;
+        }
+    }
+}
+
+__global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, ReserveState r, int attempt0,
+                                                               std::int32_t* movers, unsigned long long* mcount) {
+    constexpr int kWaves = TailShared::kWaves;
+    __shared__ TailShared s;
     const int t = threadIdx.x, w = t / kWave;
-    Stage st{sb[w], movers, mcount, 0};
-    for (int i = t; i < kWaves * kMaxParts; i += kTailThreads) wt[i / kMaxParts][i % kMaxParts] = 0;
+    Stage st{s.stage[w], movers, mcount, 0};
+    for (int i = t; i < kWaves * kMaxParts; i += kTailThreads) s.wt[i / kMaxParts][i % kMaxParts] = 0;
     int nl = static_cast<int>(r.nlive);
-    for (int i = t; i < nl; i += kTailThreads) pos[i] = static_cast<std::uint16_t>(i);
-    for (int attempt = attempt0; attempt < a.k; ++attempt) {
-        for (int p = t; p < a.k; p += kTailThreads) {
-            room[p] = r.requests[p] < r.slack[p] ? r.slack[p] - r.requests[p] : 0;
-            run[p] = 0;
+    for (int i = t; i < nl; i += kTailThreads) s.pos[i] = static_cast<std::uint16_t>(i);
+    if (t < a.k) {
+        s.requests[t] = r.requests[t];
+        s.slack[t] = r.slack[t];
+    }
+    __syncthreads();
+    int attempt = attempt0;
+    for (; attempt < a.k && nl > kTailThreads; ++attempt) {
+        if (t < a.k) {
+            s.room[t] = s.requests[t] < s.slack[t] ? s.slack[t] - s.requests[t] : 0;
+            s.run[t] = 0;
         }
-        if (t == 0) active = 0;
         __syncthreads();
-        for (int p = t; p < a.k; p += kTailThreads) {
-            int rank = 0;
-            for (int q = 0; q < a.k; ++q) rank += room[q] > room[p] || (room[q] == room[p] && q < p);
-            order[rank] = static_cast<std::uint8_t>(p);
-        }
-        __syncthreads();
+        tail_order(s, a.k);
+        bool any = false;
         for (int base = 0; base < nl; base += kTailThreads) {
             const int i = base + t;
             int key = -1;
             DonorInfo d{-1, 0, 0, 0};
             if (i < nl) {
-                d = r.live[pos[i]];
+                d = r.live[s.pos[i]];
                 const std::int64_t e = d.e;
                 // Independent loads first: the donor's state, then its row in
-                // batches, so that a choice waits for three round trips plus
-                // one per kChooseBatch parts.
+                // batches.
                 const std::uint8_t done = r.done[e];
                 const unsigned long long tried0 = r.tried[2 * e], tried1 = r.tried[2 * e + 1];
                 const int cnt = attempt ? r.conn_nnz[e] : 0;
@@ -1527,10 +1678,6 @@ __global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, Reserv
                     key = a.targets[d.v];
                 } else if (!done) {
                     const std::uint64_t wd = d.w;
-                    const int lv = d.label;
-                    auto closed = [&](int p) {
-                        return p == lv || ((((p >> 6) ? tried1 : tried0) >> (p & 63)) & 1ULL);
-                    };
                     Choice best{-1, 0, 0};
                     for (int j0 = 0; j0 < cnt; j0 += kChooseBatch) {
                         std::uint8_t part[kChooseBatch];
@@ -1544,33 +1691,27 @@ __global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, Reserv
 #pragma unroll
                         for (int q = 0; q < kChooseBatch; ++q) {
                             const int p = part[q];
-                            if (j0 + q >= cnt || closed(p) || room[p] < wd) continue;
-                            const Choice x{p, conn[q], room[p]};
+                            if (j0 + q >= cnt || part_closed(p, d.label, tried0, tried1) || s.room[p] < wd) continue;
+                            const Choice x{p, conn[q], s.room[p]};
                             if (choice_better(x, best)) best = x;
                         }
                     }
-                    if (best.p < 0)
-                        for (int q = 0; q < a.k; ++q) {
-                            const int p = order[q];
-                            if (closed(p)) continue;
-                            if (room[p] >= wd) best = Choice{p, 0, room[p]};
-                            break;
-                        }
+                    if (best.p < 0) best.p = tail_fallback(s, a.k, wd, d.label, tried0, tried1);
                     if (best.p < 0) r.done[e] = 2;
                     key = best.p;
                 }
             }
             const std::uint32_t wgt = key >= 0 ? d.w : 0;
-            const std::uint64_t ex = wave_keyed_exclusive(key, wgt, wt[w]);
+            const std::uint64_t ex = wave_keyed_exclusive(key, wgt, s.wt[w]);
             __syncthreads();
             bool admit = false;
             if (key >= 0) {
-                atomicAdd(&active, 1);
-                std::uint64_t rank = r.requests[key] + run[key] + ex;
-                for (int j = 0; j < w; ++j) rank += wt[j][key];
+                any = true;
+                std::uint64_t rank = s.requests[key] + s.run[key] + ex;
+                for (int j = 0; j < w; ++j) rank += s.wt[j][key];
                 const std::int64_t e = d.e;
                 r.tried[2 * e + (key >> 6)] |= 1ULL << (key & 63);
-                if (rank <= r.slack[key] && wgt <= r.slack[key] - rank) {
+                if (rank <= s.slack[key] && wgt <= s.slack[key] - rank) {
                     a.targets[d.v] = key;
                     a.flags[d.v] = 1;
                     r.done[e] = 1;
@@ -1579,20 +1720,21 @@ __global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, Reserv
             }
             st.push(admit, d.v);
             __syncthreads();
-            for (int p = t; p < a.k; p += kTailThreads) {
+            if (t < a.k) {
                 unsigned long long add = 0;
                 for (int j = 0; j < kWaves; ++j) {
-                    add += wt[j][p];
-                    wt[j][p] = 0;
+                    add += s.wt[j][t];
+                    s.wt[j][t] = 0;
                 }
-                run[p] += add;
+                s.run[t] += add;
             }
             __syncthreads();
         }
-        const int act = active;
-        for (int p = t; p < a.k; p += kTailThreads) r.requests[p] += run[p];
-        __syncthreads();
-        if (act == 0) break;
+        if (t < a.k) s.requests[t] += s.run[t];
+        if (!__syncthreads_or(any)) {
+            nl = 0;
+            break;
+        }
         // Stable compaction of the waiting donors: thread t keeps its
         // kPer consecutive positions in registers, a block scan of the
         // counts gives where they go.
@@ -1603,25 +1745,25 @@ __global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, Reserv
 #pragma unroll
         for (int j = 0; j < kPer; ++j) {
             const int i = t * kPer + j;
-            q[j] = i < nl ? pos[i] : 0;
+            q[j] = i < nl ? s.pos[i] : 0;
             waiting[j] = i < nl && !r.done[r.live[q[j]].e];
             keep += waiting[j];
         }
         const int inc = wave_inclusive_scan<PlusOp>(keep);
-        if (lane_id() == kWave - 1) wcount[w] = inc;
+        if (lane_id() == kWave - 1) s.wcount[w] = inc;
         __syncthreads();  // every position has been read
         int at = inc - keep, total = 0;
         for (int j = 0; j < kWaves; ++j) {
-            if (j < w) at += wcount[j];
-            total += wcount[j];
+            if (j < w) at += s.wcount[j];
+            total += s.wcount[j];
         }
 #pragma unroll
         for (int j = 0; j < kPer; ++j)
-            if (waiting[j]) pos[at++] = q[j];
+            if (waiting[j]) s.pos[at++] = q[j];
         nl = total;
         __syncthreads();
-        if (nl == 0) break;
     }
+    if (nl > 0) tail_resident(s, a, r, attempt, nl, st);
     st.flush();
 }
 
