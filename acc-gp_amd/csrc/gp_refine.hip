@@ -55,8 +55,13 @@ enum Ctr {
     kEntAfter = 9 * kCtrLine,
     kEntUpdate = kEntAfter + 2,
     kEntRepair = kEntAfter + 4,
-    kCtrCount = 10 * kCtrLine
+    // What a repair iteration's donor selection hands on (written, not added
+    // to; a read-back that clears the counters before it leaves it): eligible
+    // donors, the same when one tail launch takes them (else 0), all donors.
+    kSelected = 10 * kCtrLine,
+    kCtrCount = 11 * kCtrLine
 };
+constexpr int kCtrClear = kSelected;
 
 // Part ids inside refinement: k <= 128 fits a byte, which keeps the label
 // array of a level small enough for the neighbour gathers to hit in cache.
@@ -537,10 +542,26 @@ struct BoundaryBody : RowBody {
 // repairs of R-MAT scale 19 at k = 32.)
 constexpr int kCommitThreads = 1024;
 constexpr int kCommitBlocks = 128;
+//
+// donors: null, or the donor list of the repair iteration, of selected[2]
+// entries: those that were not admitted lose their target
+// (rebalance_graph.cuh:155) unless the reservation is still to come (not
+// settled, and more eligible donors, selected[0], than one tail launch takes,
+// selected[1]).
 __global__ void __launch_bounds__(kCommitThreads) k_commit(RefArgs a, const std::int32_t* list,
-                                                           const unsigned long long* count_ptr, bool lp, bool samples) {
+                                                           const unsigned long long* count_ptr, bool lp, bool samples,
+                                                           const std::int32_t* donors,
+                                                           const unsigned long long* selected, bool settled) {
     __shared__ unsigned long long delta[kMaxParts], loss[kMaxParts], weight[kMaxParts];
     const std::int64_t count = (std::int64_t)*count_ptr;
+    if (donors && (settled || selected[0] == selected[1])) {
+        const std::int64_t nd = (std::int64_t)selected[2];
+        for (std::int64_t i = blockIdx.x * (std::int64_t)kCommitThreads + threadIdx.x; i < nd;
+             i += (std::int64_t)gridDim.x * kCommitThreads) {
+            const std::int32_t v = donors[i];
+            if (!a.flags[v]) a.targets[v] = -1;
+        }
+    }
     if (blockIdx.x * (std::int64_t)kCommitThreads >= count) return;
     for (int p = threadIdx.x; p < a.k; p += kCommitThreads) {
         delta[p] = 0;
@@ -963,14 +984,6 @@ __global__ void __launch_bounds__(kScanThreads) k_bucket_scan(RefArgs a, unsigne
     }
 }
 
-__global__ void k_repair_flag(RefArgs a, const std::int32_t* bstar, std::uint8_t* f) {
-    for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < a.n;
-         v += (std::int64_t)gridDim.x * blockDim.x) {
-        const int b = a.bucket[v];
-        f[v] = b >= 0 && (b % kBalanceWidth) <= bstar[b / kBalanceWidth];
-    }
-}
-
 // Position of the calling lane among the team's lanes with pred set, and
 // their number (every lane of the team calls it).
 template <int W>
@@ -1177,55 +1190,196 @@ __device__ inline void tile_key_sums(const std::int32_t* keys, std::int64_t n, i
     for (int c = threadIdx.x; c < k; c += kTierThreads) S[(std::int64_t)c * nb + blockIdx.x] = acc[c];
 }
 
-// Eligibility (rebalance_graph.cuh:86-110): donors below the boundary
-// bucket are eligible; inside it, while their rank stays below the excess.
-struct EligFn {
-    RefArgs a;
-    const std::int32_t* L;
-    const unsigned long long* prefix;
-    const unsigned long long* excess;
-    std::uint8_t* elig;
-    __device__ std::uint32_t weight(std::int64_t i) const { return a.vw[L[i]]; }
-    __device__ std::int32_t vertex(std::int64_t i) const { return L[i]; }
-    __device__ bool operator()(std::int64_t i, int key, std::uint64_t, std::uint64_t rank) const {
-        elig[i] = prefix[a.bucket[L[i]]] + rank < excess[key];
-        return false;
-    }
+// Donor selection of a repair iteration (rebalance_graph.cuh:86-110): of the
+// donors in vertex order, those whose bucket lies below their part's boundary
+// bucket, and those inside it while the weight of earlier donors of that
+// bucket stays under the excess.  Three launches over tiles of consecutive
+// vertices, none of which the host waits for: each tile's weights inside the
+// boundary buckets; the eligible donors, ranked on top of the earlier tiles'
+// weights, and their number per tile; the list E of them with the state the
+// reservation starts from.  (Flags, a four-launch compaction, a read-back,
+// keys, a scan, ranks, a second compaction and read-back and the set-up took
+// its place before: 14 launches and two host waits, of 20 and three in the
+// whole iteration.)
+constexpr int kSelectThreads = 1024;
+constexpr int kSelectWaves = kSelectThreads / kWave;
+constexpr int kSelectTiles = 1024;  // at most, so that a block can add up the earlier ones
+constexpr int kSelectRounds = 4;    // rounds of kSelectThreads vertices in a tile, more above 4 M vertices
+
+// A live donor as the attempts read it: index into the eligible list, the
+// vertex, its weight and label (one 16-byte load per donor).
+struct DonorInfo {
+    std::int32_t e;
+    std::int32_t v;
+    std::uint32_t w;
+    std::int32_t label;
 };
 
-__global__ void __launch_bounds__(kTierThreads) k_elig_keys(RefArgs a, const std::int32_t* L, std::int64_t nl,
-                                                           const std::int32_t* bstar, int nb, std::int32_t* keys,
-                                                           std::uint8_t* elig, unsigned long long* S) {
-    __shared__ unsigned long long acc[kMaxParts];
-    for (int c = threadIdx.x; c < kMaxParts; c += kTierThreads) acc[c] = 0;
-    const std::int64_t base = blockIdx.x * (std::int64_t)kKeyTile;
-    for (int r = 0; r < kKeyRounds; ++r) {
-        const std::int64_t i = base + r * kTierThreads + threadIdx.x;
-        if (i >= nl) break;
-        const int b = a.bucket[L[i]];
-        const int s = b / kBalanceWidth, lb = b % kBalanceWidth;
-        keys[i] = lb == bstar[s] ? s : -1;
-        elig[i] = lb < bstar[s];
+struct SelectState {
+    const std::int32_t* bstar;          // boundary bucket per part, -1 when not overloaded
+    const unsigned long long* prefix;   // weight below each bucket of its part
+    const unsigned long long* excess;   // weight a part has to lose
+    unsigned long long* S;              // tiles x k boundary weights
+    std::int32_t* counts;               // eligible donors per tile
+    std::uint8_t* elig;                 // n
+    // The reservation's start: eligible donors, their records and cleared
+    // state (done, tried bits), each part's room and request total.
+    std::int32_t* E;
+    DonorInfo* live;
+    std::uint8_t* done;
+    unsigned long long* tried;
+    unsigned long long* slack;
+    unsigned long long* requests;
+    unsigned long long* selected;       // kSelected words
+    unsigned long long tail_limit;      // donors one tail launch takes
+};
+
+__device__ inline void select_place(const RefArgs& a, const SelectState& q, std::int64_t j, std::int32_t v) {
+    q.E[j] = v;
+    q.live[j] = DonorInfo{static_cast<std::int32_t>(j), v, a.vw[v], (std::int32_t)a.labels[v]};
+    q.done[j] = 0;
+    q.tried[2 * j] = 0;
+    q.tried[2 * j + 1] = 0;
+}
+__device__ inline void select_parts(const RefArgs& a, const SelectState& q) {
+    for (int p = threadIdx.x; p < a.k; p += blockDim.x) {
+        q.slack[p] = a.loads0[p] < a.cap ? a.cap - a.loads0[p] : 0;
+        q.requests[p] = 0;
     }
-    EligFn f{a, L, nullptr, nullptr, nullptr};
-    tile_key_sums(keys, nl, a.k, nb, f, acc, S);
+}
+// One thread, once the number of eligible donors is known.
+__device__ inline void select_counts(const RefArgs& a, const SelectState& q, unsigned long long ne) {
+    q.selected[0] = ne;
+    q.selected[1] = ne <= q.tail_limit ? ne : 0;
+    q.selected[2] = a.ctr[kDonors];
+}
+
+__global__ void __launch_bounds__(kSelectThreads) k_select_weights(RefArgs a, SelectState q, int rounds) {
+    __shared__ unsigned long long acc[kMaxParts];
+    __shared__ std::int32_t star[kMaxParts];
+    for (int p = threadIdx.x; p < a.k; p += kSelectThreads) {
+        acc[p] = 0;
+        star[p] = q.bstar[p];
+    }
+    __syncthreads();
+    const std::int64_t base = (std::int64_t)blockIdx.x * rounds * kSelectThreads + threadIdx.x;
+    for (int r = 0; r < rounds; ++r) {
+        const std::int64_t v = base + (std::int64_t)r * kSelectThreads;
+        const int b = v < a.n ? a.bucket[v] : -1;
+        if (b >= 0 && b % kBalanceWidth == star[b / kBalanceWidth])
+            atomicAdd(&acc[b / kBalanceWidth], (unsigned long long)a.vw[v]);
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < a.k; p += kSelectThreads) q.S[(std::int64_t)blockIdx.x * a.k + p] = acc[p];
+}
+
+__global__ void __launch_bounds__(kSelectThreads) k_select_eligible(RefArgs a, SelectState q, int rounds) {
+    __shared__ unsigned long long run[kMaxParts];
+    __shared__ unsigned long long wt[kSelectWaves][kMaxParts];
+    __shared__ std::int32_t star[kMaxParts];
+    __shared__ int count;
+    const int t = threadIdx.x, w = t / kWave;
+    for (int i = t; i < kSelectWaves * kMaxParts; i += kSelectThreads) wt[i / kMaxParts][i % kMaxParts] = 0;
+    if (t < kMaxParts) {
+        run[t] = 0;
+        star[t] = t < a.k ? q.bstar[t] : -1;
+    }
+    if (t == 0) count = 0;
+    __syncthreads();
+    // Boundary weights of the earlier tiles, eight threads per part.
+    const int p = t % kMaxParts;
+    if (p < a.k && star[p] >= 0) {
+        unsigned long long sum = 0;
+        for (int tile = t / kMaxParts; tile < (int)blockIdx.x; tile += kSelectThreads / kMaxParts)
+            sum += q.S[(std::int64_t)tile * a.k + p];
+        if (sum) atomicAdd(&run[p], sum);
+    }
+    __syncthreads();
+    const std::int64_t base = (std::int64_t)blockIdx.x * rounds * kSelectThreads + t;
+    int mine = 0;
+    for (int r = 0; r < rounds; ++r) {
+        const std::int64_t v = base + (std::int64_t)r * kSelectThreads;
+        const int b = v < a.n ? a.bucket[v] : -1;
+        int key = -1;
+        bool el = false;
+        std::uint32_t wgt = 0;
+        if (b >= 0) {
+            const int s = b / kBalanceWidth, lb = b % kBalanceWidth;
+            el = lb < star[s];
+            if (lb == star[s]) {
+                key = s;
+                wgt = a.vw[v];
+            }
+        }
+        if (__syncthreads_or(key >= 0)) {
+            const std::uint64_t ex = wave_keyed_exclusive(key, wgt, wt[w]);
+            __syncthreads();
+            if (key >= 0) {
+                std::uint64_t rank = run[key] + ex;
+                for (int j = 0; j < w; ++j) rank += wt[j][key];
+                el = q.prefix[b] + rank < q.excess[key];
+            }
+            __syncthreads();
+            if (t < a.k) {
+                unsigned long long add = 0;
+                for (int j = 0; j < kSelectWaves; ++j) {
+                    add += wt[j][t];
+                    wt[j][t] = 0;
+                }
+                run[t] += add;
+            }
+        }
+        if (v < a.n) q.elig[v] = el;
+        mine += __popcll(__ballot(el));
+    }
+    if (lane_id() == 0 && mine) atomicAdd(&count, mine);
+    __syncthreads();
+    if (t == 0) q.counts[blockIdx.x] = count;
+}
+
+__global__ void __launch_bounds__(kSelectThreads) k_select_place(RefArgs a, SelectState q, int rounds) {
+    __shared__ int wsum[kSelectWaves];
+    __shared__ int before;
+    const int t = threadIdx.x, w = t / kWave;
+    if (t == 0) before = 0;
+    __syncthreads();
+    int earlier = t < (int)blockIdx.x ? q.counts[t] : 0;
+    earlier = wave_sum(earlier);
+    if (lane_id() == 0 && earlier) atomicAdd(&before, earlier);
+    if (blockIdx.x == 0) select_parts(a, q);
+    __syncthreads();
+    std::int64_t at = before;
+    const std::int64_t base = (std::int64_t)blockIdx.x * rounds * kSelectThreads + t;
+    for (int r = 0; r < rounds; ++r) {
+        const std::int64_t v = base + (std::int64_t)r * kSelectThreads;
+        const bool el = v < a.n && q.elig[v];
+        const unsigned long long m = __ballot(el);
+        if (lane_id() == 0) wsum[w] = __popcll(m);
+        __syncthreads();
+        std::int64_t pos = at;
+        for (int j = 0; j < kSelectWaves; ++j) {
+            if (j < w) pos += wsum[j];
+            at += wsum[j];
+        }
+        if (el) select_place(a, q, pos + __popcll(m & ((1ULL << lane_id()) - 1ULL)), (std::int32_t)v);
+        __syncthreads();
+    }
+    if (blockIdx.x == gridDim.x - 1 && t == 0) select_counts(a, q, (unsigned long long)at);
 }
 
 // Donor selection of a repair iteration on a level of at most
 // kSelectSmallMax vertices, in one block: the flagged donors (bucket at or
 // below the part's boundary bucket) in vertex order, then their eligibility
 // (below the boundary bucket, or inside it while the weighted rank among
-// earlier donors of that bucket stays under the excess), compacted into E
-// with their number in *ne.  One pass in index order gives the same ranks
-// as the tiled form (per-tile sums, a scan over tiles, in-tile ranks), which
-// larger levels use.
+// earlier donors of that bucket stays under the excess), placed as the
+// three launches above do.
 constexpr int kDonorThreads = 1024;
 constexpr int kDonorWaves = kDonorThreads / kWave;
 
-__global__ void __launch_bounds__(kDonorThreads) k_donors_small(RefArgs a, const std::int32_t* bstar,
-                                                               const unsigned long long* prefix,
-                                                               const unsigned long long* excess, std::int32_t* E,
-                                                               std::int64_t* ne) {
+__global__ void __launch_bounds__(kDonorThreads) k_donors_small(RefArgs a, SelectState q) {
+    const std::int32_t* bstar = q.bstar;
+    const unsigned long long* prefix = q.prefix;
+    const unsigned long long* excess = q.excess;
     __shared__ std::int32_t L[kSelectSmallMax];
     __shared__ unsigned long long wt[kDonorWaves][kMaxParts];
     __shared__ unsigned long long run[kMaxParts];
@@ -1239,8 +1393,9 @@ __global__ void __launch_bounds__(kDonorThreads) k_donors_small(RefArgs a, const
     }
     if (t == 0) base = 0;
     __syncthreads();
-    // Stable compaction of `mine` over one round: writes dst[base + rank].
-    auto compact = [&](bool mine, std::int32_t value, std::int32_t* dst) {
+    select_parts(a, q);
+    // Stable compaction of `mine` over one round: place(base + rank).
+    auto compact = [&](bool mine, auto place) {
         const unsigned long long m = __ballot(mine);
         if (lane == 0) wsum[w] = __popcll(m);
         __syncthreads();
@@ -1249,7 +1404,7 @@ __global__ void __launch_bounds__(kDonorThreads) k_donors_small(RefArgs a, const
             pre += j < w ? wsum[j] : 0;
             total += wsum[j];
         }
-        if (mine) dst[pre + __popcll(m & lt)] = value;
+        if (mine) place(pre + __popcll(m & lt));
         __syncthreads();
         if (t == 0) base += total;
         __syncthreads();
@@ -1261,7 +1416,7 @@ __global__ void __launch_bounds__(kDonorThreads) k_donors_small(RefArgs a, const
             const int b = a.bucket[v];
             f = b >= 0 && (b % kBalanceWidth) <= bstar[b / kBalanceWidth];
         }
-        compact(f, static_cast<std::int32_t>(v), L);
+        compact(f, [&](int j) { L[j] = static_cast<std::int32_t>(v); });
     }
     const int nl = base;
     __syncthreads();
@@ -1299,19 +1454,10 @@ __global__ void __launch_bounds__(kDonorThreads) k_donors_small(RefArgs a, const
             }
             run[c] += add;
         }
-        compact(el, v, E);
+        compact(el, [&](int j) { select_place(a, q, j, v); });
     }
-    if (t == 0) *ne = base;
+    if (t == 0) select_counts(a, q, (unsigned long long)base);
 }
-
-// A live donor as the attempts read it: index into the eligible list, the
-// vertex, its weight and label (one 16-byte load per donor).
-struct DonorInfo {
-    std::int32_t e;
-    std::int32_t v;
-    std::uint32_t w;
-    std::int32_t label;
-};
 
 struct ReserveState {
     const std::int32_t* E;           // eligible donors in vertex order
@@ -1325,6 +1471,7 @@ struct ReserveState {
     unsigned long long* tried;       // ne x 2
     const DonorInfo* live;           // donors still choosing, ascending
     std::int64_t nlive;
+    const unsigned long long* nlive_dev;  // null, or where the device keeps nlive (the tail launch only)
 };
 
 // Choices of one attempt, one 4-lane group per live donor (many donors in
@@ -1646,7 +1793,8 @@ __global__ void __launch_bounds__(kTailThreads) k_reserve_tail(RefArgs a, Reserv
     const int t = threadIdx.x, w = t / kWave;
     Stage st{s.stage[w], movers, mcount, 0};
     for (int i = t; i < kWaves * kMaxParts; i += kTailThreads) s.wt[i / kMaxParts][i % kMaxParts] = 0;
-    int nl = static_cast<int>(r.nlive);
+    int nl = static_cast<int>(r.nlive_dev ? *r.nlive_dev : r.nlive);
+    if (nl == 0) return;
     for (int i = t; i < nl; i += kTailThreads) s.pos[i] = static_cast<std::uint16_t>(i);
     if (t < a.k) {
         s.requests[t] = r.requests[t];
@@ -1777,29 +1925,6 @@ __global__ void k_gather_info(const DonorInfo* src, const std::int32_t* idx, std
     for (std::int64_t j = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; j < count;
          j += (std::int64_t)gridDim.x * blockDim.x)
         dst[j] = src[idx[j]];
-}
-
-// Set-up of a reservation in one launch: the eligible donors E[j] =
-// L[idx[j]] in vertex order (E already holds them when idx is null; then
-// L is E) with their packed records, cleared per-donor
-// state (done, tried bits) and each part's room and request total.
-__global__ void k_reserve_setup(RefArgs a, const std::int32_t* L, const std::int32_t* idx, std::int64_t ne,
-                                std::int32_t* E, DonorInfo* live, std::uint8_t* done, unsigned long long* tried,
-                                unsigned long long* slack, unsigned long long* requests) {
-    for (std::int64_t j = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; j < ne;
-         j += (std::int64_t)gridDim.x * blockDim.x) {
-        const std::int32_t v = idx ? L[idx[j]] : L[j];
-        if (idx) E[j] = v;
-        live[j] = DonorInfo{static_cast<std::int32_t>(j), v, a.vw[v], (std::int32_t)a.labels[v]};
-        done[j] = 0;
-        tried[2 * j] = 0;
-        tried[2 * j + 1] = 0;
-    }
-    if (blockIdx.x == 0)
-        for (int p = threadIdx.x; p < a.k; p += blockDim.x) {
-            slack[p] = a.loads0[p] < a.cap ? a.cap - a.loads0[p] : 0;
-            requests[p] = 0;
-        }
 }
 
 // Start of a repair iteration in one launch: freezes the part loads
@@ -2033,16 +2158,6 @@ __global__ void k_lp_keep(const unsigned long long* flag, const Label* labels, L
     for (std::int64_t v = words * 16 + blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
          v += (std::int64_t)gridDim.x * blockDim.x)
         best[v] = labels[v];
-}
-
-// Donors that were not admitted carry no target (rebalance_graph.cuh:155).
-__global__ void k_repair_clear(RefArgs a, const std::int32_t* donors, const unsigned long long* count_ptr) {
-    const std::int64_t count = (std::int64_t)*count_ptr;
-    for (std::int64_t i = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; i < count;
-         i += (std::int64_t)gridDim.x * blockDim.x) {
-        const std::int32_t v = donors[i];
-        if (!a.flags[v]) a.targets[v] = -1;
-    }
 }
 
 // ------------------------------------------------------------ exchange
@@ -3026,9 +3141,9 @@ public:
     template <class Body>
     void tiers(const Body& body, const std::int32_t* list, std::int64_t n, const unsigned long long* count,
                std::int32_t* out, unsigned long long* out_count, unsigned long long* acc, int scratch,
-               int slot = kTier, bool zeroed = false, int entries_slot = -1) {
+               int slot = kTier, bool zeroed = false, int entries_slot = -1, std::int64_t max_rows = -1) {
         run_tiers(c_, body, list, n, count, medium_.get(), heavy_.get(), ctr_.get() + slot, out, out_count, acc,
-                  scratch, a_.n, g_.row_len_bound, zeroed,
+                  scratch, max_rows < 0 ? a_.n : max_rows, g_.row_len_bound, zeroed,
                   entries_slot >= 0 && c_.profiling() ? ctr_.get() + entries_slot : nullptr);
     }
 
@@ -3197,7 +3312,8 @@ public:
     // Update + commit of the current mover list.  zeroed: the delta and
     // third-sweep tier counters are still zero from the counter block's
     // clear at the start of the round or repair iteration.
-    void apply_launch(bool lp, bool samples, bool zeroed) {
+    // donors, settled: as k_commit takes them (null outside repair).
+    void apply_launch(bool lp, bool samples, bool zeroed, const std::int32_t* donors = nullptr, bool settled = true) {
         const hipStream_t s = c_.stream();
         if (!zeroed) fill<unsigned long long>(c_, ctr_.get() + kDelta, 1, 0ULL);
         if (!zeroed && c_.profiling()) fill<unsigned long long>(c_, ctr_.get() + kEntUpdate, 2, 0ULL);
@@ -3205,18 +3321,21 @@ public:
             tiers(UpdateBody{{a_}, samples && a_.samples}, movers_.get(), 0, ctr_.get() + kMovers, nullptr, nullptr,
                   ctr_.get() + kDelta, 0, kTierC, zeroed, kEntUpdate);
             hipLaunchKernelGGL(k_commit, dim3(grid_for(a_.n, kCommitThreads, kCommitBlocks)), dim3(kCommitThreads), 0,
-                               s, a_, movers_.get(), ctr_.get() + kMovers, lp, samples && a_.samples);
+                               s, a_, movers_.get(), ctr_.get() + kMovers, lp, samples && a_.samples, donors, ctr_.get() + kSelected,
+                               settled);
             GP_LAUNCH_CHECK();
         });
         if (samples) samples_clear_ = false;
     }
 
-    std::int64_t apply(bool lp, bool samples, std::int64_t& delta, bool zeroed = false) {
-        apply_launch(lp, samples, zeroed);
+    std::int64_t apply(bool lp, bool samples, std::int64_t& delta, bool zeroed = false,
+                       const std::int32_t* donors = nullptr, bool settled = true) {
+        apply_launch(lp, samples, zeroed, donors, settled);
         std::vector<unsigned long long> h(static_cast<std::size_t>(kCtrCount + a_.k));
         // The read also clears the counters (not the part loads behind them).
-        c_.read_clear(h.data(), ctr_.get(), h.size(), kCtrCount);
+        c_.read_clear(h.data(), ctr_.get(), h.size(), kCtrClear);
         ctr_clear_ = true;
+        selected_ = (std::int64_t)h[kSelected];
         // With no row above kTierLight entries no medium launch was made; a
         // row the light launch deferred would have gone unprocessed.
         if (g_.row_len_bound <= static_cast<std::uint64_t>(kTierLight) && (h[kTier] || h[kTierB] || h[kTierC]))
@@ -3265,49 +3384,73 @@ public:
         ++st_.strict_checks;
     }
 
-    // Sparse connection rows of the listed donors (ConnBody by the row
-    // tiers over the positions [0, ne) of E).
-    void conn_rows(const std::int32_t* E, std::int64_t ne, const std::uint8_t* skip, unsigned long long* vals,
-                   std::uint8_t* parts, std::uint8_t* nnz) {
+    // Sparse connection rows of the eligible donors (ConnBody by the row
+    // tiers over the positions [0, ne) of E): ne from the device when
+    // count_dev is not null, then at most max_rows.
+    void conn_rows(const std::int32_t* E, std::int64_t ne, const unsigned long long* count_dev, std::int64_t max_rows,
+                   const std::uint8_t* skip, unsigned long long* vals, std::uint8_t* parts, std::uint8_t* nnz) {
         // Within a repair iteration the second sweep's tier counters are
         // still zero from the iteration's counter clear (k_repair_begin).
         if (narrow_bins())
-            tiers(ConnBody<unsigned>{{a_}, E, skip, vals, parts, nnz}, nullptr, ne, nullptr, nullptr, nullptr, nullptr,
-                  a_.k, kTierB, true);
+            tiers(ConnBody<unsigned>{{a_}, E, skip, vals, parts, nnz}, nullptr, ne, count_dev, nullptr, nullptr, nullptr,
+                  a_.k, kTierB, true, -1, max_rows);
         else
-            tiers(ConnBody<unsigned long long>{{a_}, E, skip, vals, parts, nnz}, nullptr, ne, nullptr, nullptr, nullptr,
-                  nullptr, a_.k, kTierB, true);
+            tiers(ConnBody<unsigned long long>{{a_}, E, skip, vals, parts, nnz}, nullptr, ne, count_dev, nullptr,
+                  nullptr, nullptr, a_.k, kTierB, true, -1, max_rows);
     }
 
-    // Receiver reservation over the flagged donors L (vertex order).
-    void reserve(const std::int32_t* L, std::int64_t nl, const unsigned long long* prefix, const std::int32_t* bstar,
-                 const unsigned long long* excess) {
-        const hipStream_t s = c_.stream();
-        const int k = a_.k;
-        const int nbl = static_cast<int>(ceil_div(nl, kKeyTile));
-        DBuf<std::int32_t> keys = c_.buf<std::int32_t>(static_cast<std::size_t>(nl));
-        DBuf<unsigned long long> S = c_.buf<unsigned long long>(static_cast<std::size_t>(nbl) * k);
-        DBuf<std::uint8_t> elig = c_.buf<std::uint8_t>(static_cast<std::size_t>(nl));
-        hipLaunchKernelGGL(k_elig_keys, dim3(nbl), dim3(kTierThreads), 0, s, a_, L, nl, bstar, nbl, keys.get(),
-                           elig.get(), S.get());
-        GP_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_keyed_scan, dim3(1), dim3(kKeyScanThreads), 0, s, S.get(), nbl, k, nullptr);
-        GP_LAUNCH_CHECK();
-        hipLaunchKernelGGL((k_keyed_apply<EligFn>), dim3(nbl), dim3(kTierThreads), 0, s, keys.get(), nl, S.get(), nbl,
-                           EligFn{a_, L, prefix, excess, elig.get()}, nullptr, nullptr);
-        GP_LAUNCH_CHECK();
-        DBuf<std::int32_t> idx = c_.buf<std::int32_t>(static_cast<std::size_t>(nl));
-        DBuf<std::int64_t> cnt = c_.buf<std::int64_t>(1);
-        stable_select(c_, elig.get(), nl, idx.get(), cnt.get());
-        const std::int64_t ne = c_.read_scalar(cnt.get());
-        if (ne <= 0) return;
-        DBuf<std::int32_t> E = c_.buf<std::int32_t>(static_cast<std::size_t>(ne));
-        reserve_donors(E.get(), L, idx.get(), ne);
+    // Arrays of a level's repair iterations: the donor selection's, and the
+    // connection rows of what one tail launch takes.
+    struct RepairBuffers {
+        DBuf<unsigned long long> prefix, excess, S, tried, slack, requests, conn;
+        DBuf<std::int32_t> bstar, counts, E;
+        DBuf<std::uint8_t> elig, done, conn_part, conn_nnz;
+        DBuf<DonorInfo> live;
+        int rounds = 0, tiles = 0;
+    };
+
+    RepairBuffers repair_buffers() {
+        RepairBuffers b;
+        const std::size_t n = static_cast<std::size_t>(a_.n), k = static_cast<std::size_t>(a_.k);
+        b.rounds = std::max(kSelectRounds, ceil_div(a_.n, (std::int64_t)kSelectTiles * kSelectThreads));
+        b.tiles = ceil_div(a_.n, (std::int64_t)b.rounds * kSelectThreads);
+        b.prefix = c_.buf<unsigned long long>(k * kBalanceWidth);
+        b.bstar = c_.buf<std::int32_t>(k);
+        b.excess = c_.buf<unsigned long long>(k);
+        b.S = c_.buf<unsigned long long>(static_cast<std::size_t>(b.tiles) * k);
+        b.counts = c_.buf<std::int32_t>(static_cast<std::size_t>(b.tiles));
+        b.elig = c_.buf<std::uint8_t>(n);
+        b.E = c_.buf<std::int32_t>(n);
+        b.live = c_.buf<DonorInfo>(n);
+        b.done = c_.buf<std::uint8_t>(n);
+        b.tried = c_.buf<unsigned long long>(2 * n);
+        b.slack = c_.buf<unsigned long long>(k);
+        b.requests = c_.buf<unsigned long long>(k);
+        const std::size_t tail = static_cast<std::size_t>(std::min<std::int64_t>(a_.n, kTailDonors));
+        b.conn = c_.buf<unsigned long long>(tail * k);
+        b.conn_part = c_.buf<std::uint8_t>(tail * k);
+        b.conn_nnz = c_.buf<std::uint8_t>(tail);
+        return b;
     }
 
-    // Reservation over the ne eligible donors E[j] = L[idx[j]] (E = L when
-    // idx is null: the list is already the eligible donors).
-    void reserve_donors(std::int32_t* E, const std::int32_t* L, const std::int32_t* idx, std::int64_t ne) {
+    // Reservation of the selected donors when one tail launch takes them all:
+    // their connection rows (those of donors admitted in attempt 0 go unused),
+    // then all attempts.  The count stays on the device; with more donors
+    // than that it is zero there and both launches do nothing.
+    void reserve_tail(RepairBuffers& b) {
+        const unsigned long long* count = ctr_.get() + kSelected + 1;
+        const std::int64_t rows = std::min<std::int64_t>(a_.n, kTailDonors);
+        conn_rows(b.E.get(), 0, count, rows, nullptr, b.conn.get(), b.conn_part.get(), b.conn_nnz.get());
+        const ReserveState r{b.E.get(),        rows,           b.conn.get(),  b.conn_part.get(), b.conn_nnz.get(),
+                             b.requests.get(), b.slack.get(),  b.done.get(),  b.tried.get(),     b.live.get(),
+                             0,                count};
+        hipLaunchKernelGGL(k_reserve_tail, dim3(1), dim3(kTailThreads), 0, c_.stream(), a_, r, 0, movers_.get(),
+                           ctr_.get() + kMovers);
+        GP_LAUNCH_CHECK();
+    }
+
+    // Reservation of ne selected donors, more than one tail launch takes.
+    void reserve_groups(RepairBuffers& b, std::int64_t ne) {
         const hipStream_t s = c_.stream();
         const int k = a_.k;
         DBuf<std::int32_t> keys = c_.buf<std::int32_t>(static_cast<std::size_t>(ne));
@@ -3318,16 +3461,12 @@ public:
         DBuf<unsigned long long> conn = c_.buf<unsigned long long>(static_cast<std::size_t>(ne) * k);
         DBuf<std::uint8_t> conn_part = c_.buf<std::uint8_t>(static_cast<std::size_t>(ne) * k);
         DBuf<std::uint8_t> conn_nnz = c_.buf<std::uint8_t>(static_cast<std::size_t>(ne));
-        DBuf<unsigned long long> requests = c_.buf<unsigned long long>(static_cast<std::size_t>(k));
-        DBuf<unsigned long long> slack = c_.buf<unsigned long long>(static_cast<std::size_t>(k));
-        DBuf<std::uint8_t> done = c_.buf<std::uint8_t>(static_cast<std::size_t>(ne));
-        DBuf<unsigned long long> tried = c_.buf<unsigned long long>(static_cast<std::size_t>(ne) * 2);
-        DBuf<DonorInfo> live = c_.buf<DonorInfo>(static_cast<std::size_t>(ne));
-        hipLaunchKernelGGL(k_reserve_setup, dim3(grid_for(ne)), dim3(256), 0, s, a_, L, idx, ne, E, live.get(),
-                           done.get(), tried.get(), slack.get(), requests.get());
-        GP_LAUNCH_CHECK();
-        ReserveState r{E,           ne,         conn.get(), conn_part.get(), conn_nnz.get(), requests.get(),
-                       slack.get(), done.get(), tried.get(), live.get(),     ne};
+        DBuf<DonorInfo> live;  // the waiting donors after a compaction
+        const std::int32_t* E = b.E.get();
+        std::uint8_t* done = b.done.get();
+        unsigned long long* requests = b.requests.get();
+        ReserveState r{E,        ne,            conn.get(), conn_part.get(), conn_nnz.get(), requests,
+                       b.slack.get(), done, b.tried.get(), b.live.get(), ne, nullptr};
         // Attempts run in groups between host checks: an attempt without a
         // chooser changes nothing (no tried bits, no requests, no admissions),
         // so the attempts after the last active one are no-ops.  Between
@@ -3336,16 +3475,6 @@ public:
         constexpr int kAttemptGroup = 4;
         constexpr std::int64_t kCompactMin = 4096;
         DBuf<unsigned long long> active = c_.buf<unsigned long long>(kAttemptGroup);
-        if (ne <= kTailDonors) {
-            // Every donor's connection row first (the rows of donors admitted
-            // in attempt 0 go unused), then all attempts in one launch.
-            conn_rows(E, ne, nullptr, conn.get(), conn_part.get(), conn_nnz.get());
-            GP_LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_reserve_tail, dim3(1), dim3(kTailThreads), 0, s, a_, r, 0, movers_.get(),
-                               ctr_.get() + kMovers);
-            GP_LAUNCH_CHECK();
-            return;
-        }
         for (int attempt = 0; attempt < k;) {
             const int group = std::min(kAttemptGroup, k - attempt);
             const std::int64_t nlv = r.nlive;
@@ -3353,8 +3482,7 @@ public:
             fill<unsigned long long>(c_, active.get(), kAttemptGroup, 0ULL);
             for (int j = 0; j < group; ++j, ++attempt) {
                 if (attempt == 1) {
-                    conn_rows(E, ne, done.get(), conn.get(), conn_part.get(), conn_nnz.get());
-                    GP_LAUNCH_CHECK();
+                    conn_rows(E, ne, nullptr, -1, done, conn.get(), conn_part.get(), conn_nnz.get());
                 }
                 // Blocks stride over the donors: the per-block room table and
                 // part order are set up once per block.
@@ -3365,7 +3493,7 @@ public:
                                    nb, DonorWeight{r.live}, S.get());
                 GP_LAUNCH_CHECK();
                 // Ranks start at the start-of-attempt totals; totals advance.
-                hipLaunchKernelGGL(k_keyed_scan, dim3(1), dim3(kKeyScanThreads), 0, s, S.get(), nb, k, requests.get());
+                hipLaunchKernelGGL(k_keyed_scan, dim3(1), dim3(kKeyScanThreads), 0, s, S.get(), nb, k, requests);
                 GP_LAUNCH_CHECK();
                 hipLaunchKernelGGL((k_keyed_apply<AdmitFn>), dim3(nb), dim3(kTierThreads), 0, s, keys.get(), nlv,
                                    S.get(), nb, AdmitFn{a_, r}, movers_.get(), ctr_.get() + kMovers);
@@ -3376,7 +3504,7 @@ public:
                 DBuf<std::uint8_t> lf = c_.buf<std::uint8_t>(static_cast<std::size_t>(nlv));
                 DBuf<std::int32_t> li = c_.buf<std::int32_t>(static_cast<std::size_t>(nlv));
                 DBuf<std::int64_t> lc = c_.buf<std::int64_t>(1);
-                hipLaunchKernelGGL(k_live_flags, dim3(grid_for(nlv)), dim3(256), 0, s, r.live, nlv, done.get(), lf.get());
+                hipLaunchKernelGGL(k_live_flags, dim3(grid_for(nlv)), dim3(256), 0, s, r.live, nlv, done, lf.get());
                 GP_LAUNCH_CHECK();
                 stable_select(c_, lf.get(), nlv, li.get(), lc.get());
                 const std::int64_t next = c_.read_scalar(lc.get());
@@ -3407,12 +3535,14 @@ public:
         int iterations = 0;
         bool feasible = false;
         std::int64_t count = 0;
-        DBuf<unsigned long long> prefix = c_.buf<unsigned long long>(static_cast<std::size_t>(k) * kBalanceWidth);
-        DBuf<std::int32_t> bstar = c_.buf<std::int32_t>(static_cast<std::size_t>(k));
-        DBuf<unsigned long long> excess = c_.buf<unsigned long long>(static_cast<std::size_t>(k));
-        DBuf<std::uint8_t> f = c_.buf<std::uint8_t>(n);
-        DBuf<std::int32_t> list = c_.buf<std::int32_t>(n);
-        DBuf<std::int64_t> lcount = c_.buf<std::int64_t>(1);
+        RepairBuffers b = repair_buffers();
+        const SelectState q{b.bstar.get(), b.prefix.get(), b.excess.get(), b.S.get(),     b.counts.get(),
+                            b.elig.get(),  b.E.get(),      b.live.get(),   b.done.get(),  b.tried.get(),
+                            b.slack.get(), b.requests.get(), ctr_.get() + kSelected,
+                            static_cast<unsigned long long>(kTailDonors)};
+        // Whether the last iteration had more eligible donors than one tail
+        // launch takes: then the host reads their number before it goes on.
+        bool many = false;
         const std::int64_t ncounts = (std::int64_t)k * kBalanceWidth;
         do {
             static_assert(kCtrCount <= kBalanceWidth, "the counter block clears inside the bucket clear");
@@ -3441,28 +3571,38 @@ public:
                     tiers(RepairProposeBody<unsigned long long>{{a_}}, cand_.get(), 0, ctr_.get() + kDonors, nullptr,
                           nullptr, nullptr, a_.k, kTier, true, kEntRepair);
             });
-            hipLaunchKernelGGL(k_bucket_scan, dim3(k), dim3(kScanThreads), 0, s, a_, prefix.get(), bstar.get(),
-                               excess.get());
+            hipLaunchKernelGGL(k_bucket_scan, dim3(k), dim3(kScanThreads), 0, s, a_, b.prefix.get(),
+                               b.bstar.get(), b.excess.get());
             GP_LAUNCH_CHECK();
             if (n <= kSelectSmallMax) {
-                // Flagging, eligibility and both compactions in one block.
-                hipLaunchKernelGGL(k_donors_small, dim3(1), dim3(kDonorThreads), 0, s, a_, bstar.get(), prefix.get(),
-                                   excess.get(), list.get(), lcount.get());
+                hipLaunchKernelGGL(k_donors_small, dim3(1), dim3(kDonorThreads), 0, s, a_, q);
                 GP_LAUNCH_CHECK();
-                const std::int64_t ne = c_.read_scalar(lcount.get());
-                if (ne > 0) reserve_donors(list.get(), list.get(), nullptr, ne);
             } else {
-                hipLaunchKernelGGL(k_repair_flag, dim3(grid_for(n)), dim3(256), 0, s, a_, bstar.get(), f.get());
+                hipLaunchKernelGGL(k_select_weights, dim3(b.tiles), dim3(kSelectThreads), 0, s, a_, q, b.rounds);
                 GP_LAUNCH_CHECK();
-                stable_select(c_, f.get(), n, list.get(), lcount.get());
-                const std::int64_t nl = c_.read_scalar(lcount.get());
-                if (nl > 0) reserve(list.get(), nl, prefix.get(), bstar.get(), excess.get());
+                hipLaunchKernelGGL(k_select_eligible, dim3(b.tiles), dim3(kSelectThreads), 0, s, a_, q, b.rounds);
+                GP_LAUNCH_CHECK();
+                hipLaunchKernelGGL(k_select_place, dim3(b.tiles), dim3(kSelectThreads), 0, s, a_, q, b.rounds);
+                GP_LAUNCH_CHECK();
             }
-            hipLaunchKernelGGL(k_repair_clear, dim3(grid_for(n)), dim3(256), 0, s, a_, cand_.get(),
-                               ctr_.get() + kDonors);
-            GP_LAUNCH_CHECK();
+            // The number of eligible donors decides the form of the
+            // reservation.  As long as one tail launch took the last
+            // iteration's, the launches of this one go out without a look at
+            // it: with more they move nothing, and the read-back at their end
+            // says so.
             std::int64_t delta = 0;
-            count = apply(false, true, delta, true);
+            std::int64_t ne = many ? (std::int64_t)c_.read_scalar(ctr_.get() + kSelected) : 0;
+            if (ne <= kTailDonors) {
+                reserve_tail(b);
+                count = apply(false, true, delta, true, cand_.get(), false);
+                ne = selected_;
+                many = false;
+            }
+            if (ne > kTailDonors) {
+                reserve_groups(b, ne);
+                count = apply(false, true, delta, true, cand_.get(), true);
+                many = true;
+            }
             ++iterations;
             if (count) {
                 update_cut(cut, delta);
@@ -3662,6 +3802,7 @@ public:
     // repair samples are zero on the device, so their clear can be skipped.
     bool ctr_clear_ = false;
     bool samples_clear_ = false;
+    std::int64_t selected_ = 0;  // eligible donors of the last repair iteration, as the last read-back had it
 };
 
 }  // namespace
