@@ -108,7 +108,9 @@ struct RefArgs {
     const std::uint32_t* vw;
     int k;
     std::uint64_t cap;
-    double filter;
+    // Null on levels without edge weights, else nonzero when some edge weighs
+    // more than 1 (the proposal filter's constant, incremental.cuh:897-899).
+    const unsigned long long* heavy_edge;
     Label* labels;
     unsigned long long* loads;
     const double* prices;  // null unless vertex weights exceed n
@@ -393,8 +395,9 @@ struct LpProposeBody : RowBody {
             best = team_reduce(t, best, priced);
         }
         if (current == total) return RowOut{false, degree(v)};
+        const double filter = a.heavy_edge && *a.heavy_edge ? 0.75 : 0.25;
         const bool accept = best.p >= 0 && (best.conn >= current ||
-                                            current - best.conn < (std::uint64_t)(a.filter * (double)current));
+                                            current - best.conn < (std::uint64_t)(filter * (double)current));
         if (accept && t.leader()) {
             a.targets[v] = best.p;
             set_gain(a, v, best.conn >= current ? (std::int64_t)(best.conn - current) : -(std::int64_t)(current - best.conn));
@@ -1927,6 +1930,49 @@ __global__ void k_gather_info(const DonorInfo* src, const std::int32_t* idx, std
         dst[j] = src[idx[j]];
 }
 
+// One word per part handed to a kernel by value: no copy and no host wait.
+struct PartWords {
+    unsigned long long w[kMaxParts];
+};
+inline PartWords part_words(const std::vector<std::uint64_t>& v) {
+    PartWords p{};
+    for (std::size_t i = 0; i < v.size() && i < kMaxParts; ++i) p.w[i] = v[i];
+    return p;
+}
+__global__ void k_set_parts(PartWords in, unsigned long long* out, int k) {
+    for (int p = threadIdx.x; p < k; p += blockDim.x) out[p] = in.w[p];
+}
+
+// Start of a refinement level in one launch: clears the counter block, the
+// heavy-edge flag and (when the level has prices) the prices, and sets the
+// part loads.  (An upload with its host wait and three fills before.)
+__global__ void k_level_begin(unsigned long long* ctr, PartWords loads, unsigned long long* loads_out, int k,
+                              unsigned long long* heavy_edge, double* prices) {
+    for (int i = threadIdx.x; i < kCtrCount; i += blockDim.x) ctr[i] = 0;
+    for (int p = threadIdx.x; p < k; p += blockDim.x) {
+        loads_out[p] = loads.w[p];
+        if (prices) prices[p] = 0.0;
+    }
+    if (threadIdx.x == 0) *heavy_edge = 0;
+}
+
+// Raises the flag when some weight is above 1; blocks stop once it is up.
+// The proposals read it on the device: the largest weight was read back to
+// the host before, one more wait per level.
+__global__ void __launch_bounds__(256) k_heavy_edge(std::int64_t m, const std::uint32_t* ew, unsigned long long* flag) {
+    const std::int64_t stride = (std::int64_t)gridDim.x * blockDim.x;
+    for (std::int64_t base = blockIdx.x * (std::int64_t)blockDim.x; base < m; base += 8 * stride) {
+        if (*(volatile unsigned long long*)flag) return;
+        bool heavy = false;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const std::int64_t x = base + j * stride + threadIdx.x;
+            heavy |= x < m && ew[x] > 1;
+        }
+        if (heavy) *(volatile unsigned long long*)flag = 1;
+    }
+}
+
 // Start of a repair iteration in one launch: freezes the part loads
 // (loads0 = loads), clears the bucket weights and the counter block.
 __global__ void k_repair_begin(RefArgs a, unsigned long long* loads0, unsigned long long* counts, std::int64_t ncounts,
@@ -3067,8 +3113,9 @@ public:
         medium_ = c.buf<std::int32_t>(n);
         heavy_ = c.buf<std::int32_t>(n);
         // Counters and part loads share one allocation: one read returns both.
-        // Counters, part loads, then the device loop words and best loads.
-        ctr_ = c.buf<unsigned long long>(static_cast<std::size_t>(kCtrCount + k + kLoopWords + k));
+        // Counters, part loads, then the device loop words, the best loads and
+        // the heavy-edge flag.
+        ctr_ = c.buf<unsigned long long>(static_cast<std::size_t>(kCtrCount + k + kLoopWords + k + 1));
         loads0_ = c.buf<unsigned long long>(static_cast<std::size_t>(k));
         bucket_ = c.buf<std::int32_t>(n);
         counts_ = c.buf<unsigned long long>(static_cast<std::size_t>(k) * kBalanceWidth);
@@ -3085,33 +3132,33 @@ public:
         a_.loads0 = loads0_.get();
         a_.bucket = bucket_.get();
         a_.counts = counts_.get();
-        c.upload(a_.loads, loads.data(), static_cast<std::size_t>(k) * sizeof(std::uint64_t));
-        fill<unsigned long long>(c, ctr_.get(), kCtrCount, 0ULL);
+        unsigned long long* heavy_edge = ctr_.get() + kCtrCount + 2 * k + kLoopWords;
         std::uint64_t total = 0;
         for (auto x : loads) total += x;
         if (total > static_cast<std::uint64_t>(n)) {
             prices_ = c.buf<double>(static_cast<std::size_t>(k));
             samples_ = c.buf<RepairSample>(static_cast<std::size_t>(k));
-            fill<double>(c, prices_.get(), k, 0.0);
             a_.prices = prices_.get();
             a_.samples = samples_.get();
+        }
+        hipLaunchKernelGGL(k_level_begin, dim3(1), dim3(256), 0, c.stream(), ctr_.get(), part_words(loads), a_.loads, k,
+                           heavy_edge, prices_.get());
+        GP_LAUNCH_CHECK();
+        if (g.ew && g.m > 0) {
+            hipLaunchKernelGGL(k_heavy_edge, dim3(grid_for(g.m, 256 * 16, 512)), dim3(256), 0, c.stream(), g.m,
+                               g.ew.get(), heavy_edge);
+            GP_LAUNCH_CHECK();
+            a_.heavy_edge = heavy_edge;
         }
         // Boundary vertices seed the frontier; per-level resets (its tier
         // counters were cleared with the counter block above).
         tiers(BoundaryBody{{a_}}, nullptr, n, nullptr, nullptr, nullptr, nullptr, 0, kTier, true);
-        // filter constant (incremental.cuh:897-899)
-        std::uint64_t max_edge = 1;
-        if (g.ew) {
-            DBuf<unsigned long long> mx = c.buf<unsigned long long>(1);
-            fill<unsigned long long>(c, mx.get(), 1, 0ULL);
-            if (g.m > 0) {
-                hipLaunchKernelGGL((k_reduce_max<std::uint32_t>), dim3(grid_for(g.m, 256, 2048)), dim3(256), 0, c.stream(),
-                                   g.ew.get(), g.m, mx.get());
-                GP_LAUNCH_CHECK();
-            }
-            max_edge = c.read_scalar(mx.get());
-        }
-        a_.filter = max_edge <= 1 ? 0.25 : 0.75;
+    }
+
+    // The level's part loads after the host has put other labels in place.
+    void set_loads(const std::vector<std::uint64_t>& loads) {
+        hipLaunchKernelGGL(k_set_parts, dim3(1), dim3(kMaxParts), 0, c_.stream(), part_words(loads), a_.loads, a_.k);
+        GP_LAUNCH_CHECK();
     }
 
     std::uint64_t max_load() const {
@@ -3119,8 +3166,6 @@ public:
         for (auto x : loads_host_) m = std::max(m, x);
         return m;
     }
-
-    unsigned long long* loads_dev() const { return a_.loads; }
 
     // Clears the moving flag and the target (-1) of every vertex, the state
     // the exchange starts from.
@@ -3872,7 +3917,7 @@ LevelStats refine_level_impl(Context& c, const DGraph& g, Label* labels, std::ve
     }
     c.copy_d2d(labels, best_labels.get(), static_cast<std::size_t>(g.n) * sizeof(Label));
     loads = best_loads;
-    c.upload(R.loads_dev(), loads.data(), static_cast<std::size_t>(k) * sizeof(std::uint64_t));
+    R.set_loads(loads);
     cut = best_cut;
     if (rounds > 0 && o.exchange_rounds > 0 && g.n <= o.exchange_max_n) {
         R.clear_moves(c);
