@@ -64,10 +64,13 @@ struct MetaBody {
     }
 };
 
-// Per-vertex maxima and sums; one atomic per block and statistic.
-__global__ void __launch_bounds__(256) k_vertex_meta(std::int64_t n, const std::int32_t* off, const std::uint32_t* vw,
-                                                     const std::uint64_t* row_bound, MetaOut* out) {
-    __shared__ unsigned long long part[4][4];
+// Per-vertex maxima and sums; one atomic per block and statistic, from few
+// large blocks (the statistics share a line, on which atomics queue up).
+__global__ void __launch_bounds__(kResultThreads) k_vertex_meta(std::int64_t n, const std::int32_t* off,
+                                                                const std::uint32_t* vw,
+                                                                const std::uint64_t* row_bound, MetaOut* out) {
+    constexpr int kWaves = kResultThreads / kWave;
+    __shared__ unsigned long long part[kWaves][4];
     unsigned long long maxrow = 0, maxdeg = 0, totalvw = 0, maxvw = 0;
     for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
          v += (std::int64_t)gridDim.x * blockDim.x) {
@@ -91,7 +94,7 @@ __global__ void __launch_bounds__(256) k_vertex_meta(std::int64_t n, const std::
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int i = 1; i < 4; ++i) {
+        for (int i = 1; i < kWaves; ++i) {
             maxrow = maxrow > part[i][0] ? maxrow : part[i][0];
             maxdeg = maxdeg > part[i][1] ? maxdeg : part[i][1];
             maxvw = maxvw > part[i][2] ? maxvw : part[i][2];
@@ -113,15 +116,21 @@ __global__ void __launch_bounds__(256) k_edge_flags(std::int64_t m, const std::u
         zero |= w == 0;
         non_unit |= w != 1;
     }
-    const unsigned long long z = __ballot(zero), nu = __ballot(non_unit);
-    if (lane_id() == 0 && (z || nu)) atomicOr(&out->flags, (z ? 1ULL : 0ULL) | (nu ? 2ULL : 0ULL));
+    const int z = __syncthreads_or(zero), nu = __syncthreads_or(non_unit);
+    if (threadIdx.x) return;
+    // A flag that is up already needs no atomic.
+    const unsigned long long bits = (z ? 1ULL : 0ULL) | (nu ? 2ULL : 0ULL);
+    if (bits & ~*(volatile unsigned long long*)&out->flags) atomicOr(&out->flags, bits);
 }
 
 // Degree classes for this level (src/coarsening/aggregation.cuh:5-71).
 // Queue order is irrelevant: every later write is per vertex.
 struct ClassCounts {
-    unsigned long long c[8];  // 0: <=16, 1: <=64, 2: <=128, 3: <=256, 4: <=512, 5: <=4096, 6: >4096, 7: max degree
+    // 0: <=16, 1: <=64, 2: <=128, 3: <=256, 4: <=512, 5: <=4096, 6: >4096, 7: max degree, 8: rows without entries
+    unsigned long long c[9];
 };
+constexpr int kClassWords = 9;
+static_assert(sizeof(ClassCounts) == kClassWords * sizeof(unsigned long long), "class counts are words");
 
 __device__ inline int degree_class(std::int64_t d) {
     return d <= kLowDegree ? 0 : d <= 64 ? 1 : d <= 128 ? 2 : d <= 256 ? 3 : d <= kWaveDegree ? 4 : d <= kBlockDegree ? 5 : 6;
@@ -137,9 +146,10 @@ __global__ void __launch_bounds__(256) k_classify(std::int64_t rows, const Off* 
                                                   std::int64_t stride, ClassCounts* counts) {
     __shared__ unsigned int lc[8];
     __shared__ unsigned long long gb[8];
+    __shared__ unsigned long long smax[256 / kWave], sempty[256 / kWave];
     const int lane = lane_id();
     const unsigned long long lt = (1ULL << lane) - 1ULL;
-    unsigned long long maxdeg = 0;
+    unsigned long long maxdeg = 0, empty = 0;
     for (std::int64_t base = blockIdx.x * (std::int64_t)(256 * kClassItems); base < rows;
          base += (std::int64_t)gridDim.x * (256 * kClassItems)) {
         if (threadIdx.x < 8) lc[threadIdx.x] = 0;
@@ -151,6 +161,7 @@ __global__ void __launch_bounds__(256) k_classify(std::int64_t rows, const Off* 
             const std::int64_t v = base + it * 256 + threadIdx.x;
             const std::int64_t d = v < rows ? (std::int64_t)(off[v + 1] - off[v]) : 0;
             maxdeg = maxdeg > (unsigned long long)d ? maxdeg : (unsigned long long)d;
+            empty += v < rows && d == 0;
             cls[it] = v < rows ? degree_class(d) : -1;
             rank[it] = 0;
             for (int c = 0; c < 7; ++c) {
@@ -174,7 +185,20 @@ __global__ void __launch_bounds__(256) k_classify(std::int64_t rows, const Off* 
         __syncthreads();
     }
     maxdeg = wave_max(maxdeg);
-    if (lane == 0 && maxdeg) atomicMax(&counts->c[7], maxdeg);
+    empty = wave_sum(empty);
+    if (lane == 0) {
+        smax[threadIdx.x / kWave] = maxdeg;
+        sempty[threadIdx.x / kWave] = empty;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 256 / kWave; ++w) {
+            maxdeg = maxdeg > smax[w] ? maxdeg : smax[w];
+            empty += sempty[w];
+        }
+        if (maxdeg) atomicMax(&counts->c[7], maxdeg);
+        if (empty) atomicAdd(&counts->c[8], empty);
+    }
 }
 
 template <typename Off>
@@ -191,7 +215,7 @@ void classify(Context& c, std::int64_t rows, const Off* off, std::int32_t* lists
 // (weight, symmetric hash, id); rows with degree > 1024 are skipped.
 __global__ void k_match_choose(std::int64_t n, const std::int32_t* off, const std::int32_t* nbr,
                                const std::uint32_t* ew, const std::uint32_t* vw, std::uint64_t cap, std::uint32_t salt,
-                               std::int32_t* choices) {
+                               std::int32_t* choices, unsigned long long* cw) {
     const int lane = lane_id();
     for (std::int64_t base = (blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x) - lane; base < n;
          base += (std::int64_t)gridDim.x * blockDim.x) {
@@ -200,6 +224,7 @@ __global__ void k_match_choose(std::int64_t n, const std::int32_t* off, const st
         if (v < n) {
             b = off[v];
             e = off[v + 1];
+            cw[v] = 0;  // the roots' sums start here
         }
         const bool heavy = v < n && e - b > 32 && e - b <= 1024;
         if (v < n && !heavy) {
@@ -260,8 +285,9 @@ __global__ void k_match_choose(std::int64_t n, const std::int32_t* off, const st
     }
 }
 
-__global__ void k_match_roots(std::int64_t n, const std::int32_t* choices, const std::uint32_t* vw,
-                              std::int32_t* clusters, unsigned long long* cw, unsigned long long* roots) {
+__global__ void __launch_bounds__(kResultThreads) k_match_roots(std::int64_t n, const std::int32_t* choices,
+                                                                const std::uint32_t* vw, std::int32_t* clusters,
+                                                                unsigned long long* cw, HostResult result) {
     unsigned long long count = 0;
     for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
          v += (std::int64_t)gridDim.x * blockDim.x) {
@@ -272,8 +298,7 @@ __global__ void k_match_roots(std::int64_t n, const std::int32_t* choices, const
         count += root == v;
         atomicAdd(&cw[root], (unsigned long long)vw[v]);
     }
-    count = wave_sum(count);
-    if (lane_id() == 0 && count) atomicAdd(roots, count);
+    publish_result<false>(count, result);
 }
 
 __global__ void k_init_singletons(std::int64_t n, const std::uint32_t* vw, std::int32_t* clusters,
@@ -289,12 +314,13 @@ __global__ void k_init_singletons(std::int64_t n, const std::uint32_t* vw, std::
 // residual_freeze_roles (singleton_growth.cuh:27-40); also resets proposals.
 __global__ void k_roles(std::int64_t n, const std::int32_t* clusters, const std::uint32_t* vw,
                         const unsigned long long* cw, std::uint32_t salt, std::uint32_t threshold, bool all,
-                        std::uint8_t* roles, std::int32_t* proposals) {
+                        std::uint8_t* roles, std::int32_t* proposals, unsigned long long* totals) {
     for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
          v += (std::int64_t)gridDim.x * blockDim.x) {
         roles[v] = clusters[v] == v && cw[v] == (unsigned long long)vw[v] &&
                    (all || mix32((std::uint32_t)v ^ salt) < threshold);
         proposals[v] = kInvalid;
+        if (totals) totals[v] = 0;  // the admission's sums start here
     }
 }
 
@@ -951,7 +977,8 @@ __global__ void k_target_totals(std::int64_t n, const std::int32_t* targets, con
         if (targets[v] != kInvalid) atomicAdd(&tot[targets[v]], (unsigned long long)vw[v]);
 }
 __global__ void k_contended_flags(std::int64_t n, const std::int32_t* targets, const unsigned long long* cw,
-                                  const unsigned long long* tot, std::uint64_t cap, std::uint8_t* flags) {
+                                  const unsigned long long* tot, std::uint64_t cap, std::uint8_t* flags,
+                                  std::uint8_t* contended) {
     for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
          v += (std::int64_t)gridDim.x * blockDim.x) {
         const std::int32_t t = targets[v];
@@ -961,6 +988,7 @@ __global__ void k_contended_flags(std::int64_t n, const std::int32_t* targets, c
             if (base <= cap) f = tot[t] > cap - base ? 1 : 2;
         }
         flags[v] = f;
+        contended[v] = f == 1;
     }
 }
 __global__ void k_commit_uncontended(std::int64_t n, const std::int32_t* targets, const std::uint8_t* flags,
@@ -975,12 +1003,6 @@ __global__ void k_commit_uncontended(std::int64_t n, const std::int32_t* targets
         clusters[v] = t;
     }
 }
-__global__ void k_flag_is(std::int64_t n, const std::uint8_t* in, std::uint8_t value, std::uint8_t* out) {
-    for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
-         v += (std::int64_t)gridDim.x * blockDim.x)
-        out[v] = in[v] == value;
-}
-
 // Composite key, least significant first: (~tie) | (~score masked) << 32 | target << (32+sb).
 __global__ void k_admission_keys(std::int64_t count, const std::int32_t* order, const std::int32_t* targets,
                                  const std::uint64_t* score, const std::uint32_t* ties, int score_bits, bool with_target,
@@ -1042,7 +1064,80 @@ __global__ void k_admission_commit(std::int64_t count, const std::uint32_t* vals
     }
 }
 
-__global__ void k_count_nonzero(std::int64_t n, const unsigned long long* cw, unsigned long long* out) {
+// The ordered admission of a short list in one block: segment heads, weight
+// prefixes per target, the target's frozen weight and the commit, for
+// kAdmitThreads items at a time (five to seven launches otherwise).  A
+// segment's frozen weight is read at its head, before any of its commits, and
+// carried along with its prefix: targets are never sources, so only the
+// segment's own commits change it.
+constexpr int kAdmitThreads = 1024;
+constexpr int kAdmitSmallMax = 8192;
+__global__ void __launch_bounds__(kAdmitThreads) k_admission_small(int count, const std::uint32_t* vals,
+                                                                   const std::int32_t* targets, const std::uint32_t* vw,
+                                                                   std::uint64_t cap, std::int32_t* clusters,
+                                                                   unsigned long long* cw) {
+    constexpr int kWaves = kAdmitThreads / kWave;
+    __shared__ SegU64 wsum[kWaves];
+    __shared__ std::int32_t tgt[kAdmitThreads];
+    __shared__ unsigned long long base[kAdmitThreads];
+    __shared__ int wlast[kWaves];
+    const int t = threadIdx.x, w = t / kWave, lane = lane_id();
+    SegU64 carry{0, 0};           // of the segment open at the chunk's start
+    unsigned long long open = 0;  // its frozen weight
+    std::int32_t last = -1;       // its target
+    for (int c0 = 0; c0 < count; c0 += kAdmitThreads) {
+        const int i = c0 + t;
+        std::int32_t v = -1, target = -1;
+        std::uint64_t wt = 0;
+        if (i < count) {
+            v = (std::int32_t)vals[i];
+            target = targets[v];
+            wt = vw[v];
+        }
+        tgt[t] = target;
+        __syncthreads();
+        const bool head = i < count && (t == 0 ? target != last : target != tgt[t - 1]);
+        if (head) base[t] = cw[target];
+        SegU64 x = wave_inclusive_scan<SegPlusOp>(SegU64{wt, head ? 1u : 0u});
+        // Chunk position of the last head at or before this item, -1 for none.
+        int at = head ? t : -1;
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int o = __shfl_up(at, d);
+            if (lane >= d && o > at) at = o;
+        }
+        if (lane == kWave - 1) {
+            wsum[w] = x;
+            wlast[w] = at;
+        }
+        __syncthreads();
+        SegU64 pre = carry, all = carry;
+        int hat = -1, hall = -1;
+        for (int j = 0; j < kWaves; ++j) {
+            if (j == w) {
+                pre = all;
+                hat = hall;
+            }
+            all = SegPlusOp::op<SegU64>(all, wsum[j]);
+            if (wlast[j] >= 0) hall = wlast[j];
+        }
+        x = SegPlusOp::op<SegU64>(pre, x);
+        if (at < 0) at = hat;
+        const unsigned long long frozen = at >= 0 ? base[at] : open;
+        if (i < count && frozen <= cap && x.v <= cap - frozen) {
+            const std::int32_t s = clusters[v];
+            atomicAdd(&cw[s], 0ULL - (unsigned long long)wt);
+            atomicAdd(&cw[target], (unsigned long long)wt);
+            clusters[v] = target;
+        }
+        carry = SegU64{all.v, 0};
+        if (hall >= 0) open = base[hall];
+        last = tgt[kAdmitThreads - 1];
+        __syncthreads();
+    }
+}
+
+__global__ void __launch_bounds__(kResultThreads) k_count_nonzero(std::int64_t n, const unsigned long long* cw,
+                                                                  HostResult result) {
     unsigned long long c = 0;
     const std::int64_t stride = (std::int64_t)gridDim.x * blockDim.x;
     // Four independent loads per step.
@@ -1053,8 +1148,7 @@ __global__ void k_count_nonzero(std::int64_t n, const unsigned long long* cw, un
 #pragma unroll
         for (int j = 0; j < 4; ++j) c += x[j] != 0;
     }
-    c = wave_sum(c);
-    if (lane_id() == 0 && c) atomicAdd(out, c);
+    publish_result<false>(c, result);
 }
 
 // ------------------------------------------------------------ isolated
@@ -1127,11 +1221,11 @@ __global__ void k_pair_commit(std::int64_t count, const std::uint32_t* vals, con
 }
 
 // ----------------------------------------------------------- compaction
-__global__ void k_nonempty(std::int64_t n, const unsigned long long* cw, std::uint8_t* flags) {
-    for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
-         v += (std::int64_t)gridDim.x * blockDim.x)
-        flags[v] = cw[v] > 0;
-}
+// 1 for a cluster with weight, else 0: the compaction's scan reads this.
+struct Nonempty {
+    const unsigned long long* cw;
+    __device__ int operator[](std::int64_t v) const { return cw[v] > 0; }
+};
 __global__ void k_compact_map(std::int64_t n, const std::int32_t* clusters, const std::int64_t* ids,
                               const std::uint32_t* vw, std::int32_t* map, unsigned long long* sums) {
     for (std::int64_t v = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; v < n;
@@ -1141,16 +1235,15 @@ __global__ void k_compact_map(std::int64_t n, const std::int32_t* clusters, cons
         atomicAdd(&sums[c], (unsigned long long)vw[v]);
     }
 }
-__global__ void k_narrow_weights(std::int64_t n, const unsigned long long* sums, std::uint32_t* out,
-                                 unsigned long long* maxw) {
+__global__ void __launch_bounds__(kResultThreads) k_narrow_weights(std::int64_t n, const unsigned long long* sums,
+                                                                   std::uint32_t* out, HostResult result) {
     unsigned long long m = 0;
     for (std::int64_t c = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; c < n;
          c += (std::int64_t)gridDim.x * blockDim.x) {
         out[c] = (std::uint32_t)sums[c];
         m = m > sums[c] ? m : sums[c];
     }
-    m = wave_max(m);
-    if (lane_id() == 0 && m) atomicMax(maxw, m);
+    publish_result<true>(m, result);
 }
 
 // ----------------------------------------------------------- contraction
@@ -1177,6 +1270,43 @@ __global__ void k_contract_bounds(std::int64_t n, const std::int32_t* map, const
             if (seen == prev) break;
             prev = seen;
         }
+    }
+}
+
+// Largest coarse bound and longest raw coarse row.
+__global__ void __launch_bounds__(kResultThreads) k_contract_maxima(std::int64_t nc, const unsigned long long* bounds,
+                                                                    const unsigned long long* raw,
+                                                                    unsigned long long* out) {
+    __shared__ unsigned long long part[2][kResultThreads / kWave];
+    std::uint64_t b = 0, r = 0;
+    for (std::int64_t c = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; c < nc;
+         c += (std::int64_t)gridDim.x * blockDim.x) {
+        b = b > bounds[c] ? b : bounds[c];
+        r = r > raw[c] ? r : raw[c];
+    }
+    b = wave_max(b);
+    r = wave_max(r);
+    if (lane_id() == 0) {
+        part[0][threadIdx.x / kWave] = b;
+        part[1][threadIdx.x / kWave] = r;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned long long m = 0;
+        for (int w = 0; w < kResultThreads / kWave; ++w) m = m > part[threadIdx.x][w] ? m : part[threadIdx.x][w];
+        if (m) atomicMax(&out[threadIdx.x], m);
+    }
+}
+
+// Zeroes three arrays in one launch.
+__global__ void k_zero3(unsigned long long* a, std::int64_t na, unsigned long long* b, std::int64_t nb,
+                        unsigned long long* c, std::int64_t ncw) {
+    const std::int64_t most = na > nb ? (na > ncw ? na : ncw) : (nb > ncw ? nb : ncw);
+    for (std::int64_t i = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; i < most;
+         i += (std::int64_t)gridDim.x * blockDim.x) {
+        if (i < na) a[i] = 0;
+        if (i < nb) b[i] = 0;
+        if (i < ncw) c[i] = 0;
     }
 }
 
@@ -1402,12 +1532,10 @@ static bool reduce_long_rows(Context& c, const Src& src, std::int64_t count, std
                              int total_bits, std::uint64_t row_weight_bound, DBuf<std::uint64_t>& ukeys,
                              DBuf<unsigned long long>& usums, std::int64_t& nu) {
     DBuf<std::int64_t> chunk_off = c.buf<std::int64_t>(static_cast<std::size_t>(count + 1));
-    DBuf<std::int64_t> ctot = c.buf<std::int64_t>(1);
     hipLaunchKernelGGL((k_chunk_counts<Src>), dim3(grid_for(count)), dim3(256), 0, c.stream(), src, count,
                        chunk_off.get());
     GP_LAUNCH_CHECK();
-    exclusive_sum<std::int64_t>(c, chunk_off.get(), chunk_off.get(), count, ctot.get());
-    c.copy_d2d(chunk_off.get() + count, ctot.get(), sizeof(std::int64_t));
+    exclusive_sum<std::int64_t>(c, chunk_off.get(), chunk_off.get(), count, static_cast<std::int64_t*>(nullptr), true);
     DBuf<unsigned long long> ctr = c.buf<unsigned long long>(2);
     fill<unsigned long long>(c, ctr.get(), 2, 0ULL);
     DBuf<std::uint64_t> keys = c.buf<std::uint64_t>(static_cast<std::size_t>(std::max<std::int64_t>(raw_records, 1)));
@@ -1443,7 +1571,7 @@ void compute_level0_metadata(Context& c, DGraph& g, CoarsenState& st) {
         const MetaBody body{g.off.get(), g.nbr.get(), g.ew_ptr(), st.row_bound.get()};
         run_tiers(c, body, nullptr, g.n, nullptr, ta.get(), tb.get(), tn.get(), nullptr, nullptr, reinterpret_cast<unsigned long long*>(out.get()) + 1,
                   0, g.n);
-        hipLaunchKernelGGL(k_vertex_meta, dim3(grid_for(g.n, 256, 1024)), dim3(256), 0, c.stream(), g.n, g.off.get(),
+        hipLaunchKernelGGL(k_vertex_meta, dim3(result_grid(g.n)), dim3(kResultThreads), 0, c.stream(), g.n, g.off.get(),
                            g.vw.get(), st.row_bound.get(), out.get());
         GP_LAUNCH_CHECK();
         if (g.ew && g.m > 0) {
@@ -1483,19 +1611,14 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
     DBuf<std::uint64_t> gains = c.buf<std::uint64_t>(n);
     DBuf<std::uint64_t> regret = c.buf<std::uint64_t>(n);
     DBuf<std::uint32_t> ties = c.buf<std::uint32_t>(n);
-    DBuf<unsigned long long> scalar = c.buf<unsigned long long>(4);
-    // scalar[0] accumulates one count or maximum at a time; reading it back
-    // also clears it, so only its first use needs a fill.
-    bool scalar_zero = false;
-    auto scalar_ready = [&] {
-        if (!scalar_zero) fill<unsigned long long>(c, scalar.get(), 1, 0ULL);
-        scalar_zero = false;
-    };
-    auto scalar_take = [&]() -> unsigned long long {
-        unsigned long long v = 0;
-        c.read_clear(&v, scalar.get(), 1, 1);
-        scalar_zero = true;
-        return v;
+    // One word that counts and maxima gather in (publish_result leaves it
+    // zero) and the class counts, cleared together.
+    DBuf<unsigned long long> scalar = c.buf<unsigned long long>(1 + kClassWords);
+    fill<unsigned long long>(c, scalar.get(), 1 + kClassWords, 0ULL);
+    // Waits for the result of the launch that took `r`.
+    auto take = [&](const HostResult& r) -> unsigned long long {
+        c.wait_flag(r.flag, r.seq);
+        return r.host[0];
     };
     const int vb = grid_for(n);
 
@@ -1504,14 +1627,13 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
         DBuf<std::int32_t> choices = c.buf<std::int32_t>(n);
         const std::uint32_t salt = seed ^ ((std::uint32_t)level * 0x9e3779b9U);
         hipLaunchKernelGGL(k_match_choose, dim3(vb), dim3(256), 0, s, n, g.off.get(), g.nbr.get(), g.ew_ptr(),
-                           g.vw.get(), cap, salt, choices.get());
+                           g.vw.get(), cap, salt, choices.get(), cw.get());
         GP_LAUNCH_CHECK();
-        fill<unsigned long long>(c, cw.get(), n, 0ULL);
-        scalar_ready();
-        hipLaunchKernelGGL(k_match_roots, dim3(vb), dim3(256), 0, s, n, choices.get(), g.vw.get(), clusters.get(),
-                           cw.get(), scalar.get());
+        const HostResult r = host_result(c, scalar.get());
+        hipLaunchKernelGGL(k_match_roots, dim3(std::max(result_grid(n), std::min(vb, 256))), dim3(kResultThreads), 0, s,
+                           n, choices.get(), g.vw.get(), clusters.get(), cw.get(), r);
         GP_LAUNCH_CHECK();
-        cluster_count = (std::int64_t)scalar_take();
+        cluster_count = (std::int64_t)take(r);
     } else {
         hipLaunchKernelGGL(k_init_singletons, dim3(vb), dim3(256), 0, s, n, g.vw.get(), clusters.get(), cw.get());
         GP_LAUNCH_CHECK();
@@ -1519,11 +1641,9 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
 
     // Degree classes (lists built once per level).
     DBuf<std::int32_t> lists = c.buf<std::int32_t>(static_cast<std::size_t>(7 * n));
-    DBuf<ClassCounts> ccount = c.buf<ClassCounts>(1);
-    fill<unsigned long long>(c, reinterpret_cast<unsigned long long*>(ccount.get()), 8, 0ULL);
-    classify(c, n, g.off.get(), lists.get(), n, ccount.get());
-    GP_LAUNCH_CHECK();
-    ClassCounts cc = c.read_scalar(ccount.get());
+    ClassCounts* ccount = reinterpret_cast<ClassCounts*>(scalar.get() + 1);
+    classify(c, n, g.off.get(), lists.get(), n, ccount);
+    ClassCounts cc = c.read_scalar(ccount);
     std::uint64_t stats_maxdeg = cc.c[7];
     bool stats_heavy = cc.c[7] >= 4096;
     if (g.max_degree <= 8) {  // a bound <= 8 is trusted (src/coarsen.cu:84-90)
@@ -1568,13 +1688,15 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
     const int cluster_bits = std::max(1, bit_width_u64(static_cast<std::uint64_t>(n)));
     const int hub_bits = std::max(1, bit_width_u64(static_cast<std::uint64_t>(hub_count)));
 
-    auto form_proposals = [&](int round, bool filter_roles, std::uint32_t threshold, bool need_regret) {
+    // totals: null, or an array of n words that comes back zero.
+    auto form_proposals = [&](int round, bool filter_roles, std::uint32_t threshold, bool need_regret,
+                              unsigned long long* totals) {
         const std::uint32_t role_salt =
             seed ^ ((std::uint32_t)level * 0x9e3779b9U) ^ ((std::uint32_t)round * 0x85ebca6bU) ^ 0x27d4eb2dU;
         const std::uint32_t tie_salt =
             seed ^ ((std::uint32_t)level * 0xc2b2ae35U) ^ ((std::uint32_t)round * 0x165667b1U) ^ 0xd3a2646cU;
         hipLaunchKernelGGL(k_roles, dim3(vb), dim3(256), 0, s, n, clusters.get(), g.vw.get(), cw.get(), role_salt,
-                           threshold, !filter_roles, roles.get(), proposals.get());
+                           threshold, !filter_roles, roles.get(), proposals.get(), totals);
         GP_LAUNCH_CHECK();
         AffinityArgs a{g.off.get(), g.nbr.get(), g.ew_ptr(), clusters.get(), cw.get(), roles.get(), cap, tie_salt,
                        filter_roles, filter_roles && need_regret, proposals.get(), gains.get(), regret.get(),
@@ -1661,10 +1783,10 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
     };
 
     auto count_clusters = [&]() {
-        scalar_ready();
-        hipLaunchKernelGGL(k_count_nonzero, dim3(grid_for(n, 256, 1024)), dim3(256), 0, s, n, cw.get(), scalar.get());
+        const HostResult r = host_result(c, scalar.get());
+        hipLaunchKernelGGL(k_count_nonzero, dim3(result_grid(n)), dim3(kResultThreads), 0, s, n, cw.get(), r);
         GP_LAUNCH_CHECK();
-        return (std::int64_t)scalar_take();
+        return (std::int64_t)take(r);
     };
 
     const int score_bits = std::max(1, std::min(64, bit_width_u64(st.max_row_weight)));
@@ -1722,7 +1844,9 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
         const std::uint64_t degree = stats_maxdeg;
         const bool fit = fast_path && (degree == 0 || bound <= room / maxv / degree);
         const std::uint64_t next_bound = fit ? bound + bound * degree * maxv : cap;
-        form_proposals(round, true, threshold, !fit);
+        DBuf<unsigned long long> tot;
+        if (!fit) tot = c.buf<unsigned long long>(n);
+        form_proposals(round, true, threshold, !fit, tot.get());
         if (fit) {
             hipLaunchKernelGGL(k_commit_all, dim3(vb), dim3(256), 0, s, n, proposals.get(), g.vw.get(),
                                clusters.get(), cw.get());
@@ -1730,24 +1854,24 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
         } else {
             DBuf<std::uint64_t> keys;
             DBuf<std::uint32_t> vals;
-            DBuf<unsigned long long> tot = c.buf<unsigned long long>(n);
             DBuf<std::uint8_t> aflags = c.buf<std::uint8_t>(n);
             DBuf<std::uint8_t> contended = c.buf<std::uint8_t>(n);
-            fill<unsigned long long>(c, tot.get(), n, 0ULL);
             hipLaunchKernelGGL(k_target_totals, dim3(vb), dim3(256), 0, s, n, proposals.get(), g.vw.get(), tot.get());
             hipLaunchKernelGGL(k_contended_flags, dim3(vb), dim3(256), 0, s, n, proposals.get(), cw.get(), tot.get(),
-                               cap, aflags.get());
-            hipLaunchKernelGGL(k_flag_is, dim3(vb), dim3(256), 0, s, n, aflags.get(), (std::uint8_t)1,
-                               contended.get());
+                               cap, aflags.get(), contended.get());
             GP_LAUNCH_CHECK();
             const std::int64_t count = admission_order(regret.get(), keys, vals, contended.get());
-            if (count) {
+            if (count && count <= kAdmitSmallMax) {
+                hipLaunchKernelGGL(k_admission_small, dim3(1), dim3(kAdmitThreads), 0, s, static_cast<int>(count),
+                                   vals.get(), proposals.get(), g.vw.get(), cap, clusters.get(), cw.get());
+                GP_LAUNCH_CHECK();
+            } else if (count) {
                 DBuf<SegU64> items = c.buf<SegU64>(static_cast<std::size_t>(count));
                 DBuf<std::uint64_t> base = c.buf<std::uint64_t>(static_cast<std::size_t>(count));
                 hipLaunchKernelGGL(k_seg_items, dim3(grid_for(count)), dim3(256), 0, s, count, vals.get(),
                                    proposals.get(), g.vw.get(), false, items.get());
                 GP_LAUNCH_CHECK();
-                scan<SegPlusOp, SegU64, SegU64, SegU64>(c, items.get(), items.get(), count, false);
+                scan<SegPlusOp, SegU64>(c, items.get(), items.get(), count, false);
                 hipLaunchKernelGGL(k_gather_base, dim3(grid_for(count)), dim3(256), 0, s, count, vals.get(),
                                    proposals.get(), cw.get(), base.get());
                 GP_LAUNCH_CHECK();
@@ -1767,7 +1891,7 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
         if ((double)cluster_count <= 0.60 * (double)n) break;
     }
 
-    if (pack_isolated) {
+    if (pack_isolated && cc.c[8] > 1) {  // rows without entries, counted with the classes
         DBuf<std::uint8_t> flags = c.buf<std::uint8_t>(n);
         DBuf<std::int32_t> iso = c.buf<std::int32_t>(n);
         DBuf<std::int64_t> cnt = c.buf<std::int64_t>(1);
@@ -1798,7 +1922,7 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
     }
 
     if ((double)cluster_count > 0.60 * (double)n) {
-        form_proposals(4, false, 0, false);
+        form_proposals(4, false, 0, false, nullptr);
         hipLaunchKernelGGL(k_favorites, dim3(vb), dim3(256), 0, s, n, g.vw.get(), cw.get(), clusters.get(),
                            proposals.get());
         GP_LAUNCH_CHECK();
@@ -1810,7 +1934,7 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
             hipLaunchKernelGGL(k_seg_items, dim3(grid_for(count)), dim3(256), 0, s, count, vals.get(), proposals.get(),
                                g.vw.get(), true, ranks.get());
             GP_LAUNCH_CHECK();
-            scan<SegPlusOp, SegU64, SegU64, SegU64>(c, ranks.get(), ranks.get(), count, false);
+            scan<SegPlusOp, SegU64>(c, ranks.get(), ranks.get(), count, false);
             DBuf<std::uint8_t> pflags = c.buf<std::uint8_t>(static_cast<std::size_t>(count));
             DBuf<std::int64_t> pos = c.buf<std::int64_t>(static_cast<std::size_t>(count));
             hipLaunchKernelGGL(k_pair_flags, dim3(grid_for(count)), dim3(256), 0, s, count, vals.get(), g.vw.get(),
@@ -1829,26 +1953,25 @@ AggregateResult aggregate(Context& c, const DGraph& g, CoarsenState& st, int par
 
     // Compaction.
     {
-        DBuf<std::uint8_t> flags = c.buf<std::uint8_t>(n);
+        // No more clusters have weight than were counted last, so the arrays
+        // are laid out before the host knows the exact number.
         DBuf<std::int64_t> ids = c.buf<std::int64_t>(n);
         DBuf<std::int64_t> cnt = c.buf<std::int64_t>(1);
-        hipLaunchKernelGGL(k_nonempty, dim3(vb), dim3(256), 0, s, n, cw.get(), flags.get());
-        GP_LAUNCH_CHECK();
-        exclusive_sum<std::int64_t>(c, flags.get(), ids.get(), n, cnt.get());
-        const std::int64_t nc = c.read_scalar(cnt.get());
+        exclusive_sum<std::int64_t>(c, Nonempty{cw.get()}, ids.get(), n, cnt.get());
         map = c.buf<std::int32_t>(n);
-        DBuf<unsigned long long> sums = c.buf<unsigned long long>(static_cast<std::size_t>(nc));
-        fill<unsigned long long>(c, sums.get(), nc, 0ULL);
+        const std::int64_t bound = std::max<std::int64_t>(cluster_count, 1);
+        DBuf<unsigned long long> sums = c.buf<unsigned long long>(static_cast<std::size_t>(bound));
+        fill<unsigned long long>(c, sums.get(), bound, 0ULL);
         hipLaunchKernelGGL(k_compact_map, dim3(vb), dim3(256), 0, s, n, clusters.get(), ids.get(), g.vw.get(),
                            map.get(), sums.get());
         GP_LAUNCH_CHECK();
-        coarse_vw = c.buf<std::uint32_t>(static_cast<std::size_t>(nc));
-        scalar_ready();
-        hipLaunchKernelGGL(k_narrow_weights, dim3(grid_for(nc)), dim3(256), 0, s, nc, sums.get(), coarse_vw.get(),
-                           scalar.get());
+        coarse_vw = c.buf<std::uint32_t>(static_cast<std::size_t>(bound));
+        const HostResult r = host_result(c, scalar.get(), cnt.get());
+        hipLaunchKernelGGL(k_narrow_weights, dim3(result_grid(bound)), dim3(kResultThreads), 0, s, bound, sums.get(),
+                           coarse_vw.get(), r);
         GP_LAUNCH_CHECK();
-        res.max_weight = scalar_take();
-        res.coarse_n = nc;
+        res.max_weight = take(r);
+        res.coarse_n = (std::int64_t)r.host[1];
         if (res.max_weight > 0xffffffffULL) throw std::runtime_error("coarse vertex weight exceeds uint32");
         if (res.max_weight > cap) throw std::runtime_error("coarsening exceeded cluster capacity");
     }
@@ -1862,42 +1985,32 @@ std::unique_ptr<DGraph> contract(Context& c, const DGraph& fine, CoarsenState& s
     auto out = std::make_unique<DGraph>();
     out->n = nc;
     // Bounds carried through the map (src/coarsen.cu:1470-1513).
-    DBuf<unsigned long long> next_rb = c.buf<unsigned long long>(static_cast<std::size_t>(nc));
+    DBuf<std::uint64_t> next_bounds = c.buf<std::uint64_t>(static_cast<std::size_t>(nc));
+    unsigned long long* next_rb = reinterpret_cast<unsigned long long*>(next_bounds.get());
     DBuf<unsigned long long> rawc = c.buf<unsigned long long>(static_cast<std::size_t>(nc));
-    fill<unsigned long long>(c, next_rb.get(), nc, 0ULL);
-    fill<unsigned long long>(c, rawc.get(), nc, 0ULL);
+    // The level's small counters: the two maxima, the class counts (read back
+    // together), the tier counters of the scatter and of the copy, the
+    // weight-overflow flag and the entries of the coarse graph (read back
+    // together).
+    constexpr int kSmallRed = 0, kSmallClasses = 2, kSmallTierScatter = kSmallClasses + kClassWords,
+                  kSmallTierCopy = kSmallTierScatter + 2, kSmallOverflow = kSmallTierCopy + 2,
+                  kSmallEntries = kSmallOverflow + 1, kSmallWords = kSmallEntries + 1;
+    DBuf<unsigned long long> small = c.buf<unsigned long long>(kSmallWords);
+    hipLaunchKernelGGL(k_zero3, dim3(grid_for(nc, 256, 2048)), dim3(256), 0, s, next_rb, nc, rawc.get(), nc,
+                       small.get(), (std::int64_t)kSmallWords);
+    GP_LAUNCH_CHECK();
     const bool plain_bounds = st.max_row_weight == 0 || (std::uint64_t)n <= ~0ULL / st.max_row_weight;
     hipLaunchKernelGGL(k_contract_bounds, dim3(grid_for(n)), dim3(256), 0, s, n, map, fine.off.get(), st.row_bound.get(),
-                       next_rb.get(), rawc.get(), plain_bounds);
+                       next_rb, rawc.get(), plain_bounds);
     GP_LAUNCH_CHECK();
-    // The level's small counters, cleared by one fill: the two maxima, the
-    // tier counters of the scatter and of the copy, the class counts and
-    // the weight-overflow flag.
-    constexpr int kSmallRed = 0, kSmallTierScatter = 2, kSmallTierCopy = 4, kSmallClasses = 6, kSmallOverflow = 14,
-                  kSmallWords = 15;
-    static_assert(sizeof(ClassCounts) == 8 * sizeof(unsigned long long), "class counts are eight words");
-    DBuf<unsigned long long> small = c.buf<unsigned long long>(kSmallWords);
-    fill<unsigned long long>(c, small.get(), kSmallWords, 0ULL);
-    unsigned long long* red = small.get() + kSmallRed;
-    hipLaunchKernelGGL((k_reduce_max<unsigned long long>), dim3(grid_for(nc, 256, 1024)), dim3(256), 0, s, next_rb.get(), nc,
-                       red);
-    hipLaunchKernelGGL((k_reduce_max<unsigned long long>), dim3(grid_for(nc, 256, 1024)), dim3(256), 0, s, rawc.get(), nc,
-                       red + 1);
+    hipLaunchKernelGGL(k_contract_maxima, dim3(result_grid(nc)), dim3(kResultThreads), 0, s, nc, next_rb, rawc.get(),
+                       small.get() + kSmallRed);
     GP_LAUNCH_CHECK();
-    unsigned long long rb[2];
-    c.read(rb, red, sizeof rb);
-    const bool count_raw = st.positive_ew && n >= 65536 && fine.max_degree <= 512;
-    const std::uint64_t crb = rb[0];
-    const std::uint64_t craw = count_raw ? rb[1] : ~0ULL;
-    const std::uint64_t next_degree_bound = count_raw && fine.max_degree <= 128 ? craw : crb;
-
-    // Raw coarse rows.
+    // Raw coarse rows: offsets, and a copy that the scatter advances.
     DBuf<std::int64_t> raw_off = c.buf<std::int64_t>(static_cast<std::size_t>(nc + 1));
-    DBuf<std::int64_t> rawtot = c.buf<std::int64_t>(1);
-    exclusive_sum<std::int64_t>(c, rawc.get(), raw_off.get(), nc, rawtot.get());
-    c.copy_d2d(raw_off.get() + nc, rawtot.get(), sizeof(std::int64_t));
-    DBuf<unsigned long long> cursor = c.buf<unsigned long long>(static_cast<std::size_t>(nc));
-    c.copy_d2d(cursor.get(), raw_off.get(), static_cast<std::size_t>(nc) * sizeof(std::int64_t));
+    DBuf<std::int64_t> cursor = c.buf<std::int64_t>(static_cast<std::size_t>(nc));
+    exclusive_sum<std::int64_t>(c, rawc.get(), raw_off.get(), nc, static_cast<std::int64_t*>(nullptr), true,
+                                cursor.get());
     const std::int64_t m = fine.m;
     DBuf<std::int32_t> tier_a = c.buf<std::int32_t>(static_cast<std::size_t>(std::max(n, nc)));
     DBuf<std::int32_t> tier_b = c.buf<std::int32_t>(static_cast<std::size_t>(std::max(n, nc)));
@@ -1907,7 +2020,8 @@ std::unique_ptr<DGraph> contract(Context& c, const DGraph& fine, CoarsenState& s
         // Algorithmic traffic: offsets, map[v], neighbours, map[neighbour],
         // optional edge weights, and the (key, weight) record written per entry.
         const double bytes = 8.0 * (double)n + 4.0 + (double)m * (8.0 + (fine.ew ? 4.0 : 0.0) + 8.0);
-        const ScatterBody body{fine.off.get(), fine.nbr.get(), fine.ew_ptr(), map, cursor.get(), rkey.get(), rval.get()};
+        const ScatterBody body{fine.off.get(), fine.nbr.get(), fine.ew_ptr(), map, reinterpret_cast<unsigned long long*>(cursor.get()),
+                               rkey.get(), rval.get()};
         c.timed("contract_scatter", bytes,
                 [&] { run_tiers(c, body, nullptr, n, nullptr, tier_a.get(), tier_b.get(), small.get() + kSmallTierScatter,
                                 nullptr, nullptr, nullptr, 0, n, fine.row_len_bound, true); });
@@ -1915,11 +2029,19 @@ std::unique_ptr<DGraph> contract(Context& c, const DGraph& fine, CoarsenState& s
     cursor.reset();
     // Row classes by raw length.
     DBuf<std::int32_t> lists = c.buf<std::int32_t>(static_cast<std::size_t>(7 * nc));
-    ClassCounts* ccount = reinterpret_cast<ClassCounts*>(small.get() + kSmallClasses);
-    classify(c, nc, raw_off.get(), lists.get(), nc, ccount);
-    ClassCounts cc = c.read_scalar(ccount);
+    classify(c, nc, raw_off.get(), lists.get(), nc, reinterpret_cast<ClassCounts*>(small.get() + kSmallClasses));
+    unsigned long long sm[kSmallClasses + kClassWords];
+    c.read(sm, small.get(), sizeof sm);
+    ClassCounts cc;
+    std::copy(sm + kSmallClasses, sm + kSmallClasses + kClassWords, cc.c);
+    const unsigned long long* rb = sm + kSmallRed;
+    const bool count_raw = st.positive_ew && n >= 65536 && fine.max_degree <= 512;
+    const std::uint64_t crb = rb[0];
+    const std::uint64_t craw = count_raw ? rb[1] : ~0ULL;
+    const std::uint64_t next_degree_bound = count_raw && fine.max_degree <= 128 ? craw : crb;
+    // Every row of a class gets its count; long rows without records keep 0.
     DBuf<unsigned long long> ucount = c.buf<unsigned long long>(static_cast<std::size_t>(nc));
-    fill<unsigned long long>(c, ucount.get(), nc, 0ULL);
+    if (cc.c[6]) fill<unsigned long long>(c, ucount.get(), nc, 0ULL);
     unsigned long long* overflow = small.get() + kSmallOverflow;
     RowArgs r{raw_off.get(), rkey.get(), rval.get(), ucount.get(), overflow};
     // Rows of the short and block classes and the long rows are disjoint:
@@ -1993,13 +2115,14 @@ std::unique_ptr<DGraph> contract(Context& c, const DGraph& fine, CoarsenState& s
         }
     }
     if (side) c.join();
-    if (c.read_scalar(overflow)) throw std::runtime_error("coarse edge weight exceeds uint32");
     // Final offsets and copy.
     DBuf<std::int64_t> coff64 = c.buf<std::int64_t>(static_cast<std::size_t>(nc + 1));
-    DBuf<std::int64_t> mtot = c.buf<std::int64_t>(1);
-    exclusive_sum<std::int64_t>(c, ucount.get(), coff64.get(), nc, mtot.get());
-    c.copy_d2d(coff64.get() + nc, mtot.get(), sizeof(std::int64_t));
-    const std::int64_t mc = c.read_scalar(mtot.get());
+    exclusive_sum<std::int64_t>(c, ucount.get(), coff64.get(), nc,
+                                reinterpret_cast<std::int64_t*>(small.get() + kSmallEntries), true);
+    unsigned long long fin[2];
+    c.read(fin, overflow, sizeof fin);
+    if (fin[0]) throw std::runtime_error("coarse edge weight exceeds uint32");
+    const std::int64_t mc = (std::int64_t)fin[1];
     if (mc > 0x7fffffffLL) throw std::runtime_error("coarse graph exceeds int32 offsets");
     out->m = mc;
     out->off = c.buf<std::int32_t>(static_cast<std::size_t>(nc + 1));
@@ -2023,8 +2146,7 @@ std::unique_ptr<DGraph> contract(Context& c, const DGraph& fine, CoarsenState& s
     // weights, each unique entry weighing at least 1) the degree bound.
     out->row_len_bound = std::min<std::uint64_t>(rb[1], out->max_degree);
     st.max_row_weight = crb;
-    st.row_bound = c.buf<std::uint64_t>(static_cast<std::size_t>(nc));
-    c.copy_d2d(st.row_bound.get(), next_rb.get(), static_cast<std::size_t>(nc) * sizeof(std::uint64_t));
+    st.row_bound = std::move(next_bounds);
     return out;
 }
 

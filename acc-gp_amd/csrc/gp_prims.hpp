@@ -5,6 +5,8 @@
 #pragma once
 #include "gp_runtime.hpp"
 
+#include <algorithm>
+
 namespace gp {
 
 // ------------------------------------------------------------------ fill
@@ -118,9 +120,10 @@ __device__ inline SegU64 shfl_val(SegU64 x, int src) {
 
 // Tile layout: wave w owns the contiguous kScanItems * 64 elements at
 // base + w * kScanItems * 64, read in rounds of 64 consecutive elements so
-// that every load and store instruction covers contiguous memory.
+// that every load and store instruction covers contiguous memory.  In: a
+// pointer, or an object whose operator[] gives the element.
 template <typename Op, typename T, typename In>
-__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const In* in, std::int64_t n, T* partial) {
+__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(In in, std::int64_t n, T* partial) {
     __shared__ T wsum[kScanThreads / kWave];
     const int lane = lane_id(), w = threadIdx.x / kWave;
     const std::int64_t base = blockIdx.x * (std::int64_t)kScanTile + w * (kScanItems * kWave);
@@ -141,7 +144,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const In* in, std:
 
 // Exclusive scan of the block partials by one block (loops over chunks).
 template <typename Op, typename T>
-__global__ void __launch_bounds__(kScanThreads) k_scan_partials(T* partial, std::int64_t nb, T* total) {
+__global__ void __launch_bounds__(kScanThreads) k_scan_partials(T* partial, std::int64_t nb) {
     __shared__ T wsum[kScanThreads / kWave];
     T carry = Op::template id<T>();
     for (std::int64_t base = 0; base < nb; base += kScanThreads) {
@@ -152,15 +155,37 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_partials(T* partial, std:
         if (idx < nb) partial[idx] = Op::template op<T>(carry, exc);
         carry = Op::template op<T>(carry, tot);
     }
-    if (threadIdx.x == 0 && total) *total = carry;
 }
 
-// Final pass; exclusive=true writes out[i] = prefix before i.
+// Where a scan writes besides out: the total of all elements (null: nowhere),
+// and with closed also to out[n]; copy gets what out gets (null: nothing).
+template <typename T, typename Out>
+struct ScanExtra {
+    T* total;
+    bool closed;
+    Out* copy;
+};
+
+// Final pass; exclusive=true writes out[i] = prefix before i.  summed: the
+// partials are the tiles' own sums and every block combines the earlier ones
+// itself, in order; otherwise they are prefixes already.
 template <typename Op, typename T, typename In, typename Out>
-__global__ void __launch_bounds__(kScanThreads) k_scan_apply(const In* in, Out* out, std::int64_t n, const T* partial,
-                                                             bool exclusive) {
+__global__ void __launch_bounds__(kScanThreads) k_scan_apply(In in, Out* out, std::int64_t n, const T* partial,
+                                                             bool summed, bool exclusive, ScanExtra<T, Out> extra) {
     __shared__ T wsum[kScanThreads / kWave];
     const int lane = lane_id(), w = threadIdx.x / kWave;
+    T before = Op::template id<T>();
+    if (!partial) {
+    } else if (summed) {
+        const std::int64_t nb = blockIdx.x, per = (nb + kScanThreads - 1) / kScanThreads;
+        T acc = Op::template id<T>();
+        for (std::int64_t i = threadIdx.x * per; i < (threadIdx.x + 1) * per && i < nb; ++i)
+            acc = Op::template op<T>(acc, partial[i]);
+        T inc, exc;
+        block_scan<Op>(acc, wsum, inc, exc, before);
+    } else {
+        before = partial[blockIdx.x];
+    }
     const std::int64_t base = blockIdx.x * (std::int64_t)kScanTile + w * (kScanItems * kWave);
     T inc[kScanItems], own[kScanItems];
     T acc = Op::template id<T>();
@@ -173,7 +198,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const In* in, Out* 
     }
     if (lane == 0) wsum[w] = acc;
     __syncthreads();
-    T carry = partial[blockIdx.x];
+    T carry = before;
     for (int i = 0; i < w; ++i) carry = Op::template op<T>(carry, wsum[i]);
 #pragma unroll
     for (int r = 0; r < kScanItems; ++r) {
@@ -182,48 +207,126 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const In* in, Out* 
         // exclusive: the inclusive value of the previous lane (or carry)
         T prev = shfl_up_val(full, 1);
         if (lane == 0) prev = carry;
-        if (idx < n) out[idx] = static_cast<Out>(exclusive ? prev : full);
+        if (idx < n) {
+            const Out o = static_cast<Out>(exclusive ? prev : full);
+            out[idx] = o;
+            if (extra.copy) extra.copy[idx] = o;
+        }
         carry = Op::template op<T>(carry, shfl_val(inc[r], kWave - 1));
+    }
+    // The last wave of the last block now carries the total.
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanThreads - 1) {
+        if (extra.total) *extra.total = carry;
+        if (extra.closed) out[n] = static_cast<Out>(carry);
     }
 }
 
+// Blocks up to which the final pass adds the earlier tiles' sums up itself (at
+// most 8 per thread): two launches instead of three; one tile takes one.
+constexpr std::int64_t kScanSelfMax = 8 * kScanThreads;
+
 // Scan n elements of In into Out (in == out allowed).  Accumulates in T.
-// total (device, optional) receives the reduction of all elements.
 template <typename Op, typename T, typename In, typename Out>
-inline void scan(Context& c, const In* in, Out* out, std::int64_t n, bool exclusive, T* total = nullptr) {
+inline void scan(Context& c, In in, Out* out, std::int64_t n, bool exclusive,
+                 ScanExtra<T, Out> extra = ScanExtra<T, Out>{nullptr, false, nullptr}) {
     if (n <= 0) {
-        if (total) fill<T>(c, total, 1, T{});
+        if (extra.total) fill<T>(c, extra.total, 1, T{});
+        if (extra.closed) fill<Out>(c, out, 1, Out{});
         return;
     }
     const std::int64_t nb = (n + kScanTile - 1) / kScanTile;
-    DBuf<T> partial = c.buf<T>(static_cast<std::size_t>(nb));
-    hipLaunchKernelGGL((k_scan_reduce<Op, T, In>), dim3(static_cast<unsigned>(nb)), dim3(kScanThreads), 0,
-                       c.stream(), in, n, partial.get());
-    GP_LAUNCH_CHECK();
-    hipLaunchKernelGGL((k_scan_partials<Op, T>), dim3(1), dim3(kScanThreads), 0, c.stream(), partial.get(), nb,
-                       total);
-    GP_LAUNCH_CHECK();
+    DBuf<T> partial;
+    if (nb > 1) {
+        partial = c.buf<T>(static_cast<std::size_t>(nb));
+        hipLaunchKernelGGL((k_scan_reduce<Op, T, In>), dim3(static_cast<unsigned>(nb)), dim3(kScanThreads), 0,
+                           c.stream(), in, n, partial.get());
+        GP_LAUNCH_CHECK();
+    }
+    if (nb > kScanSelfMax) {
+        hipLaunchKernelGGL((k_scan_partials<Op, T>), dim3(1), dim3(kScanThreads), 0, c.stream(), partial.get(), nb);
+        GP_LAUNCH_CHECK();
+    }
     hipLaunchKernelGGL((k_scan_apply<Op, T, In, Out>), dim3(static_cast<unsigned>(nb)), dim3(kScanThreads), 0,
-                       c.stream(), in, out, n, partial.get(), exclusive);
+                       c.stream(), in, out, n, partial.get(), nb <= kScanSelfMax, exclusive, extra);
     GP_LAUNCH_CHECK();
 }
 
 template <typename T, typename In, typename Out>
-inline void exclusive_sum(Context& c, const In* in, Out* out, std::int64_t n, T* total = nullptr) {
-    scan<PlusOp, T, In, Out>(c, in, out, n, true, total);
+inline void exclusive_sum(Context& c, In in, Out* out, std::int64_t n, T* total = nullptr, bool closed = false,
+                          Out* copy = nullptr) {
+    scan<PlusOp, T, In, Out>(c, in, out, n, true, ScanExtra<T, Out>{total, closed, copy});
 }
 template <typename T, typename In, typename Out>
-inline void inclusive_sum(Context& c, const In* in, Out* out, std::int64_t n, T* total = nullptr) {
-    scan<PlusOp, T, In, Out>(c, in, out, n, false, total);
+inline void inclusive_sum(Context& c, In in, Out* out, std::int64_t n, T* total = nullptr) {
+    scan<PlusOp, T, In, Out>(c, in, out, n, false, ScanExtra<T, Out>{total, false, nullptr});
 }
 
 // ------------------------------------------------------ stable selection
-// out[pos[i]] = i for flagged i, pos = exclusive scan of flags; count -> *count.
-static __global__ void k_select_scatter(const std::uint8_t* flags, const std::int64_t* pos, std::int64_t n,
-                                        std::int32_t* out) {
-    for (std::int64_t i = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (std::int64_t)gridDim.x * blockDim.x)
-        if (flags[i]) out[pos[i]] = static_cast<std::int32_t>(i);
+// Longer inputs: flags counted per tile of consecutive elements, then each
+// block adds the earlier tiles' counts up and places its own (two launches;
+// four with a scan of the flags and a scatter).
+constexpr int kSelectThreads = 1024;
+constexpr int kSelectTiles = 1024;  // at most: one count per thread of a block
+constexpr int kSelectRounds = 4;    // rounds of kSelectThreads elements in a tile, more above 4 M elements
+inline int select_rounds(std::int64_t n) {
+    return std::max(kSelectRounds, ceil_div(n, (std::int64_t)kSelectTiles * kSelectThreads));
+}
+static __global__ void __launch_bounds__(kSelectThreads) k_select_count(const std::uint8_t* flags, std::int64_t n,
+                                                                        int rounds, std::int32_t* counts) {
+    __shared__ int total;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    const std::int64_t base = (std::int64_t)blockIdx.x * rounds * kSelectThreads + threadIdx.x;
+    int mine = 0;
+    for (int r = 0; r < rounds; ++r) {
+        const std::int64_t i = base + (std::int64_t)r * kSelectThreads;
+        mine += __popcll(__ballot(i < n && flags[i] != 0));
+    }
+    if (lane_id() == 0 && mine) atomicAdd(&total, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = total;
+}
+
+// Positions of a tile's flagged elements behind those of the earlier tiles:
+// place(position, element).  Returns the number up to the tile's end.  Every
+// thread of a kSelectThreads block calls it.
+template <typename Place>
+__device__ inline std::int64_t select_tile(const std::uint8_t* flags, std::int64_t n, int rounds,
+                                           const std::int32_t* counts, Place place) {
+    constexpr int kWaves = kSelectThreads / kWave;
+    __shared__ int wsum[kWaves];
+    __shared__ int before;
+    const int t = threadIdx.x, w = t / kWave;
+    if (t == 0) before = 0;
+    __syncthreads();
+    int earlier = t < (int)blockIdx.x ? counts[t] : 0;
+    earlier = wave_sum(earlier);
+    if (lane_id() == 0 && earlier) atomicAdd(&before, earlier);
+    __syncthreads();
+    std::int64_t at = before;
+    const std::int64_t base = (std::int64_t)blockIdx.x * rounds * kSelectThreads + t;
+    for (int r = 0; r < rounds; ++r) {
+        const std::int64_t i = base + (std::int64_t)r * kSelectThreads;
+        const bool f = i < n && flags[i] != 0;
+        const unsigned long long m = __ballot(f);
+        if (lane_id() == 0) wsum[w] = __popcll(m);
+        __syncthreads();
+        std::int64_t pos = at;
+        for (int j = 0; j < kWaves; ++j) {
+            if (j < w) pos += wsum[j];
+            at += wsum[j];
+        }
+        if (f) place(pos + __popcll(m & ((1ULL << lane_id()) - 1ULL)), i);
+        __syncthreads();
+    }
+    return at;
+}
+static __global__ void __launch_bounds__(kSelectThreads) k_select_write(const std::uint8_t* flags, std::int64_t n,
+                                                                        int rounds, const std::int32_t* counts,
+                                                                        std::int32_t* out, std::int64_t* count_dev) {
+    const std::int64_t at = select_tile(flags, n, rounds, counts,
+                                        [&](std::int64_t j, std::int64_t i) { out[j] = static_cast<std::int32_t>(i); });
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *count_dev = at;
 }
 // Short inputs: one block walks the flags in rounds of 1024 (ballot ranks
 // inside waves, wave counts through LDS), one launch instead of four.
@@ -262,13 +365,18 @@ inline void stable_select(Context& c, const std::uint8_t* flags, std::int64_t n,
         GP_LAUNCH_CHECK();
         return;
     }
-    DBuf<std::int64_t> pos = c.buf<std::int64_t>(static_cast<std::size_t>(n > 0 ? n : 1));
-    exclusive_sum<std::int64_t>(c, flags, pos.get(), n, count_dev);
-    if (n > 0) {
-        const int blocks = static_cast<int>(std::min<std::int64_t>(ceil_div(n, 256), 8192));
-        hipLaunchKernelGGL(k_select_scatter, dim3(blocks), dim3(256), 0, c.stream(), flags, pos.get(), n, out);
-        GP_LAUNCH_CHECK();
+    if (n <= 0) {
+        fill<std::int64_t>(c, count_dev, 1, 0);
+        return;
     }
+    const int rounds = select_rounds(n), tiles = ceil_div(n, (std::int64_t)rounds * kSelectThreads);
+    DBuf<std::int32_t> counts = c.buf<std::int32_t>(static_cast<std::size_t>(tiles));
+    hipLaunchKernelGGL(k_select_count, dim3(tiles), dim3(kSelectThreads), 0, c.stream(), flags, n, rounds,
+                       counts.get());
+    GP_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_select_write, dim3(tiles), dim3(kSelectThreads), 0, c.stream(), flags, n, rounds,
+                       counts.get(), out, count_dev);
+    GP_LAUNCH_CHECK();
 }
 
 // ---------------------------------------------------------------- radix sort
@@ -545,23 +653,48 @@ __device__ inline bool block_is_last(unsigned int* ticket) {
     return last;
 }
 
-// ---------------------------------------------------------- reductions
-// One global atomic per block (blocks of at most 1024 threads).
-template <typename T>
-__global__ void k_reduce_max(const T* in, std::int64_t n, unsigned long long* out) {
+// A kernel's result for the host: `word` (zero before, zero again afterwards)
+// gathers one addition or maximum per block, and the last block hands the
+// outcome over in host[0] and, when `second` is not null, *second in host[1].
+// Called by every thread of every block, of at most 16 waves; few blocks, as
+// their atomics on the word queue up (12 ns each).
+struct HostResult {
+    unsigned long long* word;
+    unsigned int* ticket;
+    unsigned long long* host;
+    unsigned long long* flag;
+    unsigned long long seq;
+    const std::int64_t* second;
+};
+constexpr int kResultThreads = 1024;
+constexpr int kResultBlocks = 128;
+template <bool Max>
+__device__ inline void publish_result(unsigned long long mine, const HostResult& r) {
     __shared__ unsigned long long part[16];
-    unsigned long long m = 0;
-    for (std::int64_t i = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (std::int64_t)gridDim.x * blockDim.x)
-        m = m > (unsigned long long)in[i] ? m : (unsigned long long)in[i];
-    m = wave_max(m);
-    if (lane_id() == 0) part[threadIdx.x / kWave] = m;
+    mine = Max ? (unsigned long long)wave_max((std::uint64_t)mine) : wave_sum(mine);
+    if (lane_id() == 0) part[threadIdx.x / kWave] = mine;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (unsigned w = 1; w < blockDim.x / kWave; ++w) m = m > part[w] ? m : part[w];
-        if (m) atomicMax(out, m);
+        for (unsigned w = 1; w < blockDim.x / kWave; ++w) mine = Max ? (part[w] > mine ? part[w] : mine) : mine + part[w];
+        if (mine) Max ? atomicMax(r.word, mine) : atomicAdd(r.word, mine);
     }
+    if (!block_is_last(r.ticket)) return;
+    if (threadIdx.x == 0) {
+        r.host[0] = atomicExch(r.word, 0ULL);
+        if (r.second) r.host[1] = (unsigned long long)*r.second;
+    }
+    publish_to_host(r.flag, r.seq);
 }
+// The launch's result words, with a new sequence number, and the wait for it.
+inline HostResult host_result(Context& c, unsigned long long* word, const std::int64_t* second = nullptr) {
+    return HostResult{word, c.ticket(), c.read_buffer(), c.read_flag(), c.next_seq(), second};
+}
+inline int result_grid(std::int64_t n) {
+    return static_cast<int>(std::max<std::int64_t>(1, std::min<std::int64_t>(ceil_div(n, kResultThreads), kResultBlocks)));
+}
+
+// ---------------------------------------------------------- reductions
+// One global atomic per block (blocks of at most 1024 threads).
 template <typename T>
 __global__ void k_reduce_sum(const T* in, std::int64_t n, unsigned long long* out) {
     __shared__ unsigned long long part[16];

@@ -1204,10 +1204,7 @@ __device__ inline void tile_key_sums(const std::int32_t* keys, std::int64_t n, i
 // keys, a scan, ranks, a second compaction and read-back and the set-up took
 // its place before: 14 launches and two host waits, of 20 and three in the
 // whole iteration.)
-constexpr int kSelectThreads = 1024;
 constexpr int kSelectWaves = kSelectThreads / kWave;
-constexpr int kSelectTiles = 1024;  // at most, so that a block can add up the earlier ones
-constexpr int kSelectRounds = 4;    // rounds of kSelectThreads vertices in a tile, more above 4 M vertices
 
 // A live donor as the attempts read it: index into the eligible list, the
 // vertex, its weight and label (one 16-byte load per donor).
@@ -1341,33 +1338,11 @@ __global__ void __launch_bounds__(kSelectThreads) k_select_eligible(RefArgs a, S
 }
 
 __global__ void __launch_bounds__(kSelectThreads) k_select_place(RefArgs a, SelectState q, int rounds) {
-    __shared__ int wsum[kSelectWaves];
-    __shared__ int before;
-    const int t = threadIdx.x, w = t / kWave;
-    if (t == 0) before = 0;
-    __syncthreads();
-    int earlier = t < (int)blockIdx.x ? q.counts[t] : 0;
-    earlier = wave_sum(earlier);
-    if (lane_id() == 0 && earlier) atomicAdd(&before, earlier);
     if (blockIdx.x == 0) select_parts(a, q);
-    __syncthreads();
-    std::int64_t at = before;
-    const std::int64_t base = (std::int64_t)blockIdx.x * rounds * kSelectThreads + t;
-    for (int r = 0; r < rounds; ++r) {
-        const std::int64_t v = base + (std::int64_t)r * kSelectThreads;
-        const bool el = v < a.n && q.elig[v];
-        const unsigned long long m = __ballot(el);
-        if (lane_id() == 0) wsum[w] = __popcll(m);
-        __syncthreads();
-        std::int64_t pos = at;
-        for (int j = 0; j < kSelectWaves; ++j) {
-            if (j < w) pos += wsum[j];
-            at += wsum[j];
-        }
-        if (el) select_place(a, q, pos + __popcll(m & ((1ULL << lane_id()) - 1ULL)), (std::int32_t)v);
-        __syncthreads();
-    }
-    if (blockIdx.x == gridDim.x - 1 && t == 0) select_counts(a, q, (unsigned long long)at);
+    const std::int64_t at = select_tile(q.elig, a.n, rounds, q.counts, [&](std::int64_t j, std::int64_t v) {
+        select_place(a, q, j, (std::int32_t)v);
+    });
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) select_counts(a, q, (unsigned long long)at);
 }
 
 // Donor selection of a repair iteration on a level of at most
@@ -3457,7 +3432,7 @@ public:
     RepairBuffers repair_buffers() {
         RepairBuffers b;
         const std::size_t n = static_cast<std::size_t>(a_.n), k = static_cast<std::size_t>(a_.k);
-        b.rounds = std::max(kSelectRounds, ceil_div(a_.n, (std::int64_t)kSelectTiles * kSelectThreads));
+        b.rounds = select_rounds(a_.n);
         b.tiles = ceil_div(a_.n, (std::int64_t)b.rounds * kSelectThreads);
         b.prefix = c_.buf<unsigned long long>(k * kBalanceWidth);
         b.bstar = c_.buf<std::int32_t>(k);
