@@ -135,92 +135,98 @@ constexpr std::int64_t kWideDegree = 16;
 constexpr int kRecursions = 8;
 constexpr int kPasses = 8;
 
+// A subset of the coarsest graph with its own adjacency: vertices in ascending
+// id, entries that leave the subset (and self loops) left out, so that a
+// bisection walks only what it can move.  Each half's is cut out of its
+// parent's.
+struct Subset {
+    std::vector<std::int32_t> ids, off, nbr;
+    std::vector<std::uint32_t> ew, vw;
+    std::int32_t size() const { return static_cast<std::int32_t>(ids.size()); }
+};
+
+// Indexed binary max-heap of subset slots keyed by (gain, lower slot); the
+// entries carry their gain, so that a comparison stays within the heap.
+struct GainHeap {
+    struct Entry {
+        std::int64_t gain;
+        std::int32_t slot;
+        bool above(const Entry& o) const { return gain != o.gain ? gain > o.gain : slot < o.slot; }
+    };
+    std::vector<Entry> heap;
+    std::vector<std::int32_t> where;  // where[i] = heap position of slot i, -1 outside
+    void place(std::size_t at, const Entry& x) {
+        heap[at] = x;
+        where[static_cast<std::size_t>(x.slot)] = static_cast<std::int32_t>(at);
+    }
+    void up(std::size_t at, const Entry x) {
+        while (at && x.above(heap[(at - 1) / 2])) {
+            place(at, heap[(at - 1) / 2]);
+            at = (at - 1) / 2;
+        }
+        place(at, x);
+    }
+    void down(std::size_t at, const Entry x) {
+        for (;;) {
+            std::size_t c = 2 * at + 1;
+            if (c >= heap.size()) break;
+            if (c + 1 < heap.size() && heap[c + 1].above(heap[c])) ++c;
+            if (!heap[c].above(x)) break;
+            place(at, heap[c]);
+            at = c;
+        }
+        place(at, x);
+    }
+    void push(std::int32_t i, std::int64_t gain) {
+        heap.push_back(Entry{gain, i});
+        up(heap.size() - 1, Entry{gain, i});
+    }
+    // Slot i has this gain now (pushed when it was outside).
+    void set(std::int32_t i, std::int64_t gain) {
+        const std::int32_t at = where[static_cast<std::size_t>(i)];
+        if (at < 0) {
+            push(i, gain);
+        } else {
+            const Entry x{gain, i};
+            if (gain > heap[static_cast<std::size_t>(at)].gain) up(static_cast<std::size_t>(at), x);
+            else down(static_cast<std::size_t>(at), x);
+        }
+    }
+    std::int32_t pop() {
+        const std::int32_t top = heap[0].slot;
+        where[static_cast<std::size_t>(top)] = -1;
+        const Entry last = heap.back();
+        heap.pop_back();
+        if (!heap.empty()) down(0, last);
+        return top;
+    }
+};
+
 struct Bisector {
-    std::int64_t n;
-    const std::int32_t* off;
-    const std::int32_t* nbr;
-    const std::uint32_t* ew;
-    const std::uint32_t* vw;
     std::uint32_t seed;
     std::int32_t* labels;
-    std::vector<std::int32_t> pos;  // subset slot of each vertex, -1 outside
     int growths_per_bisection;
     int refined_per_bisection;
+    // Scratch of one bisection, kept across the recursion.
+    std::vector<std::int64_t> gain, internal;
+    std::vector<std::uint8_t> locked, visited, grown;
+    std::vector<std::int32_t> moves, queue, slot;
+    GainHeap H;
 
-    std::uint64_t w(std::int32_t v) const { return vw ? vw[v] : 1u; }
-    std::int64_t e(std::int64_t x) const { return ew ? static_cast<std::int64_t>(ew[x]) : 1; }
     static std::uint64_t dev(std::uint64_t a, std::uint64_t b) { return a > b ? a - b : b - a; }
-
-    // Indexed binary max-heap of subset slots keyed by (gain, lower vertex id).
-    struct GainHeap {
-        std::vector<std::int32_t> heap, where;  // where[i] = heap slot of i, -1 outside
-        const std::vector<std::int64_t>* gain = nullptr;
-        const std::vector<std::int32_t>* ids = nullptr;
-        bool above(std::int32_t x, std::int32_t y) const {
-            const std::int64_t gx = (*gain)[static_cast<std::size_t>(x)], gy = (*gain)[static_cast<std::size_t>(y)];
-            return gx != gy ? gx > gy : (*ids)[static_cast<std::size_t>(x)] < (*ids)[static_cast<std::size_t>(y)];
-        }
-        void place(std::size_t slot, std::int32_t x) {
-            heap[slot] = x;
-            where[static_cast<std::size_t>(x)] = static_cast<std::int32_t>(slot);
-        }
-        void up(std::size_t slot) {
-            const std::int32_t x = heap[slot];
-            while (slot && above(x, heap[(slot - 1) / 2])) {
-                place(slot, heap[(slot - 1) / 2]);
-                slot = (slot - 1) / 2;
-            }
-            place(slot, x);
-        }
-        void down(std::size_t slot) {
-            const std::int32_t x = heap[slot];
-            for (;;) {
-                std::size_t c = 2 * slot + 1;
-                if (c >= heap.size()) break;
-                if (c + 1 < heap.size() && above(heap[c + 1], heap[c])) ++c;
-                if (!above(heap[c], x)) break;
-                place(slot, heap[c]);
-                slot = c;
-            }
-            place(slot, x);
-        }
-        bool has(std::int32_t x) const { return where[static_cast<std::size_t>(x)] >= 0; }
-        void push(std::int32_t x) {
-            heap.push_back(x);
-            up(heap.size() - 1);
-        }
-        void update(std::int32_t x) {
-            up(static_cast<std::size_t>(where[static_cast<std::size_t>(x)]));
-            down(static_cast<std::size_t>(where[static_cast<std::size_t>(x)]));
-        }
-        std::int32_t pop() {
-            const std::int32_t top = heap[0];
-            where[static_cast<std::size_t>(top)] = -1;
-            const std::int32_t last = heap.back();
-            heap.pop_back();
-            if (!heap.empty()) {
-                place(0, last);
-                down(0);
-            }
-            return top;
-        }
-    };
 
     // Flip slot i to the other side and bring its neighbours' gains (weight
     // to the other side minus weight to their own) up to date: a neighbour
     // that i joined loses 2w, one that i left gains 2w.  Calls touch(j) for
     // each neighbour slot j.
     template <typename Touch>
-    void flip(const std::vector<std::int32_t>& S, std::vector<std::uint8_t>& side, std::vector<std::int64_t>& gain,
-              std::int32_t i, Touch touch) {
-        const std::size_t ti = static_cast<std::size_t>(i);
-        side[ti] ^= 1;
-        gain[ti] = -gain[ti];
-        const std::int32_t v = S[ti];
-        for (std::int64_t x = off[v]; x < off[v + 1]; ++x) {
-            const std::int32_t j = pos[static_cast<std::size_t>(nbr[x])];
-            if (j < 0 || j == i) continue;
-            gain[static_cast<std::size_t>(j)] += side[static_cast<std::size_t>(j)] == side[ti] ? -2 * e(x) : 2 * e(x);
+    void flip(const Subset& S, std::uint8_t* side, std::int32_t i, Touch touch) {
+        side[i] ^= 1;
+        gain[static_cast<std::size_t>(i)] = -gain[static_cast<std::size_t>(i)];
+        for (std::int32_t x = S.off[static_cast<std::size_t>(i)]; x < S.off[static_cast<std::size_t>(i) + 1]; ++x) {
+            const std::int32_t j = S.nbr[static_cast<std::size_t>(x)];
+            const std::int64_t w2 = 2 * static_cast<std::int64_t>(S.ew[static_cast<std::size_t>(x)]);
+            gain[static_cast<std::size_t>(j)] += side[j] == side[i] ? -w2 : w2;
             touch(j);
         }
     }
@@ -234,26 +240,23 @@ struct Bisector {
     // prefix (balanced before unbalanced, then smaller cut, then smaller
     // deviation), flipping the rest back; passes repeat while they improve,
     // at most kPasses.  Gains carry over between passes.  Returns the cut.
-    std::int64_t refine(const std::vector<std::int32_t>& S, std::vector<std::uint8_t>& side, std::uint64_t& wa,
-                        std::uint64_t target, std::uint64_t tol, std::int64_t cut) {
-        const std::int32_t m = static_cast<std::int32_t>(S.size());
+    std::int64_t refine(const Subset& S, std::uint8_t* side, std::uint64_t& wa, std::uint64_t target,
+                        std::uint64_t tol, std::int64_t cut) {
+        const std::int32_t m = S.size();
         const int stall = std::min(std::max(m / 100, 15), 100);
-        std::vector<std::int64_t> gain(static_cast<std::size_t>(m), 0), internal(static_cast<std::size_t>(m), 0);
+        gain.assign(static_cast<std::size_t>(m), 0);
+        internal.assign(static_cast<std::size_t>(m), 0);
         for (std::int32_t i = 0; i < m; ++i) {
-            const std::int32_t v = S[static_cast<std::size_t>(i)];
-            for (std::int64_t x = off[v]; x < off[v + 1]; ++x) {
-                const std::int32_t j = pos[static_cast<std::size_t>(nbr[x])];
-                if (j < 0 || j == i) continue;
-                const bool other = side[static_cast<std::size_t>(j)] != side[static_cast<std::size_t>(i)];
-                gain[static_cast<std::size_t>(i)] += other ? e(x) : -e(x);
-                internal[static_cast<std::size_t>(i)] += e(x);
+            std::int64_t g = 0, in = 0;
+            for (std::int32_t x = S.off[static_cast<std::size_t>(i)]; x < S.off[static_cast<std::size_t>(i) + 1]; ++x) {
+                const std::int64_t e = S.ew[static_cast<std::size_t>(x)];
+                g += side[S.nbr[static_cast<std::size_t>(x)]] != side[i] ? e : -e;
+                in += e;
             }
+            gain[static_cast<std::size_t>(i)] = g;
+            internal[static_cast<std::size_t>(i)] = in;
         }
-        std::vector<std::uint8_t> locked(static_cast<std::size_t>(m));
-        std::vector<std::int32_t> moves;
-        GainHeap H;
-        H.gain = &gain;
-        H.ids = &S;
+        locked.resize(static_cast<std::size_t>(m));
         H.where.assign(static_cast<std::size_t>(m), -1);
         const auto key = [&](std::uint64_t x, std::int64_t c) {
             return std::make_tuple(dev(x, target) > tol ? 1 : 0, c, dev(x, target));
@@ -264,7 +267,8 @@ struct Bisector {
                 locked[static_cast<std::size_t>(i)] = 0;
                 H.where[static_cast<std::size_t>(i)] = -1;
                 // on the boundary: some weight to the other side
-                if (gain[static_cast<std::size_t>(i)] > -internal[static_cast<std::size_t>(i)]) H.push(i);
+                if (gain[static_cast<std::size_t>(i)] > -internal[static_cast<std::size_t>(i)])
+                    H.push(i, gain[static_cast<std::size_t>(i)]);
             }
             moves.clear();
             auto best = key(wa, cut);
@@ -275,17 +279,15 @@ struct Bisector {
             while (!H.heap.empty() && since_best <= stall) {
                 const std::int32_t i = H.pop();
                 const std::size_t ti = static_cast<std::size_t>(i);
-                const std::uint64_t wv = w(S[ti]);
-                const std::uint64_t nwa = side[ti] == 0 ? cur_wa - wv : cur_wa + wv;
+                const std::uint64_t wv = S.vw[ti];
+                const std::uint64_t nwa = side[i] == 0 ? cur_wa - wv : cur_wa + wv;
                 if (dev(nwa, target) > tol && dev(nwa, target) >= dev(cur_wa, target)) continue;
                 locked[ti] = 1;
                 cur_wa = nwa;
                 cur_cut -= gain[ti];
                 moves.push_back(i);
-                flip(S, side, gain, i, [&](std::int32_t j) {
-                    if (locked[static_cast<std::size_t>(j)]) return;
-                    if (H.has(j)) H.update(j);
-                    else H.push(j);
+                flip(S, side, i, [&](std::int32_t j) {
+                    if (!locked[static_cast<std::size_t>(j)]) H.set(j, gain[static_cast<std::size_t>(j)]);
                 });
                 const auto now = key(cur_wa, cur_cut);
                 if (now < best) {
@@ -298,9 +300,9 @@ struct Bisector {
             }
             for (std::size_t q = moves.size(); q > best_len; --q) {
                 const std::int32_t i = moves[q - 1];
-                const std::uint64_t wv = w(S[static_cast<std::size_t>(i)]);
-                cur_wa = side[static_cast<std::size_t>(i)] == 0 ? cur_wa - wv : cur_wa + wv;
-                flip(S, side, gain, i, [](std::int32_t) {});
+                const std::uint64_t wv = S.vw[static_cast<std::size_t>(i)];
+                cur_wa = side[i] == 0 ? cur_wa - wv : cur_wa + wv;
+                flip(S, side, i, [](std::int32_t) {});
             }
             wa = cur_wa;
             cut = std::get<1>(best);
@@ -309,74 +311,94 @@ struct Bisector {
         return cut;
     }
 
-    void bisect(std::vector<std::int32_t>& S, int p0, int kk) {
-        if (S.empty()) return;
+    // The vertices of S on the given side, with the entries among them.
+    Subset half(const Subset& S, const std::uint8_t* side, std::uint8_t which) {
+        Subset h;
+        const std::int32_t m = S.size();
+        slot.resize(static_cast<std::size_t>(m));
+        for (std::int32_t i = 0; i < m; ++i)
+            if (side[i] == which) {
+                slot[static_cast<std::size_t>(i)] = static_cast<std::int32_t>(h.ids.size());
+                h.ids.push_back(S.ids[static_cast<std::size_t>(i)]);
+                h.vw.push_back(S.vw[static_cast<std::size_t>(i)]);
+            }
+        h.off.reserve(h.ids.size() + 1);
+        h.off.push_back(0);
+        for (std::int32_t i = 0; i < m; ++i) {
+            if (side[i] != which) continue;
+            for (std::int32_t x = S.off[static_cast<std::size_t>(i)]; x < S.off[static_cast<std::size_t>(i) + 1]; ++x) {
+                const std::int32_t j = S.nbr[static_cast<std::size_t>(x)];
+                if (side[j] != which) continue;
+                h.nbr.push_back(slot[static_cast<std::size_t>(j)]);
+                h.ew.push_back(S.ew[static_cast<std::size_t>(x)]);
+            }
+            h.off.push_back(static_cast<std::int32_t>(h.nbr.size()));
+        }
+        return h;
+    }
+
+    void bisect(const Subset& S, int p0, int kk) {
+        if (S.ids.empty()) return;
         if (kk == 1) {
-            for (auto v : S) labels[v] = p0;
+            for (auto v : S.ids) labels[v] = p0;
             return;
         }
         const int k1 = kk / 2;
         std::uint64_t W = 0, maxw = 0;
-        for (auto v : S) {
-            W += w(v);
-            maxw = std::max(maxw, w(v));
+        for (const std::uint64_t x : S.vw) {
+            W += x;
+            maxw = std::max(maxw, x);
         }
         const std::uint64_t target = (W / kk) * k1 + ((W % kk) * k1) / kk;
         const std::uint64_t tol = std::max<std::uint64_t>(maxw, W / 100);
-        const std::int32_t m = static_cast<std::int32_t>(S.size());
-        for (std::int32_t i = 0; i < m; ++i) pos[static_cast<std::size_t>(S[static_cast<std::size_t>(i)])] = i;
+        const std::int32_t m = S.size();
         // Breadth-first growths of side 0 from hashed starts (restarting at
         // the lowest unvisited slot when a component is exhausted) until it
         // holds the target weight; the cut is kept up to date as vertices
         // join side 0.
-        std::vector<std::vector<std::uint8_t>> grown;
         std::vector<std::tuple<std::int64_t, std::uint64_t, int, std::uint64_t>> rank;  // cut, dev, growth, weight
-        std::vector<std::uint8_t> visited;
-        std::vector<std::int32_t> queue;
         const int growths = std::min<std::int32_t>(growths_per_bisection, m);
+        grown.assign(static_cast<std::size_t>(growths) * static_cast<std::size_t>(m), 1);
         for (int t = 0; t < growths; ++t) {
             const std::uint32_t h = hmix32(seed ^ ((std::uint32_t)p0 * 0x9e3779b9U) ^ ((std::uint32_t)kk * 0x85ebca6bU) ^
                                            ((std::uint32_t)t * 0xc2b2ae35U));
-            std::vector<std::uint8_t> side(static_cast<std::size_t>(m), 1);
+            std::uint8_t* side = grown.data() + static_cast<std::size_t>(t) * static_cast<std::size_t>(m);
             visited.assign(static_cast<std::size_t>(m), 0);
-            queue.clear();
-            std::size_t head = 0;
+            queue.resize(static_cast<std::size_t>(m) + 1);  // one slot to write past the last vertex
+            std::size_t head = 0, tail = 0;
             std::int32_t next_unvisited = 0;
             const std::int32_t s0 = static_cast<std::int32_t>(h % static_cast<std::uint32_t>(m));
-            queue.push_back(s0);
+            queue[tail++] = s0;
             visited[static_cast<std::size_t>(s0)] = 1;
             std::uint64_t wa = 0;
             std::int64_t cut = 0;
             while (wa < target) {
-                if (head == queue.size()) {
+                if (head == tail) {
                     while (next_unvisited < m && visited[static_cast<std::size_t>(next_unvisited)]) ++next_unvisited;
                     if (next_unvisited == m) break;
                     visited[static_cast<std::size_t>(next_unvisited)] = 1;
-                    queue.push_back(next_unvisited);
+                    queue[tail++] = next_unvisited;
                 }
                 const std::int32_t i = queue[head++];
-                side[static_cast<std::size_t>(i)] = 0;
-                const std::int32_t v = S[static_cast<std::size_t>(i)];
-                wa += w(v);
-                for (std::int64_t x = off[v]; x < off[v + 1]; ++x) {
-                    const std::int32_t j = pos[static_cast<std::size_t>(nbr[x])];
-                    if (j < 0 || j == i) continue;
-                    cut += side[static_cast<std::size_t>(j)] == 0 ? -e(x) : e(x);
-                    if (!visited[static_cast<std::size_t>(j)]) {
-                        visited[static_cast<std::size_t>(j)] = 1;
-                        queue.push_back(j);
-                    }
+                side[i] = 0;
+                wa += S.vw[static_cast<std::size_t>(i)];
+                for (std::int32_t x = S.off[static_cast<std::size_t>(i)]; x < S.off[static_cast<std::size_t>(i) + 1]; ++x) {
+                    const std::int32_t j = S.nbr[static_cast<std::size_t>(x)];
+                    const std::int64_t e = S.ew[static_cast<std::size_t>(x)];
+                    cut += e * (2 * static_cast<std::int64_t>(side[j]) - 1);  // no branches: neither is predictable
+                    queue[tail] = j;
+                    tail += !visited[static_cast<std::size_t>(j)];
+                    visited[static_cast<std::size_t>(j)] = 1;
                 }
             }
             rank.emplace_back(cut, dev(wa, target), t, wa);
-            grown.push_back(std::move(side));
         }
         std::sort(rank.begin(), rank.end());
         std::int64_t best_cut = std::numeric_limits<std::int64_t>::max();
         std::uint64_t best_dev = std::numeric_limits<std::uint64_t>::max();
-        std::vector<std::uint8_t> best_side;
+        const std::uint8_t* best_side = nullptr;
         for (std::size_t r = 0; r < rank.size() && r < static_cast<std::size_t>(refined_per_bisection); ++r) {
-            std::vector<std::uint8_t>& side = grown[static_cast<std::size_t>(std::get<2>(rank[r]))];
+            std::uint8_t* side = grown.data() + static_cast<std::size_t>(std::get<2>(rank[r])) * static_cast<std::size_t>(m);
             std::uint64_t wa = std::get<3>(rank[r]);
             const std::int64_t cut = refine(S, side, wa, target, tol, std::get<0>(rank[r]));
             const std::uint64_t d = dev(wa, target);
@@ -386,12 +408,7 @@ struct Bisector {
                 best_side = side;
             }
         }
-        std::vector<std::int32_t> A, B;
-        for (std::int32_t i = 0; i < m; ++i) {
-            (best_side[static_cast<std::size_t>(i)] == 0 ? A : B).push_back(S[static_cast<std::size_t>(i)]);
-            pos[static_cast<std::size_t>(S[static_cast<std::size_t>(i)])] = -1;
-        }
-        std::vector<std::int32_t>().swap(S);
+        const Subset A = half(S, best_side, 0), B = half(S, best_side, 1);
         bisect(A, p0, k1);
         bisect(B, p0 + k1, kk - k1);
     }
@@ -408,16 +425,30 @@ void initial_partition_host(std::int64_t n, const std::int32_t* off, const std::
     const long double raw = (long double)total * (imbalance >= 1.0 ? imbalance : 1.0) / parts;
     const std::uint64_t cap = (std::uint64_t)std::floor(raw);
     const bool wide = off[n] <= kWideEntries && off[n] <= kWideDegree * n;
+    Subset all;
+    all.off.reserve(static_cast<std::size_t>(n) + 1);
+    all.off.push_back(0);
+    for (std::int64_t v = 0; v < n; ++v) {
+        all.ids.push_back(static_cast<std::int32_t>(v));
+        all.vw.push_back(vw ? vw[v] : 1u);
+        for (std::int64_t x = off[v]; x < off[v + 1]; ++x) {
+            if (nbr[x] == v) continue;
+            all.nbr.push_back(nbr[x]);
+            all.ew.push_back(ew ? ew[x] : 1u);
+        }
+        all.off.push_back(static_cast<std::int32_t>(all.nbr.size()));
+    }
     std::vector<std::vector<std::int32_t>> trial(static_cast<std::size_t>(kRecursions));
     std::vector<std::pair<std::uint64_t, std::uint64_t>> score(static_cast<std::size_t>(kRecursions));
     auto run = [&](int t) {
         const std::uint32_t s = t == 0 ? seed : hmix32(seed ^ (0x68e31da4U * (std::uint32_t)t));
         std::vector<std::int32_t>& lab = trial[static_cast<std::size_t>(t)];
         lab.assign(static_cast<std::size_t>(n), 0);
-        Bisector b{n,   off, nbr, ew, vw, s, lab.data(), std::vector<std::int32_t>(static_cast<std::size_t>(n), -1),
-                   wide ? kWideGrowths : kGrowths, wide ? kWideRefined : kRefined};
-        std::vector<std::int32_t> all(static_cast<std::size_t>(n));
-        for (std::int64_t v = 0; v < n; ++v) all[static_cast<std::size_t>(v)] = static_cast<std::int32_t>(v);
+        Bisector b;
+        b.seed = s;
+        b.labels = lab.data();
+        b.growths_per_bisection = wide ? kWideGrowths : kGrowths;
+        b.refined_per_bisection = wide ? kWideRefined : kRefined;
         b.bisect(all, 0, parts);
         std::vector<std::uint64_t> loads(static_cast<std::size_t>(parts), 0);
         std::uint64_t directed = 0;
