@@ -1937,14 +1937,17 @@ __global__ void k_level_begin(unsigned long long* ctr, PartWords loads, unsigned
 __global__ void __launch_bounds__(256) k_heavy_edge(std::int64_t m, const std::uint32_t* ew, unsigned long long* flag) {
     const std::int64_t stride = (std::int64_t)gridDim.x * blockDim.x;
     for (std::int64_t base = blockIdx.x * (std::int64_t)blockDim.x; base < m; base += 8 * stride) {
-        if (*(volatile unsigned long long*)flag) return;
+        if (__syncthreads_or(threadIdx.x == 0 && *(volatile unsigned long long*)flag)) return;
         bool heavy = false;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const std::int64_t x = base + j * stride + threadIdx.x;
             heavy |= x < m && ew[x] > 1;
         }
-        if (heavy) *(volatile unsigned long long*)flag = 1;
+        if (__syncthreads_or(heavy)) {
+            if (threadIdx.x == 0) *(volatile unsigned long long*)flag = 1;
+            return;
+        }
     }
 }
 
@@ -2526,6 +2529,9 @@ __global__ void __launch_bounds__(kGrowWaves* kWave) k_joint_grow(RefArgs a, con
 }
 
 // Orders for the archive and the transaction pool (complementary_moves.cuh:5-14, exchange.cuh:33-40).
+struct MoveKeys {
+    std::int64_t first, second, third;
+};
 struct NetOrder {
     __device__ bool operator()(const JMove& x, const JMove& y) const {  // x before y
         if (x.a != y.a) return x.a < y.a;
@@ -2536,6 +2542,10 @@ struct NetOrder {
             if (x.v[j] != y.v[j]) return x.v[j] < y.v[j];
         return x.id < y.id;
     }
+    // Within a part the order starts with these, ascending.
+    __device__ static MoveKeys keys(const JMove& x) {
+        return MoveKeys{x.net, ~x.gain, (std::int64_t)x.size << 32 | (std::uint32_t)x.v[0]};
+    }
 };
 struct JointOrder {
     __device__ bool operator()(const JMove& x, const JMove& y) const {
@@ -2544,140 +2554,212 @@ struct JointOrder {
         if (x.gain != y.gain) return x.gain > y.gain;
         return x.id < y.id;
     }
+    __device__ static MoveKeys keys(const JMove& x) { return MoveKeys{~x.gain, x.id, 0}; }
 };
 
-template <typename Cmp>
-__device__ inline bool idx_after(int x, int y, const JMove* m, Cmp cmp) {  // x sorts after y
-    if (x < 0) return y >= 0;
-    if (y < 0) return false;
-    return cmp(m[y], m[x]);
-}
-
-template <typename Cmp>
-__global__ void k_bitonic_global(int* idx, int N, int j, int kk, const JMove* m, Cmp cmp) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const int l = i ^ j;
-    if (l <= i) return;
-    const int x = idx[i], y = idx[l];
-    const bool asc = (i & kk) == 0;
-    if (asc ? idx_after(x, y, m, cmp) : idx_after(y, x, m, cmp)) {
-        idx[i] = y;
-        idx[l] = x;
-    }
-}
-// x sorts after y, for local slots of moves staged in LDS (g holds each
-// slot's global index, -1 for padding, which sorts last).
-template <typename Cmp>
-__device__ inline bool slot_after(int x, int y, const int* g, const JMove* mv, Cmp cmp) {
-    if (g[x] < 0) return g[y] >= 0;
-    if (g[y] < 0) return false;
-    return cmp(mv[y], mv[x]);
-}
-
-// Bitonic stages over C indices held by one block, with the moves they
-// name copied into LDS once so that every comparison reads LDS: stages
-// (kk, j) for kk from kk_first to kk_last and j from min(kk, C) / 2 down to
-// 1.  Directions use the global position base + t.
-template <int C, typename Cmp>
-__device__ inline void bitonic_lds(int* idx, int base, int kk_first, int kk_last, const JMove* m, Cmp cmp,
-                                   JMove* mv, int* g, short* s) {
-    for (int i = threadIdx.x; i < C; i += blockDim.x) {
-        const int x = idx[base + i];
-        g[i] = x;
-        s[i] = (short)i;
-        if (x >= 0) mv[i] = m[x];
+// Moves in order without a sorting network over 64-byte records.  Both orders
+// go by the part first and start with three words (keys()); only full ties
+// look at the rest of the records.  Four launches: the non-empty moves per part
+// and block of the source, with the parts' starts from the last block; their
+// indices grouped by part (any order inside); runs of 256 moves of a part
+// sorted by merges in LDS; the runs of a part merged, all by binary searches
+// for each move's place.  The moves of a pair of parts carry its lower part,
+// so a part has up to some 2,000.
+// The bitonic networks that this replaces ran 66 dependent stages over records
+// 64 bytes apart in LDS, 16 lanes to a bank, 64 to 74 us for each chunk of
+// 2,048 moves and several launches for more; comparing all pairs of a part took
+// 96 us for the archive of R-MAT scale 18 (k = 64), runs and merges take 43.
+constexpr int kOrderThreads = 1024;
+__global__ void __launch_bounds__(kOrderThreads) k_moves_count(const JMove* src, int count, int k, int* block_at,
+                                                               int* starts, unsigned int* ticket,
+                                                               unsigned long long* host, unsigned long long* flag,
+                                                               unsigned long long seq) {
+    __shared__ int hist[kMaxParts];
+    __shared__ int first[kMaxParts + 1];
+    const int t = threadIdx.x;
+    if (t < kMaxParts) hist[t] = 0;
+    __syncthreads();
+    const int i = blockIdx.x * kOrderThreads + t;
+    if (i < count && src[i].size) atomicAdd(&hist[src[i].a], 1);
+    __syncthreads();
+    if (t < k) block_at[blockIdx.x * k + t] = hist[t];
+    if (!block_is_last(ticket)) return;
+    int total = 0;
+    if (t < k)
+        for (int b = 0; b < (int)gridDim.x; ++b) total += block_at[b * k + t];
+    if (t < kMaxParts) hist[t] = t < k ? total : 0;
+    __syncthreads();
+    if (t < kWave) {
+        int sum = 0;
+        for (int p0 = 0; p0 < kMaxParts; p0 += kWave) {
+            const int n = hist[p0 + t], inc = wave_inclusive_scan<PlusOp>(n);
+            first[p0 + t] = sum + inc - n;
+            sum += __shfl(inc, kWave - 1);
+        }
+        if (t == 0) first[kMaxParts] = sum;
     }
     __syncthreads();
-    for (int kk = kk_first; kk <= kk_last; kk <<= 1)
-        for (int j = (kk < C ? kk : C) >> 1; j > 0; j >>= 1) {
-            // One compare-exchange pair (t, t + j) per thread.
-            for (int q = threadIdx.x; q < C / 2; q += blockDim.x) {
-                const int t = ((q & ~(j - 1)) << 1) | (q & (j - 1)), l = t + j;
-                const bool asc = ((base + t) & kk) == 0;
-                const int x = s[t], y = s[l];
-                if (asc ? slot_after(x, y, g, mv, cmp) : slot_after(y, x, g, mv, cmp)) {
-                    s[t] = (short)y;
-                    s[l] = (short)x;
+    if (t < k) {
+        int at = first[t];
+        for (int b = 0; b < (int)gridDim.x; ++b) {
+            const int n = block_at[b * k + t];
+            block_at[b * k + t] = at;
+            at += n;
+        }
+        starts[t] = first[t];
+    }
+    if (t == 0) {
+        starts[k] = first[kMaxParts];
+        if (host) host[0] = (unsigned long long)first[kMaxParts];
+    }
+    if (host) publish_to_host(flag, seq);
+}
+
+__global__ void __launch_bounds__(kOrderThreads) k_moves_group(const JMove* src, int count, int k, const int* block_at,
+                                                               int* order) {
+    __shared__ int at[kMaxParts];
+    const int t = threadIdx.x;
+    if (t < k) at[t] = block_at[blockIdx.x * k + t];
+    __syncthreads();
+    const int i = blockIdx.x * kOrderThreads + t;
+    if (i < count && src[i].size) order[atomicAdd(&at[src[i].a], 1)] = i;
+}
+
+constexpr int kRankThreads = 256;
+constexpr int kRankSplit = 8;  // blocks per part
+__device__ inline bool keys_less(const MoveKeys& x, const MoveKeys& y) {
+    return x.first < y.first ||
+           (x.first == y.first && (x.second < y.second || (x.second == y.second && x.third < y.third)));
+}
+__device__ inline bool keys_equal(const MoveKeys& x, const MoveKeys& y) {
+    return x.first == y.first && x.second == y.second && x.third == y.third;
+}
+
+// Sorts each run of kRankThreads moves of a part (indices in order[]) into
+// runs[]: merges of doubling width in LDS, a move's new place in each found by
+// a binary search in the neighbouring run (36 search steps in all).  Equal
+// moves (nothing tells them apart) keep their order.
+template <typename Cmp>
+__global__ void __launch_bounds__(kRankThreads) k_moves_runs(const JMove* src, const int* starts, const int* order,
+                                                             Cmp before, JMove* runs) {
+    __shared__ JMove tile[kRankThreads];
+    __shared__ std::int64_t first[kRankThreads], second[kRankThreads], third[kRankThreads];
+    __shared__ short at[2][kRankThreads];  // slots of the moves, by place
+    const int t = threadIdx.x, b0 = starts[blockIdx.x], n = starts[blockIdx.x + 1] - b0;
+    for (int j0 = blockIdx.y * kRankThreads; j0 < n; j0 += kRankSplit * kRankThreads) {
+        const int c = n - j0 < kRankThreads ? n - j0 : kRankThreads;
+        __syncthreads();
+        if (t < c) {
+            tile[t] = src[order[b0 + j0 + t]];
+            const MoveKeys k = Cmp::keys(tile[t]);
+            first[t] = k.first;
+            second[t] = k.second;
+            third[t] = k.third;
+            at[0][t] = (short)t;
+        }
+        __syncthreads();
+        int from = 0;
+        for (int width = 1; width < c; width <<= 1, from ^= 1) {
+            if (t < c) {
+                const int run = t / width, other = run ^ 1, r0 = other * width;
+                const int slot = at[from][t];
+                const MoveKeys mine{first[slot], second[slot], third[slot]};
+                int lo = 0, hi = c - r0 < width ? c - r0 : width;
+                while (lo < hi) {  // moves of the other run before this one
+                    const int mid = (lo + hi) >> 1, y = at[from][r0 + mid];
+                    const MoveKeys o{first[y], second[y], third[y]};
+                    bool earlier = keys_less(o, mine);
+                    if (!earlier && keys_equal(o, mine))
+                        earlier = before(tile[y], tile[slot]) || (other < run && !before(tile[slot], tile[y]));
+                    if (earlier) lo = mid + 1;
+                    else hi = mid;
                 }
+                at[from ^ 1][(run & ~1) * width + (t & (width - 1)) + lo] = (short)slot;
             }
             __syncthreads();
         }
-    for (int i = threadIdx.x; i < C; i += blockDim.x) idx[base + i] = g[s[i]];
-}
-
-// The stages of a bitonic network whose partners lie in one aligned chunk
-// of kBitonicChunk indices, run in LDS by one block per chunk: every stage
-// of the merges up to the chunk size (kk == 0), or the stages j < chunk of
-// the merge of size kk.  The chunk's moves (64 bytes each) take 128 KiB of
-// LDS.
-constexpr int kBitonicChunk = 2048;
-template <typename Cmp>
-__global__ void __launch_bounds__(1024) k_bitonic_chunk(int* idx, int kk_fixed, const JMove* m, Cmp cmp) {
-    __shared__ JMove mv[kBitonicChunk];
-    __shared__ int g[kBitonicChunk];
-    __shared__ short s[kBitonicChunk];
-    const int base = blockIdx.x * kBitonicChunk;
-    if (kk_fixed == 0)
-        bitonic_lds<kBitonicChunk>(idx, base, 2, kBitonicChunk, m, cmp, mv, g, s);
-    else
-        bitonic_lds<kBitonicChunk>(idx, base, kk_fixed, kk_fixed, m, cmp, mv, g, s);
-}
-
-// Whole sort of N <= 1024 indices (N a power of two) in one block.
-template <typename Cmp>
-__global__ void __launch_bounds__(1024) k_bitonic_local(int* idx, int N, const JMove* m, Cmp cmp) {
-    __shared__ JMove mv[1024];
-    __shared__ int g[1024];
-    __shared__ short s[1024];
-    for (int i = threadIdx.x; i < N; i += blockDim.x) {
-        const int x = idx[i];
-        g[i] = x;
-        s[i] = (short)i;
-        if (x >= 0) mv[i] = m[x];
+        if (t < c) runs[b0 + j0 + t] = tile[at[from][t]];
     }
-    __syncthreads();
-    for (int kk = 2; kk <= N; kk <<= 1)
-        for (int j = kk >> 1; j > 0; j >>= 1) {
-            for (int q = threadIdx.x; q < N / 2; q += blockDim.x) {
-                const int t = ((q & ~(j - 1)) << 1) | (q & (j - 1)), l = t + j;
-                const bool asc = (t & kk) == 0;
-                const int x = s[t], y = s[l];
-                if (asc ? slot_after(x, y, g, mv, cmp) : slot_after(y, x, g, mv, cmp)) {
-                    s[t] = (short)y;
-                    s[l] = (short)x;
-                }
-            }
-            __syncthreads();
-        }
-    for (int i = threadIdx.x; i < N; i += blockDim.x) idx[i] = g[s[i]];
 }
 
-__global__ void k_nonempty_moves(const JMove* m, int count, std::uint8_t* f) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) f[i] = m[i].size != 0;
+// Merges a part's runs: a move's place is its place in its run plus, for every
+// other run, the moves of that run before it, found by binary search over keys
+// staged kMergeRuns runs at a time.  Of equal moves the earlier run's are first.
+constexpr int kMergeRuns = 8;
+template <typename Cmp>
+__global__ void __launch_bounds__(kRankThreads) k_moves_merge(const JMove* runs, const int* starts, Cmp before,
+                                                              JMove* out) {
+    __shared__ MoveKeys key[kMergeRuns * kRankThreads];
+    const int t = threadIdx.x, b0 = starts[blockIdx.x], n = starts[blockIdx.x + 1] - b0;
+    for (int j0 = blockIdx.y * kRankThreads; j0 < n; j0 += kRankSplit * kRankThreads) {
+        const bool have = j0 + t < n;
+        const JMove own = have ? runs[b0 + j0 + t] : jmove_empty();
+        const MoveKeys mine = Cmp::keys(own);
+        int rank = t;
+        for (int s0 = 0; s0 < n; s0 += kMergeRuns * kRankThreads) {
+            __syncthreads();
+            for (int x = t; x < kMergeRuns * kRankThreads && s0 + x < n; x += kRankThreads)
+                key[x] = Cmp::keys(runs[b0 + s0 + x]);
+            __syncthreads();
+            for (int r = 0; r < kMergeRuns; ++r) {
+                const int r0 = s0 + r * kRankThreads;
+                if (r0 >= n) break;
+                if (r0 == j0 || !have) continue;
+                int lo = 0, hi = n - r0 < kRankThreads ? n - r0 : kRankThreads;
+                while (lo < hi) {  // moves of the run before this one
+                    const int mid = (lo + hi) >> 1;
+                    const MoveKeys o = key[r * kRankThreads + mid];
+                    bool earlier = keys_less(o, mine);
+                    if (!earlier && keys_equal(o, mine)) {
+                        const JMove m = runs[b0 + r0 + mid];
+                        earlier = before(m, own) || (r0 < j0 && !before(own, m));
+                    }
+                    if (earlier) lo = mid + 1;
+                    else hi = mid;
+                }
+                rank += lo;
+            }
+        }
+        if (have) out[b0 + rank] = own;
+    }
 }
-__global__ void k_gather_moves(const JMove* src, const int* idx, int count, JMove* dst) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) dst[i] = src[idx[i]];
-}
-// exchange.cuh:19-32 equality of consecutive sorted archive entries.
-__global__ void k_unique_flags(const JMove* m, int count, std::uint8_t* f) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    bool keep = true;
-    if (i > 0) {
-        const JMove& x = m[i - 1];
-        const JMove& y = m[i];
+
+// exchange.cuh:19-32 equality of consecutive sorted archive entries: flags the
+// moves that do not repeat the one before, and counts them per tile; the
+// second launch places them in order and hands their number to the host.  The
+// number of moves is read on the device; the grid covers the most there can be.
+__global__ void __launch_bounds__(kSelectThreads) k_unique_flags(const JMove* m, const int* count_dev,
+                                                                 std::uint8_t* flags, std::int32_t* counts) {
+    __shared__ int total;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    const int count = *count_dev, i = blockIdx.x * kSelectThreads + threadIdx.x;
+    bool keep = i < count;
+    if (keep && i > 0) {
+        const JMove x = m[i - 1], y = m[i];
         bool same = x.size && x.size == y.size && x.a == y.a && x.b == y.b && x.gain == y.gain && x.net == y.net;
         for (int j = 0; same && j < x.size; ++j) {
             bool found = false;
-            for (int t = 0; t < y.size; ++t) found |= x.v[j] == y.v[t];
+            for (int q = 0; q < y.size; ++q) found |= x.v[j] == y.v[q];
             same = found;
         }
         keep = !same;
     }
-    f[i] = keep;
+    if (i < count) flags[i] = keep;
+    const int mine = __popcll(__ballot(keep));
+    if (lane_id() == 0 && mine) atomicAdd(&total, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = total;
+}
+__global__ void __launch_bounds__(kSelectThreads) k_unique_place(const JMove* m, const int* count_dev,
+                                                                 const std::uint8_t* flags, const std::int32_t* counts,
+                                                                 JMove* out, unsigned long long* host,
+                                                                 unsigned long long* flag, unsigned long long seq) {
+    const std::int64_t at =
+        select_tile(flags, *count_dev, 1, counts, [&](std::int64_t j, std::int64_t i) { out[j] = m[i]; });
+    if (blockIdx.x != gridDim.x - 1) return;
+    if (threadIdx.x == 0) host[0] = (unsigned long long)at;
+    publish_to_host(flag, seq);
 }
 
 __device__ inline int jnet_bound(const JMove* r, int count, int pa, std::int64_t net, bool upper) {
@@ -2801,12 +2883,6 @@ __global__ void k_joint_resolve(JMove* m, int count, const std::int32_t* owners)
             break;
         }
 }
-// idx[0, m) then -1 up to N (the power-of-two length a bitonic sort takes).
-__global__ void k_pad_index(const std::int32_t* idx, int m, std::int32_t* out, int N) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < N) out[i] = i < m ? idx[i] : -1;
-}
-
 // Clears the owner of every vertex and its moving flag before the claimed
 // transactions are marked and accepted (nothing in between reads the flag).
 __global__ void k_exchange_reset(std::int64_t n, std::int32_t* owners, std::uint32_t* state) {
@@ -3120,7 +3196,7 @@ public:
                            heavy_edge, prices_.get());
         GP_LAUNCH_CHECK();
         if (g.ew && g.m > 0) {
-            hipLaunchKernelGGL(k_heavy_edge, dim3(grid_for(g.m, 256 * 16, 512)), dim3(256), 0, c.stream(), g.m,
+            hipLaunchKernelGGL(k_heavy_edge, dim3(grid_for(g.m, 256 * 16, 256)), dim3(256), 0, c.stream(), g.m,
                                g.ew.get(), heavy_edge);
             GP_LAUNCH_CHECK();
             a_.heavy_edge = heavy_edge;
@@ -3734,61 +3810,46 @@ public:
         ctr_clear_ = false;
     }
 
-    // Stable compaction of non-empty moves, sort by cmp, optional unique.
+    // The non-empty moves of src in cmp order, repeats dropped when unique is
+    // set; their number (out holds room for `count`).
     template <typename Cmp>
     int compact_sort(const JMove* src, int count, Cmp cmp, DBuf<JMove>& out, bool unique) {
         const hipStream_t s = c_.stream();
         if (count <= 0) return 0;
-        DBuf<std::uint8_t> f = c_.buf<std::uint8_t>(static_cast<std::size_t>(count));
-        DBuf<std::int32_t> idx = c_.buf<std::int32_t>(static_cast<std::size_t>(count));
-        DBuf<std::int64_t> cnt = c_.buf<std::int64_t>(1);
-        hipLaunchKernelGGL(k_nonempty_moves, dim3(ceil_div(count, 256)), dim3(256), 0, s, src, count, f.get());
+        const int k = a_.k, blocks = ceil_div(count, kOrderThreads);
+        DBuf<std::int32_t> block_at = c_.buf<std::int32_t>(static_cast<std::size_t>(blocks) * k);
+        DBuf<std::int32_t> starts = c_.buf<std::int32_t>(static_cast<std::size_t>(k) + 1);
+        DBuf<std::int32_t> order = c_.buf<std::int32_t>(static_cast<std::size_t>(count));
+        out = c_.buf<JMove>(static_cast<std::size_t>(count));
+        const unsigned long long seq = c_.next_seq();
+        hipLaunchKernelGGL(k_moves_count, dim3(blocks), dim3(kOrderThreads), 0, s, src, count, k, block_at.get(),
+                           starts.get(), c_.ticket(), unique ? nullptr : c_.read_buffer(), c_.read_flag(), seq);
         GP_LAUNCH_CHECK();
-        stable_select(c_, f.get(), count, idx.get(), cnt.get());
-        const int m = (int)c_.read_scalar(cnt.get());
-        if (!m) return 0;
-        int N = 1;
-        while (N < m) N <<= 1;
-        DBuf<std::int32_t> sidx = c_.buf<std::int32_t>(static_cast<std::size_t>(N));
-        hipLaunchKernelGGL(k_pad_index, dim3(ceil_div(N, 256)), dim3(256), 0, s, idx.get(), m, sidx.get(), N);
+        hipLaunchKernelGGL(k_moves_group, dim3(blocks), dim3(kOrderThreads), 0, s, src, count, k, block_at.get(),
+                           order.get());
         GP_LAUNCH_CHECK();
-        if (N <= 1024) {
-            hipLaunchKernelGGL((k_bitonic_local<Cmp>), dim3(1), dim3(1024), 0, s, sidx.get(), N, src, cmp);
+        DBuf<JMove> runs = c_.buf<JMove>(static_cast<std::size_t>(count));
+        hipLaunchKernelGGL((k_moves_runs<Cmp>), dim3(k, kRankSplit), dim3(kRankThreads), 0, s, src, starts.get(),
+                           order.get(), cmp, runs.get());
+        GP_LAUNCH_CHECK();
+        hipLaunchKernelGGL((k_moves_merge<Cmp>), dim3(k, kRankSplit), dim3(kRankThreads), 0, s, runs.get(),
+                           starts.get(), cmp, out.get());
+        GP_LAUNCH_CHECK();
+        if (unique) {
+            DBuf<JMove> left = c_.buf<JMove>(static_cast<std::size_t>(count));
+            DBuf<std::uint8_t> flags = c_.buf<std::uint8_t>(static_cast<std::size_t>(count));
+            const int tiles = ceil_div(count, kSelectThreads);
+            DBuf<std::int32_t> counts = c_.buf<std::int32_t>(static_cast<std::size_t>(tiles));
+            hipLaunchKernelGGL(k_unique_flags, dim3(tiles), dim3(kSelectThreads), 0, s, out.get(), starts.get() + k,
+                               flags.get(), counts.get());
             GP_LAUNCH_CHECK();
-        } else {
-            // N is a power of two above 1024: chunk-local stages in LDS, one
-            // launch per cross-chunk stage.
-            const int chunks = N / kBitonicChunk;
-            hipLaunchKernelGGL((k_bitonic_chunk<Cmp>), dim3(chunks), dim3(1024), 0, s, sidx.get(), 0, src, cmp);
+            hipLaunchKernelGGL(k_unique_place, dim3(tiles), dim3(kSelectThreads), 0, s, out.get(), starts.get() + k,
+                               flags.get(), counts.get(), left.get(), c_.read_buffer(), c_.read_flag(), seq);
             GP_LAUNCH_CHECK();
-            for (int kk = 2 * kBitonicChunk; kk <= N; kk <<= 1) {
-                for (int j = kk >> 1; j >= kBitonicChunk; j >>= 1) {
-                    hipLaunchKernelGGL((k_bitonic_global<Cmp>), dim3(ceil_div(N, 256)), dim3(256), 0, s, sidx.get(), N,
-                                       j, kk, src, cmp);
-                    GP_LAUNCH_CHECK();
-                }
-                hipLaunchKernelGGL((k_bitonic_chunk<Cmp>), dim3(chunks), dim3(1024), 0, s, sidx.get(), kk, src, cmp);
-                GP_LAUNCH_CHECK();
-            }
+            out.swap(left);
         }
-        DBuf<JMove> sorted = c_.buf<JMove>(static_cast<std::size_t>(m));
-        hipLaunchKernelGGL(k_gather_moves, dim3(ceil_div(m, 256)), dim3(256), 0, s, src, sidx.get(), m, sorted.get());
-        GP_LAUNCH_CHECK();
-        if (!unique) {
-            out = std::move(sorted);
-            return m;
-        }
-        DBuf<std::uint8_t> uf = c_.buf<std::uint8_t>(static_cast<std::size_t>(m));
-        DBuf<std::int32_t> uidx = c_.buf<std::int32_t>(static_cast<std::size_t>(m));
-        hipLaunchKernelGGL(k_unique_flags, dim3(ceil_div(m, 256)), dim3(256), 0, s, sorted.get(), m, uf.get());
-        GP_LAUNCH_CHECK();
-        stable_select(c_, uf.get(), m, uidx.get(), cnt.get());
-        const int u = (int)c_.read_scalar(cnt.get());
-        out = c_.buf<JMove>(static_cast<std::size_t>(u));
-        hipLaunchKernelGGL(k_gather_moves, dim3(ceil_div(u, 256)), dim3(256), 0, s, sorted.get(), uidx.get(), u,
-                           out.get());
-        GP_LAUNCH_CHECK();
-        return u;
+        c_.wait_flag(c_.read_flag(), seq);
+        return static_cast<int>(c_.read_buffer()[0]);
     }
 
     void publish_prices() {
