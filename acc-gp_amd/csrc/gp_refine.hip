@@ -536,6 +536,222 @@ struct BoundaryBody : RowBody {
     }
 };
 
+// ------------------------------------------------- device LP loop control
+// The LP round loop of one level decided on the device (the rules of the
+// host loop, incremental.cuh:911-961, which lp_graph.cuh:57-92 records as a
+// GPU-controlled loop), so the host can issue rounds ahead instead of reading
+// counters back after each.  Its words sit behind the part loads in the
+// counter block; the best loads (k words) follow them.
+enum LoopWord {
+    kRun = 0,      // 1 while rounds run; a round issued after the stop does nothing
+    kPhase,        // rounds run
+    kStale,
+    kEmpty,
+    kCut,
+    kBestCut,
+    kLpMoves,
+    kReason,       // LoopReason of the stop
+    kImproved,     // the last round set a new best cut: checkpoint its labels
+    kAccFrontier,  // profiled runs: rows and entries of the three sweeps, summed
+    kAccRowSum,
+    kAccAfterE,
+    kAccAfterR,
+    kAccUpdateE,
+    kAccUpdateR,
+    kLoopWords
+};
+enum LoopReason { kRunning = 0, kEnded = 1, kNeedRepair = 2, kCutUnderflow = 3, kDeferred = 4 };
+// Words of the loop state mirrored into the host mailbox after each round.
+constexpr int kMailWords = kImproved + 1;
+
+struct LoopParams {
+    int k;
+    int rounds;
+    int stale_rounds;
+    int graph_mode;  // stale rule in integers (graph loop) or long double
+    int light_only;  // no medium launch: a deferred row is an error
+    int profiling;
+    std::uint64_t cap;
+    std::uint64_t m0999;  // 64-bit significand of the long double 0.999, scaled by 2^64
+};
+
+// (long double)cut < 0.999L * (long double)best exactly as x87 extended
+// precision evaluates it (64-bit significands, round to nearest even), in
+// integers: 0.999L = m0999 / 2^64, so the product is best * m0999 / 2^64
+// rounded to 64 significant bits.
+__host__ __device__ inline bool below_0999(std::uint64_t cut, std::uint64_t best, std::uint64_t m0999) {
+    using u128 = unsigned __int128;
+    u128 p = (u128)best * m0999;
+    const std::uint64_t hi = (std::uint64_t)(p >> 64);
+    const int len = hi ? 128 - __builtin_clzll(hi) : 0;
+    if (len > 64) {
+        const int s = len - 64;
+        const u128 q = p >> s;
+        const u128 rem = p - (q << s);
+        const u128 half = (u128)1 << (s - 1);
+        const u128 r = (rem > half || (rem == half && (q & 1))) ? q + 1 : q;
+        p = r << s;
+    }
+    return ((u128)cut << 64) < p;
+}
+
+// 0.999L as m / 2^64 (0.999L lies in [1/2, 1), so m has 64 bits).
+inline std::uint64_t significand_0999() { return static_cast<std::uint64_t>(std::ldexp(0.999L, 64)); }
+
+// Loop state at the start of a run of device-controlled rounds; clears the
+// counter block; copy_best: the best loads take the current loads.
+__global__ void k_lp_arm(unsigned long long* ctr, int k, unsigned long long run, unsigned long long phase,
+                         unsigned long long stale, unsigned long long empty, unsigned long long cut,
+                         unsigned long long best, unsigned long long lp_moves, int copy_best) {
+    unsigned long long* loads = ctr + kCtrCount;
+    unsigned long long* L = loads + k;
+    for (int i = threadIdx.x; i < kCtrCount; i += blockDim.x) ctr[i] = 0;
+    if (copy_best)
+        for (int p = threadIdx.x; p < k; p += blockDim.x) L[kLoopWords + p] = loads[p];
+    if (threadIdx.x == 0) {
+        L[kRun] = run;
+        L[kPhase] = phase;
+        L[kStale] = stale;
+        L[kEmpty] = empty;
+        L[kCut] = cut;
+        L[kBestCut] = best;
+        L[kLpMoves] = lp_moves;
+        L[kReason] = kRunning;
+        L[kImproved] = 0;
+        for (int i = kAccFrontier; i < kLoopWords; ++i) L[i] = 0;
+    }
+}
+
+// What the last block of a commit does once every block is through: nothing,
+// the end of an LP round (lp_decide), or the read-back of the counters and
+// loads.  (A launch of its own for either took 5 us and the gap before it,
+// once per round and per repair iteration.)
+enum RoundEndMode { kEndNothing = 0, kEndDecide = 1, kEndRead = 2 };
+struct RoundEnd {
+    int mode;
+    LoopParams P;
+    unsigned int* ticket;
+    unsigned long long* host;  // mailbox or read-back buffer
+    unsigned long long* flag;
+    unsigned long long seq;
+    Label* keep;  // kEndDecide: see lp_decide
+    bool vec;
+    int words;    // kEndRead: words of the counter block on, the first kCtrClear of them cleared
+};
+
+// Copies n bytes by one block; vec: both arrays are 16-byte aligned.
+__device__ inline void copy_labels(const Label* from, Label* to, std::int64_t n, bool vec) {
+    const std::int64_t words = vec ? n / 16 : 0;
+    for (std::int64_t i = threadIdx.x; i < words; i += blockDim.x)
+        reinterpret_cast<uint4*>(to)[i] = reinterpret_cast<const uint4*>(from)[i];
+    for (std::int64_t v = words * 16 + threadIdx.x; v < n; v += blockDim.x) to[v] = from[v];
+}
+
+// End of one LP round, by one block: the movers, cut delta and part loads of
+// the round decide whether the loop goes on; the counter block is cleared for
+// the next round and the state is mirrored to the host mailbox.
+// keep: non-null on levels of at most kKeepInline vertices, where this block
+// also checkpoints the labels of an improving round (n bytes from labels to
+// keep) instead of a separate k_lp_keep launch.
+constexpr std::int64_t kKeepInline = 131072;
+__device__ inline void lp_decide(unsigned long long* ctr, const LoopParams& P, unsigned long long* mailbox,
+                                 unsigned long long* flag, unsigned long long seq, const Label* labels, Label* keep,
+                                 bool vec, std::int64_t n) {
+    unsigned long long* loads = ctr + kCtrCount;
+    unsigned long long* L = loads + P.k;
+    __shared__ int s_run, s_improved, s_stop;
+    __shared__ unsigned long long s_words[kLoopWords];
+    __shared__ unsigned long long s_max[1024 / kWave];
+    // Largest part load, by every thread.
+    unsigned long long mx = 0;
+    for (int p = threadIdx.x; p < P.k; p += blockDim.x) mx = loads[p] > mx ? loads[p] : mx;
+    mx = wave_max(mx);
+    if (lane_id() == 0) s_max[threadIdx.x / kWave] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (unsigned i = 1; i < blockDim.x / kWave; ++i) mx = s_max[i] > mx ? s_max[i] : mx;
+        s_run = L[kRun] != 0;
+        s_improved = 0;
+        s_stop = 0;
+        L[kImproved] = 0;
+        if (s_run) {
+            const std::uint64_t phase = L[kPhase] + 1;
+            std::uint64_t stale = L[kStale], empty = L[kEmpty], cut = L[kCut], best = L[kBestCut];
+            const std::uint64_t movers = ctr[kMovers];
+            const std::int64_t delta = (std::int64_t)ctr[kDelta];
+            int reason = kRunning;
+            if (P.profiling) {
+                L[kAccFrontier] += ctr[kFrontier];
+                L[kAccRowSum] += ctr[kRowSum];
+                L[kAccAfterE] += ctr[kEntAfter];
+                L[kAccAfterR] += ctr[kEntAfter + 1];
+                L[kAccUpdateE] += ctr[kEntUpdate];
+                L[kAccUpdateR] += ctr[kEntUpdate + 1];
+            }
+            if (P.light_only && (ctr[kTier] || ctr[kTierB] || ctr[kTierC])) {
+                reason = kDeferred;
+            } else if (!movers) {
+                if (++empty >= 2)
+                    reason = kEnded;
+                else
+                    ++stale;
+            } else {
+                empty = 0;
+                if (delta >= 0 && (std::uint64_t)delta > cut) {
+                    reason = kCutUnderflow;
+                } else {
+                    cut = delta >= 0 ? cut - (std::uint64_t)delta : cut + (std::uint64_t)(-delta);
+                    L[kLpMoves] += movers;
+                    if (mx > P.cap) {
+                        reason = kNeedRepair;  // the host repairs and finishes the round
+                    } else {
+                        ++stale;
+                        if (cut < best) {
+                            if (P.graph_mode ? best - cut > best / 1000 : below_0999(cut, best, P.m0999)) stale = 0;
+                            best = cut;
+                            s_improved = 1;
+                            L[kImproved] = 1;
+                        }
+                    }
+                }
+            }
+            if (reason == kRunning && !(phase < (std::uint64_t)P.rounds && stale < (std::uint64_t)P.stale_rounds))
+                reason = kEnded;
+            L[kPhase] = phase;
+            L[kStale] = stale;
+            L[kEmpty] = empty;
+            L[kCut] = cut;
+            L[kBestCut] = best;
+            L[kReason] = reason;
+            if (reason != kRunning) {
+                L[kRun] = 0;
+                s_stop = 1;
+            }
+            for (int i = 0; i < kLoopWords; ++i) s_words[i] = L[i];
+        }
+    }
+    __syncthreads();
+    if (!s_run) {
+        publish_to_host(flag, seq);
+        return;
+    }
+    // Running: the first kMailWords loop words to the mailbox; stopped:
+    // every loop word, then the loads and the best loads.
+    for (int i = threadIdx.x; i < (s_stop ? (int)kLoopWords : kMailWords); i += blockDim.x) mailbox[i] = s_words[i];
+    for (int p = threadIdx.x; p < P.k; p += blockDim.x) {
+        const unsigned long long load = loads[p];
+        const unsigned long long best = s_improved ? load : L[kLoopWords + p];
+        if (s_improved) L[kLoopWords + p] = load;
+        if (s_stop) {
+            mailbox[kLoopWords + p] = load;
+            mailbox[kLoopWords + P.k + p] = best;
+        }
+    }
+    publish_to_host(flag, seq);
+    for (int i = threadIdx.x; i < kCtrCount; i += blockDim.x) ctr[i] = 0;
+    if (keep && s_improved) copy_labels(labels, keep, n, vec);
+}
+
 // incremental_commit (incremental.cuh:532-547) with per-block load deltas;
 // with samples also the repair's price samples, from the gains the update
 // sweep left at the movers.  Sums per part meet in LDS and reach global memory
@@ -554,7 +770,8 @@ constexpr int kCommitBlocks = 128;
 __global__ void __launch_bounds__(kCommitThreads) k_commit(RefArgs a, const std::int32_t* list,
                                                            const unsigned long long* count_ptr, bool lp, bool samples,
                                                            const std::int32_t* donors,
-                                                           const unsigned long long* selected, bool settled) {
+                                                           const unsigned long long* selected, bool settled,
+                                                           RoundEnd end) {
     __shared__ unsigned long long delta[kMaxParts], loss[kMaxParts], weight[kMaxParts];
     const std::int64_t count = (std::int64_t)*count_ptr;
     if (donors && (settled || selected[0] == selected[1])) {
@@ -565,34 +782,45 @@ __global__ void __launch_bounds__(kCommitThreads) k_commit(RefArgs a, const std:
             if (!a.flags[v]) a.targets[v] = -1;
         }
     }
-    if (blockIdx.x * (std::int64_t)kCommitThreads >= count) return;
-    for (int p = threadIdx.x; p < a.k; p += kCommitThreads) {
-        delta[p] = 0;
-        loss[p] = 0;
-        weight[p] = 0;
-    }
-    __syncthreads();
-    for (std::int64_t i = blockIdx.x * (std::int64_t)kCommitThreads + threadIdx.x; i < count;
-         i += (std::int64_t)gridDim.x * kCommitThreads) {
-        const std::int32_t v = list[i];
-        const int s = a.labels[v], t = a.targets[v];
-        const unsigned long long w = a.vw[v];
-        atomicAdd(&delta[s], 0ULL - w);
-        atomicAdd(&delta[t], w);
-        if (samples) {
-            const std::int64_t gain = a.gains32 ? (std::int64_t)a.gains32[v] : a.gains[v];
-            atomicAdd(&loss[s], (unsigned long long)(-gain));
-            atomicAdd(&weight[s], w);
+    if (blockIdx.x * (std::int64_t)kCommitThreads < count) {
+        for (int p = threadIdx.x; p < a.k; p += kCommitThreads) {
+            delta[p] = 0;
+            loss[p] = 0;
+            weight[p] = 0;
         }
-        a.labels[v] = (Label)t;
-        if (lp) a.locks[v] = 1;
-        a.member[v] = 1;
+        __syncthreads();
+        for (std::int64_t i = blockIdx.x * (std::int64_t)kCommitThreads + threadIdx.x; i < count;
+             i += (std::int64_t)gridDim.x * kCommitThreads) {
+            const std::int32_t v = list[i];
+            const int s = a.labels[v], t = a.targets[v];
+            const unsigned long long w = a.vw[v];
+            atomicAdd(&delta[s], 0ULL - w);
+            atomicAdd(&delta[t], w);
+            if (samples) {
+                const std::int64_t gain = a.gains32 ? (std::int64_t)a.gains32[v] : a.gains[v];
+                atomicAdd(&loss[s], (unsigned long long)(-gain));
+                atomicAdd(&weight[s], w);
+            }
+            a.labels[v] = (Label)t;
+            if (lp) a.locks[v] = 1;
+            a.member[v] = 1;
+        }
+        __syncthreads();
+        for (int p = threadIdx.x; p < a.k; p += kCommitThreads) {
+            if (delta[p]) atomicAdd(&a.loads[p], delta[p]);
+            if (loss[p]) atomicAdd(&a.samples[p].loss, loss[p]);
+            if (weight[p]) atomicAdd(&a.samples[p].weight, weight[p]);
+        }
     }
-    __syncthreads();
-    for (int p = threadIdx.x; p < a.k; p += kCommitThreads) {
-        if (delta[p]) atomicAdd(&a.loads[p], delta[p]);
-        if (loss[p]) atomicAdd(&a.samples[p].loss, loss[p]);
-        if (weight[p]) atomicAdd(&a.samples[p].weight, weight[p]);
+    if (end.mode == kEndNothing || !block_is_last(end.ticket)) return;
+    if (end.mode == kEndDecide) {
+        lp_decide(a.ctr, end.P, end.host, end.flag, end.seq, a.labels, end.keep, end.vec, a.n);
+    } else {
+        for (int i = threadIdx.x; i < end.words; i += kCommitThreads) {
+            end.host[i] = a.ctr[i];
+            if (i < kCtrClear) a.ctr[i] = 0;
+        }
+        publish_to_host(end.flag, end.seq);
     }
 }
 
@@ -1976,200 +2204,7 @@ __global__ void k_publish_prices(RepairSample* samples, double* prices, int k) {
     }
 }
 
-// ------------------------------------------------- device LP loop control
-// The LP round loop of one level decided on the device (the rules of the
-// host loop, incremental.cuh:911-961, which lp_graph.cuh:57-92 records as a
-// GPU-controlled loop), so the host can issue rounds ahead instead of reading
-// counters back after each.  Its words sit behind the part loads in the
-// counter block; the best loads (k words) follow them.
-enum LoopWord {
-    kRun = 0,      // 1 while rounds run; a round issued after the stop does nothing
-    kPhase,        // rounds run
-    kStale,
-    kEmpty,
-    kCut,
-    kBestCut,
-    kLpMoves,
-    kReason,       // LoopReason of the stop
-    kImproved,     // the last round set a new best cut: checkpoint its labels
-    kAccFrontier,  // profiled runs: rows and entries of the three sweeps, summed
-    kAccRowSum,
-    kAccAfterE,
-    kAccAfterR,
-    kAccUpdateE,
-    kAccUpdateR,
-    kLoopWords
-};
-enum LoopReason { kRunning = 0, kEnded = 1, kNeedRepair = 2, kCutUnderflow = 3, kDeferred = 4 };
-// Words of the loop state mirrored into the host mailbox after each round.
-constexpr int kMailWords = kImproved + 1;
-
-struct LoopParams {
-    int k;
-    int rounds;
-    int stale_rounds;
-    int graph_mode;  // stale rule in integers (graph loop) or long double
-    int light_only;  // no medium launch: a deferred row is an error
-    int profiling;
-    std::uint64_t cap;
-    std::uint64_t m0999;  // 64-bit significand of the long double 0.999, scaled by 2^64
-};
-
-// (long double)cut < 0.999L * (long double)best exactly as x87 extended
-// precision evaluates it (64-bit significands, round to nearest even), in
-// integers: 0.999L = m0999 / 2^64, so the product is best * m0999 / 2^64
-// rounded to 64 significant bits.
-__host__ __device__ inline bool below_0999(std::uint64_t cut, std::uint64_t best, std::uint64_t m0999) {
-    using u128 = unsigned __int128;
-    u128 p = (u128)best * m0999;
-    const std::uint64_t hi = (std::uint64_t)(p >> 64);
-    const int len = hi ? 128 - __builtin_clzll(hi) : 0;
-    if (len > 64) {
-        const int s = len - 64;
-        const u128 q = p >> s;
-        const u128 rem = p - (q << s);
-        const u128 half = (u128)1 << (s - 1);
-        const u128 r = (rem > half || (rem == half && (q & 1))) ? q + 1 : q;
-        p = r << s;
-    }
-    return ((u128)cut << 64) < p;
-}
-
-// 0.999L as m / 2^64 (0.999L lies in [1/2, 1), so m has 64 bits).
-inline std::uint64_t significand_0999() { return static_cast<std::uint64_t>(std::ldexp(0.999L, 64)); }
-
-// Loop state at the start of a run of device-controlled rounds; clears the
-// counter block; copy_best: the best loads take the current loads.
-__global__ void k_lp_arm(unsigned long long* ctr, int k, unsigned long long run, unsigned long long phase,
-                         unsigned long long stale, unsigned long long empty, unsigned long long cut,
-                         unsigned long long best, unsigned long long lp_moves, int copy_best) {
-    unsigned long long* loads = ctr + kCtrCount;
-    unsigned long long* L = loads + k;
-    for (int i = threadIdx.x; i < kCtrCount; i += blockDim.x) ctr[i] = 0;
-    if (copy_best)
-        for (int p = threadIdx.x; p < k; p += blockDim.x) L[kLoopWords + p] = loads[p];
-    if (threadIdx.x == 0) {
-        L[kRun] = run;
-        L[kPhase] = phase;
-        L[kStale] = stale;
-        L[kEmpty] = empty;
-        L[kCut] = cut;
-        L[kBestCut] = best;
-        L[kLpMoves] = lp_moves;
-        L[kReason] = kRunning;
-        L[kImproved] = 0;
-        for (int i = kAccFrontier; i < kLoopWords; ++i) L[i] = 0;
-    }
-}
-
-// End of one LP round: the movers, cut delta and part loads of the round
-// decide whether the loop goes on; the counter block is cleared for the next
-// round and the state is mirrored to the host mailbox.
-// keep: non-null on small levels, where this block also checkpoints the
-// labels of an improving round (n bytes from labels to keep) instead of a
-// separate k_lp_keep launch.
-__global__ void __launch_bounds__(256) k_lp_decide(unsigned long long* ctr, LoopParams P,
-                                                   unsigned long long* mailbox, unsigned long long* flag,
-                                                   unsigned long long seq, const Label* labels, Label* keep,
-                                                   std::int64_t n) {
-    unsigned long long* loads = ctr + kCtrCount;
-    unsigned long long* L = loads + P.k;
-    __shared__ int s_run, s_improved, s_stop;
-    __shared__ unsigned long long s_words[kLoopWords];
-    __shared__ unsigned long long s_max[256 / kWave];
-    // Largest part load, by every thread.
-    unsigned long long mx = 0;
-    for (int p = threadIdx.x; p < P.k; p += blockDim.x) mx = loads[p] > mx ? loads[p] : mx;
-    mx = wave_max(mx);
-    if (lane_id() == 0) s_max[threadIdx.x / kWave] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (unsigned i = 1; i < blockDim.x / kWave; ++i) mx = s_max[i] > mx ? s_max[i] : mx;
-        s_run = L[kRun] != 0;
-        s_improved = 0;
-        s_stop = 0;
-        L[kImproved] = 0;
-        if (s_run) {
-            const std::uint64_t phase = L[kPhase] + 1;
-            std::uint64_t stale = L[kStale], empty = L[kEmpty], cut = L[kCut], best = L[kBestCut];
-            const std::uint64_t movers = ctr[kMovers];
-            const std::int64_t delta = (std::int64_t)ctr[kDelta];
-            int reason = kRunning;
-            if (P.profiling) {
-                L[kAccFrontier] += ctr[kFrontier];
-                L[kAccRowSum] += ctr[kRowSum];
-                L[kAccAfterE] += ctr[kEntAfter];
-                L[kAccAfterR] += ctr[kEntAfter + 1];
-                L[kAccUpdateE] += ctr[kEntUpdate];
-                L[kAccUpdateR] += ctr[kEntUpdate + 1];
-            }
-            if (P.light_only && (ctr[kTier] || ctr[kTierB] || ctr[kTierC])) {
-                reason = kDeferred;
-            } else if (!movers) {
-                if (++empty >= 2)
-                    reason = kEnded;
-                else
-                    ++stale;
-            } else {
-                empty = 0;
-                if (delta >= 0 && (std::uint64_t)delta > cut) {
-                    reason = kCutUnderflow;
-                } else {
-                    cut = delta >= 0 ? cut - (std::uint64_t)delta : cut + (std::uint64_t)(-delta);
-                    L[kLpMoves] += movers;
-                    if (mx > P.cap) {
-                        reason = kNeedRepair;  // the host repairs and finishes the round
-                    } else {
-                        ++stale;
-                        if (cut < best) {
-                            if (P.graph_mode ? best - cut > best / 1000 : below_0999(cut, best, P.m0999)) stale = 0;
-                            best = cut;
-                            s_improved = 1;
-                            L[kImproved] = 1;
-                        }
-                    }
-                }
-            }
-            if (reason == kRunning && !(phase < (std::uint64_t)P.rounds && stale < (std::uint64_t)P.stale_rounds))
-                reason = kEnded;
-            L[kPhase] = phase;
-            L[kStale] = stale;
-            L[kEmpty] = empty;
-            L[kCut] = cut;
-            L[kBestCut] = best;
-            L[kReason] = reason;
-            if (reason != kRunning) {
-                L[kRun] = 0;
-                s_stop = 1;
-            }
-            for (int i = 0; i < kLoopWords; ++i) s_words[i] = L[i];
-        }
-    }
-    __syncthreads();
-    if (!s_run) {
-        publish_to_host(flag, seq);
-        return;
-    }
-    // Running: the first kMailWords loop words to the mailbox; stopped:
-    // every loop word, then the loads and the best loads.
-    for (int i = threadIdx.x; i < (s_stop ? (int)kLoopWords : kMailWords); i += blockDim.x) mailbox[i] = s_words[i];
-    for (int p = threadIdx.x; p < P.k; p += blockDim.x) {
-        const unsigned long long load = loads[p];
-        const unsigned long long best = s_improved ? load : L[kLoopWords + p];
-        if (s_improved) L[kLoopWords + p] = load;
-        if (s_stop) {
-            mailbox[kLoopWords + p] = load;
-            mailbox[kLoopWords + P.k + p] = best;
-        }
-    }
-    publish_to_host(flag, seq);
-    for (int i = threadIdx.x; i < kCtrCount; i += blockDim.x) ctr[i] = 0;
-    if (keep && s_improved)
-        for (std::int64_t v = threadIdx.x; v < n; v += blockDim.x) keep[v] = labels[v];
-}
-
 // Checkpoint of the labels of a round that set a new best cut.
-constexpr std::int64_t kKeepInline = 16384;
 // vec: both arrays are 16-byte aligned (copied in 16-byte words).
 __global__ void k_lp_keep(const unsigned long long* flag, const Label* labels, Label* best, std::int64_t n, bool vec) {
     if (!*flag) return;
@@ -3271,14 +3306,20 @@ public:
         hipLaunchKernelGGL(k_compact_flags<StateLane<std::uint8_t>>, dim3(grid_for(n, kCompactTile, 512)), dim3(kCompactThreads), 0, s, n, a_.member, frontier_.get(), ctr_.get() + kFrontier, L + kRun);
         GP_LAUNCH_CHECK();
         propose_sweeps();
-        apply_launch(true, false, true);
-        // Levels of at most kKeepInline vertices checkpoint inside the
-        // decision kernel; larger ones in a launch of their own.
+        // Levels of at most kKeepInline vertices checkpoint where the round is
+        // decided; larger ones in a launch of their own.
         const bool inline_keep = n <= kKeepInline;
         const unsigned long long seq = c_.next_seq();
-        hipLaunchKernelGGL(k_lp_decide, dim3(1), dim3(256), 0, s, ctr_.get(), P, c_.mailbox(), c_.mailbox_flag(), seq,
-                           a_.labels, inline_keep ? best_labels : nullptr, n);
-        GP_LAUNCH_CHECK();
+        RoundEnd end{};
+        end.mode = kEndDecide;
+        end.P = P;
+        end.ticket = c_.ticket();
+        end.host = c_.mailbox();
+        end.flag = c_.mailbox_flag();
+        end.seq = seq;
+        end.keep = inline_keep ? best_labels : nullptr;
+        end.vec = vec;
+        apply_launch(true, false, true, end);
         if (!inline_keep) {
             hipLaunchKernelGGL(k_lp_keep, dim3(grid_for(ceil_div(n, 16), 256, 1024)), dim3(256), 0, s, L + kImproved,
                                a_.labels, best_labels, n, vec);
@@ -3409,7 +3450,8 @@ public:
     // third-sweep tier counters are still zero from the counter block's
     // clear at the start of the round or repair iteration.
     // donors, settled: as k_commit takes them (null outside repair).
-    void apply_launch(bool lp, bool samples, bool zeroed, const std::int32_t* donors = nullptr, bool settled = true) {
+    void apply_launch(bool lp, bool samples, bool zeroed, const RoundEnd& end, const std::int32_t* donors = nullptr,
+                      bool settled = true) {
         const hipStream_t s = c_.stream();
         if (!zeroed) fill<unsigned long long>(c_, ctr_.get() + kDelta, 1, 0ULL);
         if (!zeroed && c_.profiling()) fill<unsigned long long>(c_, ctr_.get() + kEntUpdate, 2, 0ULL);
@@ -3418,7 +3460,7 @@ public:
                   ctr_.get() + kDelta, 0, kTierC, zeroed, kEntUpdate);
             hipLaunchKernelGGL(k_commit, dim3(grid_for(a_.n, kCommitThreads, kCommitBlocks)), dim3(kCommitThreads), 0,
                                s, a_, movers_.get(), ctr_.get() + kMovers, lp, samples && a_.samples, donors, ctr_.get() + kSelected,
-                               settled);
+                               settled, end);
             GP_LAUNCH_CHECK();
         });
         if (samples) samples_clear_ = false;
@@ -3426,10 +3468,18 @@ public:
 
     std::int64_t apply(bool lp, bool samples, std::int64_t& delta, bool zeroed = false,
                        const std::int32_t* donors = nullptr, bool settled = true) {
-        apply_launch(lp, samples, zeroed, donors, settled);
         std::vector<unsigned long long> h(static_cast<std::size_t>(kCtrCount + a_.k));
-        // The read also clears the counters (not the part loads behind them).
-        c_.read_clear(h.data(), ctr_.get(), h.size(), kCtrClear);
+        // The read-back also clears the counters (not the part loads behind them).
+        RoundEnd end{};
+        end.mode = kEndRead;
+        end.ticket = c_.ticket();
+        end.host = c_.read_buffer();
+        end.flag = c_.read_flag();
+        end.seq = c_.next_seq();
+        end.words = static_cast<int>(h.size());
+        apply_launch(lp, samples, zeroed, end, donors, settled);
+        c_.wait_flag(end.flag, end.seq);
+        std::memcpy(h.data(), c_.read_buffer(), h.size() * sizeof(unsigned long long));
         ctr_clear_ = true;
         selected_ = (std::int64_t)h[kSelected];
         // With no row above kTierLight entries no medium launch was made; a
