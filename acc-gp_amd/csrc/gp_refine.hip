@@ -1341,29 +1341,23 @@ __device__ inline std::uint64_t wave_keyed_exclusive(int key, std::uint32_t w, u
     return at - first;
 }
 
-// Per-key exclusive scan over tiles (one wave per key); with requests,
-// ranks start at the request totals and the totals advance by this
-// attempt's requests.
-constexpr int kKeyScanThreads = 1024;
-
-__global__ void __launch_bounds__(kKeyScanThreads) k_keyed_scan(unsigned long long* S, int nb, int k,
-                                                               unsigned long long* requests) {
+// Per-key exclusive scan over tiles (one wave per key, four keys a block);
+// with requests, ranks start at the request totals and the totals advance by
+// this attempt's requests.
+__global__ void __launch_bounds__(kTierThreads) k_keyed_scan(unsigned long long* S, int nb, int k,
+                                                            unsigned long long* requests) {
     const int lane = lane_id();
-    for (int c = threadIdx.x / kWave; c < k; c += kKeyScanThreads / kWave) {
-        unsigned long long carry = requests ? requests[c] : 0;
-        for (int b0 = 0; b0 < nb; b0 += kWave) {
-            const int b = b0 + lane;
-            const unsigned long long own = b < nb ? S[(std::int64_t)c * nb + b] : 0;
-            unsigned long long x = own;
-            for (int d = 1; d < kWave; d <<= 1) {
-                const unsigned long long y = __shfl_up(x, d);
-                if (lane >= d) x += y;
-            }
-            if (b < nb) S[(std::int64_t)c * nb + b] = carry + x - own;
-            carry += __shfl(x, kWave - 1);
-        }
-        if (requests && lane == 0) requests[c] = carry;
+    const int c = blockIdx.x * (kTierThreads / kWave) + threadIdx.x / kWave;
+    if (c >= k) return;
+    unsigned long long carry = requests ? requests[c] : 0;
+    for (int b0 = 0; b0 < nb; b0 += kWave) {
+        const int b = b0 + lane;
+        const unsigned long long own = b < nb ? S[(std::int64_t)c * nb + b] : 0;
+        const std::uint64_t x = wave_inclusive_scan<PlusOp>((std::uint64_t)own);
+        if (b < nb) S[(std::int64_t)c * nb + b] = carry + x - own;
+        carry += __shfl(x, kWave - 1);
     }
+    if (requests && lane == 0) requests[c] = carry;
 }
 
 // In-tile ranks in index order; f(i, key, weight, rank) returns whether i
@@ -3640,7 +3634,8 @@ public:
                                    nb, DonorWeight{r.live}, S.get());
                 GP_LAUNCH_CHECK();
                 // Ranks start at the start-of-attempt totals; totals advance.
-                hipLaunchKernelGGL(k_keyed_scan, dim3(1), dim3(kKeyScanThreads), 0, s, S.get(), nb, k, requests);
+                hipLaunchKernelGGL(k_keyed_scan, dim3(ceil_div(k, kTierThreads / kWave)), dim3(kTierThreads), 0, s,
+                                   S.get(), nb, k, requests);
                 GP_LAUNCH_CHECK();
                 hipLaunchKernelGGL((k_keyed_apply<AdmitFn>), dim3(nb), dim3(kTierThreads), 0, s, keys.get(), nlv,
                                    S.get(), nb, AdmitFn{a_, r}, movers_.get(), ctr_.get() + kMovers);
