@@ -270,10 +270,11 @@ __global__ void k_match_choose(std::int64_t n, const std::int32_t* off, const st
                     bh = h;
                 }
             }
+#pragma unroll
             for (int d = kWave / 2; d; d >>= 1) {
-                const std::int32_t ob = __shfl_xor(best, d);
-                const std::uint64_t ow = __shfl_xor(bw, d);
-                const std::uint32_t oh = __shfl_xor(bh, d);
+                const std::int32_t ob = lane_xor(best, d);
+                const std::uint64_t ow = lane_xor(bw, d);
+                const std::uint32_t oh = lane_xor(bh, d);
                 if (ob >= 0 && (best < 0 || ow > bw || (ow == bw && (oh > bh || (oh == bh && ob > best))))) {
                     best = ob;
                     bw = ow;
@@ -391,6 +392,8 @@ __device__ inline Top2 top2_merge(const Top2& x, const Top2& y) {
 
 template <int W>
 __device__ inline Top2 top2_group_reduce(Top2 t) {
+    // Shuffles in a rolled loop: unrolled lane exchanges of these eight words
+    // cost the affinity kernels registers and made them 30 to 60 % slower.
     for (int d = W / 2; d; d >>= 1) {
         Top2 o;
         o.current = __shfl_xor(t.current, d, W);
@@ -1027,8 +1030,9 @@ __global__ void __launch_bounds__(256) k_hub_reduce(AffinityArgs a, const std::i
                     b2 = val[q];
             }
         }
+#pragma unroll
         for (int d = kWave / 2; d; d >>= 1) {
-            const unsigned long long o1 = __shfl_xor(b1, d), o2 = __shfl_xor(b2, d), oc = __shfl_xor(cur, d);
+            const unsigned long long o1 = lane_xor(b1, d), o2 = lane_xor(b2, d), oc = lane_xor(cur, d);
             const unsigned long long lo = b1 < o1 ? b1 : o1, hi2 = b2 > o2 ? b2 : o2;
             b1 = b1 > o1 ? b1 : o1;
             b2 = lo > hi2 ? lo : hi2;

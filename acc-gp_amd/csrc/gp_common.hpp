@@ -68,15 +68,69 @@ __device__ inline void block_stores_done() {
     __syncthreads();
 }
 
+// ------------------------------------------------ lane exchanges
+// The value of lane ^ d (d a power of two below 64) without the LDS crossbar
+// that __shfl_xor goes through: DPP within rows of 16 lanes (quad_perm for 1
+// and 2, half mirror i <-> 7 - i followed by the quad mirror for 4, rotation
+// by 8 for 8), row and half-wave swaps above (v_permlane16_swap_b32 and
+// v_permlane32_swap_b32 on gfx950).  d has to be a constant after unrolling;
+// the lanes that exchange have to be active.  The crossbar is one unit for a
+// CU's four SIMDs: a 512-entry bitonic row sort issues 624 of these moves, and
+// the contraction of rows of 257 to 512 entries (R-MAT scale 20) took 33 us a
+// launch with shuffles and takes 26, their affinity on scale 18 28 and 24.
+constexpr int kDppQuadXor1 = 0xB1;
+constexpr int kDppQuadXor2 = 0x4E;
+constexpr int kDppQuadMirror = 0x1B;
+constexpr int kDppRowHalfMirror = 0x141;
+constexpr int kDppRowMirror = 0x140;
+constexpr int kDppRowRor8 = 0x128;
+
+template <int Ctrl>
+__device__ inline int dpp_word(int x) {
+    return __builtin_amdgcn_update_dpp(x, x, Ctrl, 0xf, 0xf, false);
+}
+__device__ inline int lane_xor_word(int x, int d) {
+    switch (d) {
+        case 1: return dpp_word<kDppQuadXor1>(x);
+        case 2: return dpp_word<kDppQuadXor2>(x);
+        case 4: return dpp_word<kDppQuadMirror>(dpp_word<kDppRowHalfMirror>(x));
+        case 8: return dpp_word<kDppRowRor8>(x);
+        case 16: {
+            // [0]: rows 0 0 2 2, [1]: rows 1 1 3 3
+            const auto r = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)x, false, false);
+            return (int)((lane_id() & 16) ? r[0] : r[1]);
+        }
+        default: {
+            // [0]: the lower half twice, [1]: the upper half twice
+            const auto r = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)x, false, false);
+            return (int)((lane_id() & 32) ? r[0] : r[1]);
+        }
+    }
+}
+template <typename T>
+__device__ inline T lane_xor(const T& v, int d) {
+    static_assert(sizeof(T) % 4 == 0, "lane moves are 32-bit words");
+    constexpr int words = sizeof(T) / 4;
+    int in[words], out[words];
+    __builtin_memcpy(in, &v, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < words; ++i) out[i] = lane_xor_word(in[i], d);
+    T r;
+    __builtin_memcpy(&r, out, sizeof(T));
+    return r;
+}
+
 template <typename T>
 __device__ inline T wave_sum(T v) {
-    for (int d = kWave / 2; d; d >>= 1) v += __shfl_xor(v, d);
+#pragma unroll
+    for (int d = kWave / 2; d; d >>= 1) v += lane_xor(v, d);
     return v;
 }
 template <typename T>
 __device__ inline T wave_max(T v) {
+#pragma unroll
     for (int d = kWave / 2; d; d >>= 1) {
-        const T o = __shfl_xor(v, d);
+        const T o = lane_xor(v, d);
         v = o > v ? o : v;
     }
     return v;
@@ -84,54 +138,13 @@ __device__ inline T wave_max(T v) {
 // Reduction within aligned groups of W lanes (W divides 64).
 template <int W, typename T>
 __device__ inline T group_sum(T v) {
-    for (int d = W / 2; d; d >>= 1) v += __shfl_xor(v, d, W);
+#pragma unroll
+    for (int d = W / 2; d; d >>= 1) v += lane_xor(v, d);
     return v;
 }
 
 __device__ inline unsigned long long atomic_add_u64(unsigned long long* p, unsigned long long v) {
     return atomicAdd(p, v);
-}
-
-// ------------------------------------------------ wave butterflies by DPP
-// DPP controls (GFX9 encoding) of the row-local exchanges a 64-lane
-// butterfly uses: quad_perm [1,0,3,2] (lane ^ 1), quad_perm [2,3,0,1]
-// (lane ^ 2), row_half_mirror (lane i <-> 7 - i in each group of 8) and
-// row_mirror (lane i <-> 15 - i in each row of 16).  After the two quad
-// exchanges every lane holds its quad's result; the half mirror pairs each
-// lane with a lane of the other quad of its 8, the mirror with a lane of the
-// other 8 of its row, so four DPP moves combine a whole row.
-constexpr int kDppQuadXor1 = 0xB1;
-constexpr int kDppQuadXor2 = 0x4E;
-constexpr int kDppRowHalfMirror = 0x141;
-constexpr int kDppRowMirror = 0x140;
-
-// Moves a trivially copyable value (a whole number of 32-bit words) across
-// lanes by one DPP pattern; every lane of the wave must be active.
-template <int Ctrl, typename T>
-__device__ inline T dpp_move(const T& v) {
-    static_assert(sizeof(T) % 4 == 0, "DPP moves 32-bit words");
-    constexpr int words = sizeof(T) / 4;
-    int in[words], out[words];
-    __builtin_memcpy(in, &v, sizeof(T));
-#pragma unroll
-    for (int i = 0; i < words; ++i) out[i] = __builtin_amdgcn_update_dpp(in[i], in[i], Ctrl, 0xf, 0xf, false);
-    T r;
-    __builtin_memcpy(&r, out, sizeof(T));
-    return r;
-}
-
-// The same across rows (lane ^ d for d = 16, 32) through the LDS crossbar.
-template <typename T>
-__device__ inline T xor_move(const T& v, int d) {
-    static_assert(sizeof(T) % 4 == 0, "lane moves are 32-bit words");
-    constexpr int words = sizeof(T) / 4;
-    int in[words], out[words];
-    __builtin_memcpy(in, &v, sizeof(T));
-#pragma unroll
-    for (int i = 0; i < words; ++i) out[i] = __shfl_xor(in[i], d);
-    T r;
-    __builtin_memcpy(&r, out, sizeof(T));
-    return r;
 }
 
 // Every lane gets combine() over the 64 lanes' values.  combine must be
@@ -140,12 +153,8 @@ __device__ inline T xor_move(const T& v, int d) {
 // converged control flow only.
 template <typename T, typename Combine>
 __device__ inline T wave_allreduce(T v, Combine combine) {
-    v = combine(v, dpp_move<kDppQuadXor1>(v));
-    v = combine(v, dpp_move<kDppQuadXor2>(v));
-    v = combine(v, dpp_move<kDppRowHalfMirror>(v));
-    v = combine(v, dpp_move<kDppRowMirror>(v));
-    v = combine(v, xor_move(v, 16));
-    v = combine(v, xor_move(v, 32));
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) v = combine(v, lane_xor(v, d));
     return v;
 }
 

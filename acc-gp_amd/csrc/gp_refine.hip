@@ -291,6 +291,8 @@ __device__ inline bool cand_better(const Cand& x, const Cand& y, bool priced) {
 
 template <int W>
 __device__ inline Cand cand_group_reduce(Cand c, bool priced) {
+    // Shuffles: with lane exchanges here the proposals of medium rows took
+    // 46 us instead of 39 (R-MAT scale 18), for their registers.
     for (int d = W / 2; d; d >>= 1) {
         Cand o;
         o.p = __shfl_xor(c.p, d, W);
@@ -937,7 +939,7 @@ __device__ inline bool pick_better(const RepairPick& x, const RepairPick& y) {
 }
 template <int W>
 __device__ inline RepairPick pick_group_reduce(RepairPick c) {
-    for (int d = W / 2; d; d >>= 1) {
+    for (int d = W / 2; d; d >>= 1) {  // shuffles, as in cand_group_reduce
         RepairPick o;
         o.p = __shfl_xor(c.p, d, W);
         o.conn = __shfl_xor(c.conn, d, W);

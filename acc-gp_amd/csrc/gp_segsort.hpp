@@ -35,8 +35,8 @@ __device__ inline void group_bitonic_sort(std::int32_t (&k)[I], std::uint32_t (&
                     ok = k[it ^ (dist / W)];
                     ov = v[it ^ (dist / W)];
                 } else {
-                    ok = __shfl_xor(k[it], dist, W);
-                    ov = __shfl_xor(v[it], dist, W);
+                    ok = lane_xor(k[it], dist);
+                    ov = lane_xor(v[it], dist);
                 }
                 const bool lower = ((idx & dist) == 0) == ((idx & size) == 0);
                 const bool take = lower ? ok < k[it] : ok > k[it];
