@@ -3188,7 +3188,7 @@ public:
         a_.labels = labels;
         state_ = c.buf<std::uint32_t>(n);
         // Gains of at most the row weight: 32 bits below 2^31.
-        if (g.incident_bound < (1ULL << 31))
+        if (row_weight_bound() < (1ULL << 31))
             gains32_ = c.buf<std::int32_t>(n);
         else
             gains_ = c.buf<std::int64_t>(n);
@@ -3262,7 +3262,12 @@ public:
 
     // Short-row bins fit 32 bits when every row of the level weighs less
     // than 2^32 (the level's incident-weight bound).
-    bool narrow_bins() const { return g_.incident_bound <= 0xffffffffULL; }
+    bool narrow_bins() const { return row_weight_bound() <= 0xffffffffULL; }
+    // Rows of unit weights weigh their length, whose bound a changed graph
+    // keeps when its weight bound is unknown.
+    std::uint64_t row_weight_bound() const {
+        return g_.ew ? g_.incident_bound : std::min(g_.incident_bound, g_.row_len_bound);
+    }
 
     // slot: the two tier list counters; zeroed: they are known to be zero
     // (cleared with the counter block since their last use).
