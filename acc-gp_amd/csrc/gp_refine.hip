@@ -3420,8 +3420,8 @@ public:
                 const double w = a_.ew ? 4.0 : 0.0;
                 c_.add_bytes("lp_propose", 28.0 * (double)h[kAccFrontier] + (8.0 + w) * (double)h[kAccRowSum]);
                 const double g = a_.gains32 ? 4.0 : 0.0;  // 32-bit gains: 4 B less per row and entry
-                c_.add_bytes("after", (16.0 - g) * (double)h[kAccAfterR] + (20.0 - g + w) * (double)h[kAccAfterE]);
-                c_.add_bytes("update", 24.0 * (double)h[kAccUpdateR] + (16.0 + w) * (double)h[kAccUpdateE]);
+                c_.add_bytes("after", (16.0 - g) * (double)h[kAccAfterR] + (16.0 - g + w) * (double)h[kAccAfterE]);
+                c_.add_bytes("update", 24.0 * (double)h[kAccUpdateR] + (8.0 + w) * (double)h[kAccUpdateE]);
             }
             const int reason = static_cast<int>(h[kReason]);
             if (reason == kCutUnderflow) throw std::runtime_error("incremental cut underflow");
@@ -3502,9 +3502,9 @@ public:
             if (lp) {
                 c_.add_bytes("lp_propose", 28.0 * (double)h[kFrontier] + (8.0 + w) * (double)h[kRowSum]);
                 const double g = a_.gains32 ? 4.0 : 0.0;
-                c_.add_bytes("after", (16.0 - g) * (double)h[kEntAfter + 1] + (20.0 - g + w) * (double)h[kEntAfter]);
+                c_.add_bytes("after", (16.0 - g) * (double)h[kEntAfter + 1] + (16.0 - g + w) * (double)h[kEntAfter]);
             }
-            c_.add_bytes("update", 24.0 * (double)h[kEntUpdate + 1] + (16.0 + w) * (double)h[kEntUpdate]);
+            c_.add_bytes("update", 24.0 * (double)h[kEntUpdate + 1] + (8.0 + w) * (double)h[kEntUpdate]);
             if (samples)
                 c_.add_bytes("repair_propose", 24.0 * (double)h[kEntRepair + 1] + (8.0 + w) * (double)h[kEntRepair]);
         }
