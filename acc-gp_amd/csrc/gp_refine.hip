@@ -3299,7 +3299,7 @@ public:
 
     // The launches of one LP round of a device-controlled loop: the frontier
     // compaction does nothing once the loop word kRun is zero, so every later
-    // launch of the round finds empty lists; k_lp_decide ends the round.
+    // launch of the round finds empty lists; the commit's last block ends it.
     // Returns the number the round publishes in the mailbox flag.
     unsigned long long round_issue(const LoopParams& P, Label* best_labels, bool vec) {
         const hipStream_t s = c_.stream();
@@ -3352,7 +3352,7 @@ public:
     }
 
     // The LP round loop of the level with its control on the device
-    // (k_lp_decide applies the host loop's rules after each round).  The
+    // (lp_decide applies the host loop's rules after each round).  The
     // host issues each round before it has seen the previous one end
     // (ahead) or right after, watching only the mailbox; it takes over when
     // a round leaves a part over capacity, for the repair and the rest of
