@@ -310,6 +310,14 @@ int gp_debug_radix_sort(gp_context* ctx, uint64_t* keys, uint32_t* vals, int64_t
     });
 }
 
+int gp_debug_batch_cut(const int32_t* row_ends, const int32_t* row_labels, int rows, int64_t first, int count,
+                       const int32_t* neighbor_labels, uint64_t* cut) {
+    return guarded([&] {
+        if (!row_ends || !row_labels || !neighbor_labels || !cut) throw std::invalid_argument("null argument");
+        *cut = gp::debug_batch_cut(row_ends, row_labels, rows, first, count, neighbor_labels);
+    });
+}
+
 int gp_capacity(uint64_t total, int parts, double imbalance, uint64_t* out) {
     if (!out) return fail(GP_ERR_INVALID, "null output");
     return guarded([&] { *out = gp::capacity_of(total, parts, imbalance); });

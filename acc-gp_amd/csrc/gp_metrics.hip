@@ -44,7 +44,6 @@ namespace {
 
 constexpr int kCutThreads = 1024;
 constexpr int kCutWaves = kCutThreads / kWave;
-constexpr int kCutBatch = 4;                // entries per lane in flight
 constexpr int kCutPer = 4;                  // staged rows per lane
 constexpr int kCutRows = kCutPer * kWave;   // rows of a window
 
@@ -136,22 +135,7 @@ __global__ void __launch_bounds__(kCutThreads) k_edge_cut(std::int64_t n, const 
             L lu[kCutBatch];
 #pragma unroll
             for (int j = 0; j < kCutBatch; ++j) lu[j] = labels[u[j]];
-            const L lab0 = slab[w][r0];
-#pragma unroll
-            for (int j = 0; j < kCutBatch; ++j) {
-                const std::int32_t e = (std::int32_t)pos + j * kWave + lane;
-                L lab = lab0;
-                if (r0 != r1) {
-                    int lo = r0, hi = r1;  // first staged row whose end lies after e
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if (send[w][mid] <= e) lo = mid + 1;
-                        else hi = mid;
-                    }
-                    lab = slab[w][lo];
-                }
-                if (e < batch && lab != lu[j]) cut += wt[j];
-            }
+            cut += batch_cut(send[w], slab[w], r0, r1, pos, (int)(batch - pos), lane, lu, wt);
             pos = batch;
         }
         row += kCutRows;
@@ -272,6 +256,30 @@ std::uint64_t recount(Context& c, const DGraph& g, const L* labels, int k, std::
 }
 template std::uint64_t recount(Context&, const DGraph&, const std::uint8_t*, int, std::uint64_t*);
 template std::uint64_t recount(Context&, const DGraph&, const std::int32_t*, int, std::uint64_t*);
+
+std::uint64_t debug_batch_cut(const std::int32_t* ends, const std::int32_t* labels, int rows, std::int64_t pos,
+                              int len, const std::int32_t* lu) {
+    if (rows < 1 || rows > kCutRows || len < 1 || len > kCutBatch * kWave || pos < 0 ||
+        pos > (std::int64_t)ends[rows - 1] - len)
+        throw std::invalid_argument("the batch lies outside the staged rows");
+    // The kernel's ballots: row ends at or below the first, and below the last.
+    int r0 = 0, r1 = 0;
+    for (int r = 0; r < rows; ++r) {
+        r0 += ends[r] <= pos;
+        r1 += ends[r] < pos + len;
+    }
+    std::uint64_t cut = 0;
+    for (int lane = 0; lane < kWave; ++lane) {
+        std::int32_t own[kCutBatch];
+        std::uint32_t wt[kCutBatch];
+        for (int j = 0; j < kCutBatch; ++j) {
+            own[j] = lu[std::min(j * kWave + lane, len - 1)];
+            wt[j] = 1;
+        }
+        cut += batch_cut(ends, labels, r0, r1, pos, len, lane, own, wt);
+    }
+    return cut;
+}
 
 void edge_cut(Context& c, const DGraph& g, const std::int32_t* labels, int k, std::uint64_t* cut,
               std::uint64_t* loads) {

@@ -83,7 +83,7 @@ EXPORTS = [
     "gp_profile_enable", "gp_profile_query", "gp_profile_reset", "gp_server_create", "gp_server_submit",
     "gp_server_wait", "gp_server_destroy", "gp_partition_batch", "gp_server_graph_add", "gp_server_graph_download",
     "gp_server_graph_release", "gp_graph_apply_delta", "gp_debug_below_0999",
-    "gp_debug_radix_sort",
+    "gp_debug_radix_sort", "gp_debug_batch_cut",
 ]
 
 
@@ -169,6 +169,7 @@ def lib():
         L.gp_graph_apply_delta.argtypes = [vp, vp, i64, vp, vp, vp, vp, vp]
         L.gp_debug_below_0999.argtypes = [u64, u64]
         L.gp_debug_radix_sort.argtypes = [vp, vp, vp, i64, i32, i32]
+        L.gp_debug_batch_cut.argtypes = [vp, vp, i32, i64, i32, vp, vp]
         _LIB = L
     return _LIB
 
@@ -186,6 +187,15 @@ def below_0999(cut, best):
     """The device loop control's integer form of the small-level stale rule
     cut < 0.999 * best (long double)."""
     return bool(lib().gp_debug_below_0999(cut, best))
+
+
+def batch_cut(row_ends, row_labels, first, neighbor_labels):
+    """What one batch of the edge cut adds: its entries start at `first` and
+    lie in consecutive rows with these ends and labels (unit edge weights)."""
+    ends, rows, other = (np.ascontiguousarray(a, dtype=np.int32) for a in (row_ends, row_labels, neighbor_labels))
+    cut = ctypes.c_uint64()
+    check(lib().gp_debug_batch_cut(_p(ends), _p(rows), len(ends), first, len(other), _p(other), ctypes.byref(cut)))
+    return cut.value
 
 
 def radix_sort(ctx, keys, vals=None, begin_bit=0, end_bit=64):

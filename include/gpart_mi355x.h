@@ -357,6 +357,14 @@ int gp_debug_below_0999(uint64_t cut, uint64_t best);
  * tests. */
 int gp_debug_radix_sort(gp_context* ctx, uint64_t* keys, uint32_t* vals, int64_t n, int begin_bit, int end_bit);
 
+/* What one batch of the edge cut (host_cut, graph.hpp:67-69) adds on a graph
+ * of unit edge weights, by the device code's own arithmetic, on the host: the
+ * entries [first, first + count), at most 256, of `rows` consecutive rows, at
+ * most 256, that end at row_ends and have row_labels; neighbor_labels[i] is the
+ * label of the batch's i-th neighbour.  For tests. */
+int gp_debug_batch_cut(const int32_t* row_ends, const int32_t* row_labels, int rows, int64_t first, int count,
+                       const int32_t* neighbor_labels, uint64_t* cut);
+
 #ifdef __cplusplus
 }
 #endif
