@@ -1449,8 +1449,9 @@ struct SelectState {
     unsigned long long* S;              // tiles x k boundary weights
     std::int32_t* counts;               // eligible donors per tile
     std::uint8_t* elig;                 // n
-    // The reservation's start: eligible donors, their records and cleared
-    // state (done, tried bits), each part's room and request total.
+    // The reservation's start: eligible donors (n), the records and cleared
+    // state (done, tried bits) of the first tail_limit of them, each part's
+    // room and request total.
     std::int32_t* E;
     DonorInfo* live;
     std::uint8_t* done;
@@ -1461,12 +1462,25 @@ struct SelectState {
     unsigned long long tail_limit;      // donors one tail launch takes
 };
 
+__device__ inline void donor_start(const RefArgs& a, std::int64_t j, std::int32_t v, DonorInfo* live,
+                                   std::uint8_t* done, unsigned long long* tried) {
+    live[j] = DonorInfo{static_cast<std::int32_t>(j), v, a.vw[v], (std::int32_t)a.labels[v]};
+    done[j] = 0;
+    tried[2 * j] = 0;
+    tried[2 * j + 1] = 0;
+}
+// With more donors than one tail launch takes, k_donor_start lays their state
+// out once the host knows how many: arrays for all n vertices would take 33
+// bytes each at the peak of the finest level.
 __device__ inline void select_place(const RefArgs& a, const SelectState& q, std::int64_t j, std::int32_t v) {
     q.E[j] = v;
-    q.live[j] = DonorInfo{static_cast<std::int32_t>(j), v, a.vw[v], (std::int32_t)a.labels[v]};
-    q.done[j] = 0;
-    q.tried[2 * j] = 0;
-    q.tried[2 * j + 1] = 0;
+    if ((unsigned long long)j < q.tail_limit) donor_start(a, j, v, q.live, q.done, q.tried);
+}
+__global__ void k_donor_start(RefArgs a, const std::int32_t* E, std::int64_t ne, DonorInfo* live, std::uint8_t* done,
+                              unsigned long long* tried) {
+    for (std::int64_t j = blockIdx.x * (std::int64_t)blockDim.x + threadIdx.x; j < ne;
+         j += (std::int64_t)gridDim.x * blockDim.x)
+        donor_start(a, j, E[j], live, done, tried);
 }
 __device__ inline void select_parts(const RefArgs& a, const SelectState& q) {
     for (int p = threadIdx.x; p < a.k; p += blockDim.x) {
@@ -3548,7 +3562,7 @@ public:
     }
 
     // Arrays of a level's repair iterations: the donor selection's, and the
-    // connection rows of what one tail launch takes.
+    // state and connection rows of what one tail launch takes.
     struct RepairBuffers {
         DBuf<unsigned long long> prefix, excess, S, tried, slack, requests, conn;
         DBuf<std::int32_t> bstar, counts, E;
@@ -3569,12 +3583,12 @@ public:
         b.counts = c_.buf<std::int32_t>(static_cast<std::size_t>(b.tiles));
         b.elig = c_.buf<std::uint8_t>(n);
         b.E = c_.buf<std::int32_t>(n);
-        b.live = c_.buf<DonorInfo>(n);
-        b.done = c_.buf<std::uint8_t>(n);
-        b.tried = c_.buf<unsigned long long>(2 * n);
+        const std::size_t tail = static_cast<std::size_t>(std::min<std::int64_t>(a_.n, kTailDonors));
+        b.live = c_.buf<DonorInfo>(tail);
+        b.done = c_.buf<std::uint8_t>(tail);
+        b.tried = c_.buf<unsigned long long>(2 * tail);
         b.slack = c_.buf<unsigned long long>(k);
         b.requests = c_.buf<unsigned long long>(k);
-        const std::size_t tail = static_cast<std::size_t>(std::min<std::int64_t>(a_.n, kTailDonors));
         b.conn = c_.buf<unsigned long long>(tail * k);
         b.conn_part = c_.buf<std::uint8_t>(tail * k);
         b.conn_nnz = c_.buf<std::uint8_t>(tail);
@@ -3609,12 +3623,17 @@ public:
         DBuf<unsigned long long> conn = c_.buf<unsigned long long>(static_cast<std::size_t>(ne) * k);
         DBuf<std::uint8_t> conn_part = c_.buf<std::uint8_t>(static_cast<std::size_t>(ne) * k);
         DBuf<std::uint8_t> conn_nnz = c_.buf<std::uint8_t>(static_cast<std::size_t>(ne));
-        DBuf<DonorInfo> live;  // the waiting donors after a compaction
+        DBuf<DonorInfo> live = c_.buf<DonorInfo>(static_cast<std::size_t>(ne));  // later the waiting donors only
+        DBuf<std::uint8_t> done_buf = c_.buf<std::uint8_t>(static_cast<std::size_t>(ne));
+        DBuf<unsigned long long> tried = c_.buf<unsigned long long>(static_cast<std::size_t>(ne) * 2);
         const std::int32_t* E = b.E.get();
-        std::uint8_t* done = b.done.get();
+        std::uint8_t* done = done_buf.get();
         unsigned long long* requests = b.requests.get();
+        hipLaunchKernelGGL(k_donor_start, dim3(grid_for(ne)), dim3(256), 0, s, a_, E, ne, live.get(), done,
+                           tried.get());
+        GP_LAUNCH_CHECK();
         ReserveState r{E,        ne,            conn.get(), conn_part.get(), conn_nnz.get(), requests,
-                       b.slack.get(), done, b.tried.get(), b.live.get(), ne, nullptr};
+                       b.slack.get(), done, tried.get(), live.get(), ne, nullptr};
         // Attempts run in groups between host checks: an attempt without a
         // chooser changes nothing (no tried bits, no requests, no admissions),
         // so the attempts after the last active one are no-ops.  Between

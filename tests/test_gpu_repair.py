@@ -53,3 +53,26 @@ def test_repair_of_a_lopsided_start_equals_the_oracle(gp, og, ctx, n, k, share, 
                 "group_moves", "repair_iterations"):
         assert st[key] == ost[key], key
     assert np.array_equal(got, want)
+
+
+def test_repair_workspace_does_not_grow_with_the_vertices(gp):
+    """A repair of some thousand donors keeps two arrays by vertex: the donor
+    list (4 bytes) and its flags (1 byte).  Records, tried parts and connection
+    rows go by the donors."""
+    n, k, over = 1 << 20, 2, 1000
+    off, nbr, _ = _path(n, False)
+    init = np.zeros(n, np.int32)
+    init[int(1.03 * n / k) + over:] = 1
+    with gp.Context(0) as own:
+        g = gp.Graph(own, off, nbr, None, None)
+        try:
+            _, st = g.refine(init, gp.refine_options(k))
+            taken = gp.reserved_bytes(own)
+        finally:
+            g.close()
+    assert st["repair_moves"] >= over
+    # By vertex: offsets, weights and labels of the caller 12, labels as bytes
+    # and their checkpoint 2, state 4, gains 8, five lists and the buckets 24,
+    # the repair's two 5: 55.  An array is rounded up by an eighth at most; the
+    # connection rows of 4,096 donors and the rest are far below 4 MiB.
+    assert taken <= 9 / 8 * (55 * n + 4 * len(nbr)) + (4 << 20), (taken, n, len(nbr))
