@@ -1385,6 +1385,21 @@ static void og_dense_affinity(og_ref* R, uint64_t* A) {
     for (int64_t v = 0; v < R->n; ++v) og_affinity(R, v, A + (size_t)v * R->k);
 }
 
+/* Most moves of one part that an exchange ordered (archive, pool) since the
+ * last reset; which forms of the device's ordering a check reaches. */
+static int og_most_moves[2];
+static void og_note_moves(const og_move* m, int count, int* most) {
+    for (int i = 0, from = 0; i < count; ++i) {
+        if (m[i].a != m[from].a) from = i;
+        if (i - from + 1 > *most) *most = i - from + 1;
+    }
+}
+void og_t_most_moves(int reset, int32_t* archive, int32_t* pool) {
+    *archive = og_most_moves[0];
+    *pool = og_most_moves[1];
+    if (reset) og_most_moves[0] = og_most_moves[1] = 0;
+}
+
 /* Capacity-complementary exchange driver: incremental.cuh:974-1041. */
 static int og_exchange(og_ref* R, int passes, uint64_t* best_cut) {
     const og_graph* g = R->g;
@@ -1454,6 +1469,7 @@ static int og_exchange(og_ref* R, int passes, uint64_t* best_cut) {
         int fr = 0;
         for (int i = 0; i < slots * OG_JOINT_ARCHIVE; ++i) if (archive[i].size) archive[fr++] = archive[i];
         qsort(archive, (size_t)fr, sizeof(og_move), cmp_joint_net);
+        og_note_moves(archive, fr, &og_most_moves[0]);
         int uq = 0;
         for (int i = 0; i < fr; ++i) {
             if (uq && og_same_move(&archive[uq - 1], &archive[i])) continue;
@@ -1466,6 +1482,7 @@ static int og_exchange(og_ref* R, int passes, uint64_t* best_cut) {
         for (int i = 0; i < slots + 2 * fragments; ++i) if (pool[i].size) pool[active++] = pool[i];
         if (!active) { if (++empty >= 2) break; continue; }
         qsort(pool, (size_t)active, sizeof(og_move), cmp_joint_order);
+        og_note_moves(pool, active, &og_most_moves[1]);
         /* claim / resolve / mark: exchange.cuh:205-226 */
         for (int64_t v = 0; v < n; ++v) owners[v] = INT32_MAX;
         for (int i = 0; i < active; ++i)

@@ -142,6 +142,7 @@ int64_t og_t_afterburner(int64_t n, const int32_t* off, const int32_t* nbr, cons
                          const int32_t* targets, const int64_t* gains, uint8_t* keep);
 /* Repair gain bucket of a gain per unit of relief. */
 int og_t_gain_bucket(double gain);
+void og_t_most_moves(int reset, int32_t* archive, int32_t* pool);
 /* Repair destination of vertex v (-1 none), with A(v, dest) and A(v, own). */
 int og_t_repair_destination(int64_t n, const int32_t* off, const int32_t* nbr, const uint32_t* ew,
                             const uint32_t* vw, int k, const int32_t* labels, const uint64_t* loads, uint64_t cap,

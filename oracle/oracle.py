@@ -242,6 +242,7 @@ def _bind_stages():
     L.og_t_afterburner.restype = i64
     L.og_t_afterburner.argtypes = [i64, vp, vp, vp, vp, ci, vp, vp, u64, vp, vp, vp, vp]
     L.og_t_gain_bucket.argtypes = [dbl]
+    L.og_t_most_moves.argtypes = [ci, vp, vp]
     L.og_t_repair_destination.argtypes = [i64, vp, vp, vp, vp, ci, vp, vp, u64, ctypes.c_int32, vp, vp]
     L.og_t_repair_iteration.restype = i64
     L.og_t_repair_iteration.argtypes = [i64, vp, vp, vp, vp, ci, vp, vp, u64, vp, vp, vp, vp]
@@ -264,6 +265,15 @@ def seed_match(off, nbr, ew, vw, cap, salt):
     roots = np.zeros(n, np.int32)
     count = lib().og_t_seed_match(n, _p(off), _p(nbr), _p(ew), _p(vw), cap, salt, _p(roots))
     return roots, int(count)
+
+
+def most_moves(reset=False):
+    """Most moves of one part that an exchange ordered since the last reset:
+    (archive, pool)."""
+    _bind_stages()
+    archive, pool = ctypes.c_int32(), ctypes.c_int32()
+    lib().og_t_most_moves(int(reset), ctypes.byref(archive), ctypes.byref(pool))
+    return archive.value, pool.value
 
 
 def below_0999(cut, best):

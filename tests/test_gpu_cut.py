@@ -1,8 +1,11 @@
-"""gp_edge_cut and gp_edge_cut_noalloc on shapes where the even split of the
-entries over waves can go wrong: rows without entries (also runs of more than
-64, at either end), one row over many waves' spans, entry counts around
-multiples of 64, vertex counts around a window of 64 rows, weights whose
-sum passes 2^32, 2 and 128 parts.  Whole numbers: exact.
+"""gp_edge_cut and gp_edge_cut_noalloc on shapes where the even split of rows
+and entries over the waves can go wrong.  A wave's share is at most 256 steps
+(a row is one, an entry is one) until a graph has more than 512 x 4,096 of
+them, and grows from there; it walks its entries in windows of 256 rows and
+batches of 256 entries.  So: rows without entries (a few, a share's worth, whole
+windows inside a share), one row over many shares, row counts around a window,
+sizes just below and above 512 x 4,096 steps in byte and int32 labels, weights
+whose sum passes 2^32, 2 and 128 parts.  Whole numbers: exact.
 """
 import ctypes
 
@@ -45,12 +48,35 @@ def _heavy(n, m):
     return off, nbr, ew, vw
 
 
+def _scattered_edges(n, gap):
+    """Three edges, to the next vertex and two across the gap, after every
+    `gap` rows without entries."""
+    at = np.arange(gap, n - gap, gap, dtype=np.int64)
+    u = np.concatenate([at, at, at[:-1] + 1])
+    v = np.concatenate([at + 1, at + 2, at[1:]])
+    src, dst = np.concatenate([u, v]), np.concatenate([v, u])
+    order = np.lexsort((dst, src))
+    off = np.zeros(n + 1, np.int64)
+    np.cumsum(np.bincount(src, minlength=n), out=off[1:])
+    return off.astype(np.int32), dst[order].astype(np.int32), None, None
+
+
 CASES = {
     "one_edge": lambda gp: _star(2, 0, 0),
     "edge_after_70_empty_rows": lambda gp: _star(2, 70, 0),
     "edge_before_200_empty_rows": lambda gp: _star(2, 0, 200),
     "star_40000_among_empty_rows": lambda gp: _star(40000, 130, 65),
     "path_33": lambda gp: graphs.grid(1, 33) + (None, None),
+    "path_255": lambda gp: graphs.grid(1, 255) + (None, None),
+    "path_256": lambda gp: graphs.grid(1, 256) + (None, None),
+    "path_257": lambda gp: graphs.grid(1, 257) + (None, None),
+    # Shares of 613 steps, windows without an entry before the first edge in
+    # one; shares of 864, a window without an entry between two of their edges.
+    "edges_every_1500_of_5000000_rows": lambda gp: _scattered_edges(5000000, 1500),
+    "edges_every_600_of_7000000_rows": lambda gp: _scattered_edges(7000000, 600),
+    # 2,093,690 and 2,100,166 steps: 512 blocks with shares of 256 and 257.
+    "grid_647x648": lambda gp: gp.generate_grid(647, 648) + (None, None),
+    "grid_648x649": lambda gp: gp.generate_grid(648, 649) + (None, None),
     "grid_64x63": lambda gp: gp.generate_grid(64, 63) + (None, None),
     "grid_129x127": lambda gp: gp.generate_grid(129, 127) + (None, None),
     "grid_520x511": lambda gp: gp.generate_grid(520, 511) + (None, None),  # labels narrowed to bytes
