@@ -32,8 +32,9 @@
 #include <unordered_map>
 
 // Scratch of the allocation-free evaluation (edge_cut_noalloc): room for the
-// partial rows of the largest evaluation, at most 1025 rows of 130 words
-// (cut, out-of-range count, 128 loads), 1,066,000 bytes.  Every GPU holds its own copy until the process ends.
+// partial rows of the largest evaluation, 512 rows of 130 words (cut,
+// out-of-range count, 128 loads), 532,480 bytes.  Every GPU holds its own copy
+// until the process ends.
 // Host code never passes this name to a kernel: it is a host-side stand-in,
 // and the device address comes from hipGetSymbolAddress per device.
 static __device__ __align__(256) unsigned long long scratch[gp::kNoAllocScratchWords];

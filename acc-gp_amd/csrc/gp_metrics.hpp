@@ -57,10 +57,10 @@ void edge_cut_into(Context& c, const DGraph& g, const std::int32_t* labels, int 
 void edge_cut(Context& c, const DGraph& g, const std::int32_t* labels, int k, std::uint64_t* cut,
               std::uint64_t* loads_host);
 
-// Words of the static device scratch of edge_cut_noalloc: more than the
-// largest evaluation takes (kEdgeCutMaxBlocks partial rows).
-constexpr std::size_t kNoAllocScratchWords = 1025 * static_cast<std::size_t>(kMaxParts + 2);
-static_assert(kEdgeCutMaxBlocks <= 1025, "the static scratch holds every partial row");
+// Words of the static device scratch of edge_cut_noalloc: what the largest
+// evaluation takes.
+constexpr std::size_t kNoAllocScratchWords =
+    static_cast<std::size_t>(kEdgeCutMaxBlocks) * static_cast<std::size_t>(kMaxParts + 2);
 // Resolves (once per device, that device current) and caches the device
 // address of the static scratch; called at context creation.
 unsigned long long* resolve_noalloc_scratch(int device);

@@ -238,7 +238,7 @@ int gp_edge_cut(gp_context* ctx, const gp_graph* g, const int32_t* labels, int p
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments, results and errors as gp_edge_cut; the per-block partials live
- * in a static device array of 1025 x 130 words (1,066,000 bytes, held by
+ * in a static device array of 512 x 130 words (532,480 bytes, held by
  * each GPU the library runs on until the process ends) instead of the
  * context arena, so the call makes no hipMalloc and touches no arena.  It
  * covers every graph size at parts <= 128 (GP_ERR_INVALID above).  Calls
