@@ -726,7 +726,6 @@ __global__ void k_chunk_counts(Src src, std::int64_t count, std::int64_t* out) {
 // key, as the reduction reads it.  R-MAT scale 22, all long rows of a
 // partition: 15.3 ms of histograms and scatters, now 7.9.
 struct RowSort {
-    std::int64_t rows;
     const std::int64_t* raw_base;   // where a row's records start before the first pass
     const std::int64_t* base;       // and after it (rows + 1 entries)
     const std::int64_t* tile_base;  // first tile of a row (rows + 1 entries)
@@ -1702,7 +1701,7 @@ static std::int64_t reduce_hashed_rows(Context& c, const Src& src, std::int64_t 
     DBuf<std::int32_t> tile_row = c.buf<std::int32_t>(static_cast<std::size_t>(tiles));
     hipLaunchKernelGGL(k_tile_rows, dim3(grid_for(count, 4)), dim3(256), 0, s, count, tile_base.get(), tile_row.get());
     GP_LAUNCH_CHECK();
-    const RowSort q{count, raw_base, base.get(), tile_base.get(), tile_row.get()};
+    const RowSort q{raw_base, base.get(), tile_base.get(), tile_row.get()};
     DBuf<std::uint32_t> keys2, vals2 = c.buf<std::uint32_t>(static_cast<std::size_t>(records));
     if (key_bits > 8) keys2 = c.buf<std::uint32_t>(static_cast<std::size_t>(records));
     DBuf<std::uint64_t> wide = c.buf<std::uint64_t>(static_cast<std::size_t>(records));

@@ -82,7 +82,6 @@ constexpr int kDppQuadXor1 = 0xB1;
 constexpr int kDppQuadXor2 = 0x4E;
 constexpr int kDppQuadMirror = 0x1B;
 constexpr int kDppRowHalfMirror = 0x141;
-constexpr int kDppRowMirror = 0x140;
 constexpr int kDppRowRor8 = 0x128;
 
 template <int Ctrl>
