@@ -36,10 +36,6 @@ struct MetaOut {
     unsigned long long max_vw;    // 6
 };
 
-__device__ inline std::uint64_t sat_add(std::uint64_t a, std::uint64_t b) {
-    return ~0ULL - a < b ? ~0ULL : a + b;
-}
-
 // Row sums (exact: u32 weights over int32 rows stay below 2^63) and the
 // sorted-row check; the body's accumulator counts unsorted rows.
 struct MetaBody {

@@ -142,10 +142,6 @@ __device__ inline T group_sum(T v) {
     return v;
 }
 
-__device__ inline unsigned long long atomic_add_u64(unsigned long long* p, unsigned long long v) {
-    return atomicAdd(p, v);
-}
-
 // Every lane gets combine() over the 64 lanes' values.  combine must be
 // associative and commutative (a sum, or the better of two under a total
 // order), so the result does not depend on the pairing.  Called from

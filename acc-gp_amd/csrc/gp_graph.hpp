@@ -101,11 +101,4 @@ public:
     const DGraph& level(int i) const { return i == 0 ? *input : *coarse[static_cast<std::size_t>(i - 1)]; }
 };
 
-// Kernel-time accounting for the roofline report (HIP events on the stream).
-struct KernelStat {
-    double ms = 0.0;
-    double bytes = 0.0;
-    long launches = 0;
-};
-
 }  // namespace gp

@@ -16,7 +16,8 @@
 // [0, k), load_0 .. load_{k-1}]; the last block to finish adds the rows up and
 // writes the totals straight to the host's read-back buffer.
 //
-// R-MAT scale 20 (31 M entries, k = 64): 145 us; 64 vertices per wave, the
+// R-MAT scale 20 (31 M entries, k = 64), counted again and again: 141 us (168
+// when graph and labels change from call to call); 64 vertices per wave, the
 // earlier split, took 14.5 ms, one wave walking all the hubs, and an even
 // split of the entries alone 360 us, where a wave meets hundreds of rows with
 // an entry or none.  kCutBatch 8 instead of 4: 196 us.
@@ -189,9 +190,9 @@ __global__ void __launch_bounds__(256) k_byte_labels(std::int64_t n, const std::
 
 // From this many vertices on (1 MiB of int32 labels, a quarter of an XCD's L2),
 // int32 labels are narrowed to bytes before the entries gather them, where
-// scratch can be allocated.  Whole calls with and without: R-MAT scale 18 63
-// and 66 us, scale 20 145 and 174, a mesh of 2 M points 120 and 190, a grid of
-// 4 M cells (its gathers are local) 83 and 80.
+// scratch can be allocated.  Whole calls with and without, counting again and
+// again: R-MAT scale 18 63 and 64 us, scale 20 141 and 169, a mesh of 2 M
+// points 117 and 191, a grid of 4 M cells (its gathers are local) 81 and 77.
 constexpr std::int64_t kByteLabelsMin = 1 << 18;
 
 // Launch and read-back: `totals` gets the directed cut, the number of labels

@@ -45,12 +45,6 @@ struct PlusOp {
     template <typename T>
     __device__ static T op(T a, T b) { return a + b; }
 };
-struct MaxOp {
-    template <typename T>
-    __device__ static T id() { return T(0); }
-    template <typename T>
-    __device__ static T op(T a, T b) { return a > b ? a : b; }
-};
 
 // Segmented value: head marks the first element of a segment.
 struct SegU64 {

@@ -2611,8 +2611,10 @@ struct JointOrder {
 // and block of the source, with the parts' starts from the last block; their
 // indices grouped by part (any order inside); runs of 256 moves of a part
 // sorted by merges in LDS; the runs of a part merged, all by binary searches
-// for each move's place.  The moves of a pair of parts carry its lower part,
-// so a part has up to some 2,000.
+// for each move's place.  The moves of a pair of parts carry its lower part:
+// up to k = 32 a pair has 512 grown moves and 4 archived ones for each of them,
+// and two more moves for every archived one, so a part has at most 2,048 moves
+// in the archive and 4,608 in the pool (fewer above: 1,024 and 2,304 at k = 64).
 // The bitonic networks that this replaces ran 66 dependent stages over records
 // 64 bytes apart in LDS, 16 lanes to a bank, 64 to 74 us for each chunk of
 // 2,048 moves and several launches for more; comparing all pairs of a part took
@@ -3507,11 +3509,10 @@ public:
         if (c_.profiling()) {
             // Algorithmic bytes per row and per entry of each sweep (weighted
             // graphs add 4 B of edge weight per entry): LP proposal 28 + 8;
-            // afterburner 16 + 20 (neighbour, target, gain, label; 4 B less
-            // each with 32-bit gains); update and
-            // commit 24 + 16 (neighbour, label, target, flag); repair proposal
-            // 24 + 8 (offsets, label, weight, bucket and target out; neighbour
-            // and its label per entry).
+            // afterburner 16 + 16 (neighbour, state word, gain; 4 B less each
+            // with 32-bit gains); update and commit 24 + 8 (neighbour, state
+            // word); repair proposal 24 + 8 (offsets, label, weight, bucket and
+            // target out; neighbour and its label per entry).
             const double w = a_.ew ? 4.0 : 0.0;
             if (lp) {
                 c_.add_bytes("lp_propose", 28.0 * (double)h[kFrontier] + (8.0 + w) * (double)h[kRowSum]);

@@ -1,11 +1,12 @@
 // Three-tier row processing for skewed degree distributions.
 //
-// A "body" processes one CSR row with a team of lanes: a 16-lane group
-// (rows <= kTierLight entries), a full wave (rows <= kTierMedium) or a
-// 256-thread block (longer rows).  Light kernels defer longer rows to a
-// medium list and medium kernels defer to a heavy list, with wave-aggregated
-// appends (one atomic per wave).  Loops are wave-uniform so every lane of a
-// wave reaches the ballots.
+// A "body" processes one CSR row with a team of lanes: 4 lanes (8 or 16 when
+// the context or the tables' LDS ask for it; rows <= kTierLight entries), a
+// wave or half of one (rows <= kTierMedium) or a block of kHeavyThreads
+// (longer rows).  The light kernel hands longer rows to a medium and a heavy
+// list.  Appends are staged per wave in LDS: one atomic per kStage of them,
+// and at the kernel's end one per block for what is left.  Loops are
+// wave-uniform so every lane of a wave reaches the ballots.
 #pragma once
 #include "gp_prims.hpp"
 
@@ -20,20 +21,8 @@ constexpr int kTierThreads = 256;
 constexpr int kHeavyThreads = 512;  // one block per heavy row: many entries in flight
 constexpr int kBlockRed = 3 * (kHeavyThreads / kWave);  // u64 words of block-team reduction scratch
 
-// Appends v for every lane with pred set; all lanes of the wave must call it.
-__device__ inline void wave_append(bool pred, std::int32_t v, std::int32_t* list, unsigned long long* count) {
-    const unsigned long long mask = __ballot(pred);
-    if (!mask) return;
-    const int lane = lane_id();
-    const int leader = __ffsll(mask) - 1;
-    unsigned long long base = 0;
-    if (lane == leader) base = atomicAdd(count, (unsigned long long)__popcll(mask));
-    base = __shfl(base, leader);
-    if (pred) list[base + __popcll(mask & ((1ULL << lane) - 1ULL))] = v;
-}
-
 // Wave-private LDS staging of list appends: one global atomic per kStage
-// entries instead of one per wave step.  List order is unspecified; every
+// entries instead of one per wave step; block_flush takes the rest.  List order is unspecified; every
 // list built this way is consumed by per-vertex work.  All lanes of the
 // wave call push() and flush() together.
 constexpr int kStage = 256;

@@ -291,7 +291,7 @@ public:
 
     // Words of coherent host memory that device-side loop control kernels
     // write their state to, so the host can follow a loop without a copy.
-    // Its flag word takes the sequence numbers of loop_seq().
+    // Its flag word takes numbers of next_seq().
     unsigned long long* mailbox() const { return static_cast<unsigned long long*>(mailbox_); }
     unsigned long long* mailbox_flag() const { return mailbox() + kMailboxBytes / 8 - 1; }
     // The read-back buffer, its flag word and the next sequence number, for
