@@ -89,7 +89,8 @@ REFERENCE_CONSTANTS = [
 ]
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="reference tree not present")
+@pytest.mark.skipif(not os.path.isfile(os.path.join(REFERENCE, REFERENCE_CONSTANTS[0][0])),
+                    reason="reference tree not present")
 def test_constants_match_reference_source():
     oracle_text = open(ORACLE_C).read().lower().replace(" ", "")
     for rel, line, text in REFERENCE_CONSTANTS:
