@@ -15,8 +15,8 @@ struct HostGraph {
 };
 
 // Deterministic recursive-bisection partitioner for the coarsest graph.
-// This is not METIS: breadth-first region growing from hashed seeds followed
-// by greedy boundary refinement, best of four trials per bisection.
+// This is not METIS: breadth-first regions from hashed starts, the best of them
+// refined by Fiduccia-Mattheyses passes, best of eight recursions.
 void initial_partition_host(std::int64_t n, const std::int32_t* off, const std::int32_t* nbr, const std::uint32_t* ew,
                             const std::uint32_t* vw, int parts, double imbalance, std::uint32_t seed,
                             std::int32_t* labels);
