@@ -1715,6 +1715,12 @@ static std::int64_t reduce_hashed_rows(Context& c, const Src& src, std::int64_t 
         keys.swap(keys2);
         vals.swap(vals2);
     }
+    // What the sums do not read goes back first: records and sums together
+    // would be the peak of coarsening.
+    keys.reset();
+    keys2.reset();
+    vals2.reset();
+    hist.reset();
     return reduce_sorted(c, wide, vals, records, ukeys, usums);
 }
 
